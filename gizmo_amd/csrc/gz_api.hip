@@ -86,6 +86,7 @@ struct gz_context {
     // the cell ranges and stencils depend only on the order (key_version) and the level: they
     // are kept across calls while both stay the same
     long key_version = 0, grid_version = -1;
+    bool sten_valid = false;  // the cells' stencils belong to the current grid
     // an upper bound on every kernel radius (< 0: unknown, reduce over all particles)
     double hmax_bound = -1;
     double hmax_rows = -1;  // the largest clamped radius of the active rows, when already known
@@ -506,8 +507,9 @@ int copy_dev(gz_context *ctx, void *dst, const void *src, size_t bytes)
     return 0;
 }
 
-// grid of level L over the current device order; the stencil of each cell
-int build_grid(gz_context *ctx, double rmax, bool need_chmax = false)
+// grid of level L over the current device order; with cell_walk (the walks of one wavefront per
+// cell: passes over many rows) also the stencil of each cell, which the row kernels find themselves
+int build_grid(gz_context *ctx, double rmax, bool cell_walk, bool need_chmax = false)
 {
     const double box = ctx->par.box_size;
     // cell side >= the largest search radius plus twice the distance any particle has moved
@@ -519,7 +521,8 @@ int build_grid(gz_context *ctx, double rmax, bool need_chmax = false)
     int L = 0;
     while (L < kFineLevel && box / (double)(1 << (L + 1)) >= reach * (1.0 + 1e-6)) L++;
     const long ncell = 1L << (3 * L);
-    if (L == ctx->level && ctx->grid_version == ctx->key_version && !need_chmax) return 0;
+    const bool same = L == ctx->level && ctx->grid_version == ctx->key_version;
+    if (same && (ctx->sten_valid || !cell_walk) && !need_chmax) return 0;
     if (ncell > ctx->grid_cells_alloc) {
         CHK(dalloc(ctx, &ctx->cstart, ncell)); CHK(dalloc(ctx, &ctx->cend, ncell)); CHK(dalloc(ctx, &ctx->nsten, ncell));
         CHK(dalloc(ctx, &ctx->sten, ncell * 27)); CHK(dalloc(ctx, &ctx->chmax, ncell));
@@ -536,9 +539,14 @@ int build_grid(gz_context *ctx, double rmax, bool need_chmax = false)
         ctx->cell = box / (double)(1 << L);
         k_cell_clear<<<nblk(ncell), kBlock, 0, ctx->stream>>>(ncell, ctx->cstart, ctx->cend, ctx->chmax);
         k_cell_bounds<<<nblk(ctx->n), kBlock, 0, ctx->stream>>>(ctx->n, ctx->key, 3 * (kFineLevel - L), ctx->cstart, ctx->cend);
-        k_cell_stencil<<<nblk(ncell), kBlock, 0, ctx->stream>>>(L, ctx->cstart, ctx->cend, ctx->sten, ctx->nsten);
         HIPCHK(hipGetLastError());
         ctx->grid_version = ctx->key_version;
+        ctx->sten_valid = false;
+    }
+    if (cell_walk && !ctx->sten_valid) {
+        k_cell_stencil<<<nblk(32 * ncell), kBlock, 0, ctx->stream>>>(L, ctx->cstart, ctx->cend, ctx->sten, ctx->nsten);
+        HIPCHK(hipGetLastError());
+        ctx->sten_valid = true;
     }
     if (need_chmax) {
         k_cell_hmax<<<nblk(ncell), kBlock, 0, ctx->stream>>>(ncell, ctx->cstart, ctx->cend, ctx->H, ctx->chmax);
@@ -870,9 +878,9 @@ int density_stage(gz_context *ctx)
     }
     const bool wide = ctx->wide != 0;
     if (wide) CHK(build_wide(ctx, false));
-    else CHK(build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size)));
-    CHK(drift_stencil(ctx));
     const bool few = wide || na <= ctx->few_rows;
+    if (!wide) CHK(build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size), !few));
+    CHK(drift_stencil(ctx));
     if (!few) CHK(build_cell_rows(ctx));
     // a step of the run loop with few rows may launch the passes behind the first round before
     // its counters are read (they are gated on the round's gate word); the radius bound the symmetric
@@ -976,7 +984,7 @@ int density_rounds(gz_context *ctx, int iters, bool speculate)
         if (rebuild && !wide) {
             // a radius outgrew the cell side: a coarser grid for the rows still iterating
             CHK(max_on_device(ctx, ctx->it_h, na, &hmax));
-            CHK(build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size)));
+            CHK(build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size), !few));
             CHK(drift_stencil(ctx));
             if (!few) CHK(build_cell_rows(ctx));
             ctx->st.ngb_rebuilds += 1;
@@ -1048,7 +1056,7 @@ int ensure_sym(gz_context *ctx)
     const bool few = ctx->nact <= ctx->few_rows;
     // the row walks drop stencil cells beyond reach: every radius is at most hmax
     if (wide) CHK(build_wide(ctx, true));
-    else CHK(build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size)));
+    else CHK(build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size), !few));
     CHK(drift_stencil(ctx));
     GridView gs = grid_view(ctx);
     gs.chmax = nullptr;
@@ -2195,7 +2203,7 @@ long gz_neighbors(gz_context *ctx, int symmetric, long *offsets, int *nbr, long 
     int capl = 0;
     double hmax = 0;
     if (max_on_device(ctx, ctx->H, n, &hmax)) return -GZ_E_HIP;
-    if (build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size), true)) return -GZ_E_HIP;
+    if (build_grid(ctx, std::min(hmax, 0.5 * ctx->par.box_size), true, true)) return -GZ_E_HIP;
     if (dalloc(ctx, &cnt, ctx->nact)) return -GZ_E_MEMORY;
     int rc = 0;
     if (symmetric && ctx->wide) {

@@ -252,38 +252,46 @@ __global__ void k_cell_hmax(long ncell, const int *__restrict__ cstart, const in
 
 
 // the (deduplicated) 27 neighbour cells of each cell, non-empty ones only, sorted by start;
-// each entry packs start, end and the offset code (dx+1)*9+(dy+1)*3+(dz+1)
+// each entry packs start, end and the offset code (dx+1)*9+(dy+1)*3+(dz+1).  Half a wavefront per
+// cell, one lane per neighbour: a lane's place is its rank among the kept starts, counted over
+// shuffles.  (One thread per cell with its entries sorted in scratch took 145-175 us whatever the
+// grid, all of it the chain of 27 dependent loads and the insertion sort: a third of a pass over a
+// few thousand particles.)
 #ifdef GZ_DEFINE_COMMON_KERNELS
-__global__ void k_cell_stencil(int level, const int *__restrict__ cstart, const int *__restrict__ cend,
-                               int4 *__restrict__ sten, int *__restrict__ nsten)
+__global__ void __launch_bounds__(256) k_cell_stencil(int level, const int *__restrict__ cstart, const int *__restrict__ cend,
+                                                      int4 *__restrict__ sten, int *__restrict__ nsten)
 {
-    long ncell = 1L << (3 * level);
-    long c = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
-    int nc = 1 << level;
-    int cx = compact10((uint32_t)c >> 2), cy = compact10((uint32_t)c >> 1), cz = compact10((uint32_t)c);
-    int4 e[27];
-    int m = 0;
-    for (int dx = -1; dx <= 1; dx++)
-        for (int dy = -1; dy <= 1; dy++)
-            for (int dz = -1; dz <= 1; dz++) {
-                int a = (cx + dx + nc) % nc, b = (cy + dy + nc) % nc, d = (cz + dz + nc) % nc;
-                uint32_t code = (spread10(a) << 2) | (spread10(b) << 1) | spread10(d);
-                int st = cstart[code], en = cend[code];
-                if (en <= st) continue;
-                bool dup = false;
-                for (int q = 0; q < m; q++) if (e[q].x == st) { dup = true; break; }
-                if (dup) continue;
-                e[m++] = make_int4(st, en, (dx + 1) * 9 + (dy + 1) * 3 + (dz + 1), (int)code);
-            }
-    for (int a = 1; a < m; a++) {  // insertion sort by start
-        int4 t = e[a];
-        int b = a - 1;
-        while (b >= 0 && e[b].x > t.x) { e[b + 1] = e[b]; b--; }
-        e[b + 1] = t;
+    const long ncell = 1L << (3 * level);
+    const long c = (blockIdx.x * (long)blockDim.x + threadIdx.x) >> 5;
+    if (c >= ncell) return;  // whole halves of a wavefront leave: the shuffles stay within one half
+    const int lane = threadIdx.x & 31;
+    const int nc = 1 << level;
+    const int cx = compact10((uint32_t)c >> 2), cy = compact10((uint32_t)c >> 1), cz = compact10((uint32_t)c);
+    const int none = 0x7fffffff;
+    int st = none, en = 0;
+    uint32_t code = 0;
+    if (lane < 27) {
+        const int dx = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
+        const int a = (cx + dx + nc) % nc, b = (cy + dy + nc) % nc, d = (cz + dz + nc) % nc;
+        code = (spread10(a) << 2) | (spread10(b) << 1) | spread10(d);
+        st = cstart[code];
+        en = cend[code];
+        if (en <= st) st = none;
     }
-    for (int q = 0; q < m; q++) sten[c * 27 + q] = e[q];
-    nsten[c] = m;
+    if (nc < 3) {
+        // neighbours coincide on such grids: the first lane of each start stays
+        bool dup = false;
+        for (int q = 0; q < 27; q++) dup |= __shfl(st, q, 32) == st && q < lane;
+        if (dup) st = none;
+    }
+    int rank = 0, m = 0;
+    for (int q = 0; q < 27; q++) {
+        const int s = __shfl(st, q, 32);
+        rank += s < st;
+        m += s != none;
+    }
+    if (st != none) sten[c * 27 + rank] = make_int4(st, en, lane, (int)code);
+    if (lane == 0) nsten[c] = m;
 }
 #endif
 
