@@ -938,10 +938,12 @@ int density_rounds(gz_context *ctx, int iters, bool speculate)
                     k_density_rows<KERN, R, 64><<<xcd_grid(nround), 64, 0, ctx->stream>>>(
                         ctx->dp, grid_view(ctx), na, ctx->act, ctx->need, ctx->key, ctx->X, ctx->Y, ctx->Z, ctx->VX, ctx->VY, ctx->VZ,
                         ctx->M, ctx->it_h, ctx->dacc, BoxTable{}, npairs, rows, nround);
-                else
-                    k_density_cells<KERN, R><<<xcd_grid(ctx->ncells), 64, 0, ctx->stream>>>(
+                else {
+                    auto cells_kernel = ctx->fd ? k_density_cells<KERN, R, true> : k_density_cells<KERN, R, false>;
+                    cells_kernel<<<xcd_grid(ctx->ncells), 64, 0, ctx->stream>>>(
                         ctx->dp, grid_view(ctx), cell_rows(ctx), ctx->act, ctx->need, ctx->X, ctx->Y, ctx->Z, ctx->VX, ctx->VY, ctx->VZ,
                         ctx->M, ctx->it_h, ctx->dacc);
+                }
             }
             if (npairs) k_sum_counts<<<std::min(nblk(nround), 256u), kBlock, 0, ctx->stream>>>(nround, npairs, ctx->u64c + 77);
             // the speculative first round: its closing launch also writes the pass's gate word

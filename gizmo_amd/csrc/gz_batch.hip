@@ -520,9 +520,9 @@ int density(gz_batch *b)
         BHIP(hipMemsetAsync(b->counters, 0, 3 * sizeof(int), b->stream));
         if (na > b->few_rows) {
             BCHK(build_groups(b));
-            k_density_cells<KERN, R><<<xcd_grid(b->grp.ngroups), 64, 0, b->stream>>>(b->dp, gview(b), b->grp.view(bt), b->act, b->need,
-                                                                                      b->X, b->Y, b->Z, b->VX, b->VY, b->VZ, b->M,
-                                                                                      b->it_h, b->dacc);
+            auto cells_kernel = b->dp.fd4alpha > 0 ? k_density_cells<KERN, R, true> : k_density_cells<KERN, R, false>;
+            cells_kernel<<<xcd_grid(b->grp.ngroups), 64, 0, b->stream>>>(b->dp, gview(b), b->grp.view(bt), b->act, b->need, b->X, b->Y,
+                                                                         b->Z, b->VX, b->VY, b->VZ, b->M, b->it_h, b->dacc);
         } else {
             k_density_rows<KERN, R, kRowThreads><<<xcd_grid(na), kRowThreads, 0, b->stream>>>(b->dp, gview(b), na, b->act, b->need, b->key, b->X, b->Y, b->Z,
                                                                          b->VX, b->VY, b->VZ, b->M, b->it_h, b->dacc, bt);

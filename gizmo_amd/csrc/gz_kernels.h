@@ -284,7 +284,8 @@ __global__ void k_cell_rows_list(int nact, const int *act, const uint32_t *key, 
 __global__ void k_build_sym_cells(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
                                   const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
 
-template <int KERN, typename R>
+// FD: with the sums of the first-derivative volume correction
+template <int KERN, typename R, bool FD>
 __global__ void k_density_cells(DevParams P, GridView g, CellRows cr, const int *act, const uint8_t *need, const double *X,
                                 const double *Y, const double *Z, const double *VX, const double *VY, const double *VZ,
                                 const double *M, const double *hcur, double *accout);

@@ -26,10 +26,15 @@ namespace gz {
                                                           const double *, const double *, const double *, const double *,       \
                                                           const double *, double *, BoxTable, int *, const int *, int);
 
+#define GZ_INST_DCELLS(KERN, R, FD)                                                                                             \
+    template __global__ void k_density_cells<KERN, R, FD>(DevParams, GridView, CellRows, const int *, const uint8_t *,          \
+                                                          const double *, const double *, const double *, const double *,       \
+                                                          const double *, const double *, const double *, const double *,       \
+                                                          double *);
+
 #define GZ_INST(KERN, R)                                                                                                         \
-    template __global__ void k_density_cells<KERN, R>(DevParams, GridView, CellRows, const int *, const uint8_t *,              \
-                                                      const double *, const double *, const double *, const double *,           \
-                                                      const double *, const double *, const double *, const double *, double *);\
+    GZ_INST_DCELLS(KERN, R, false)                                                                                               \
+    GZ_INST_DCELLS(KERN, R, true)                                                                                                \
     GZ_INST_LANES(KERN, R, false)                                                                                                \
     GZ_INST_LANES(KERN, R, true)                                                                                                 \
     GZ_INST_DROWS(KERN, R, 64)                                                                                                   \

@@ -477,14 +477,89 @@ __device__ __forceinline__ int kept_rank(bool keep, int &count)
     return __popcll(m & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
 }
 
+// The difference of two coordinates of a pair closer than half a box: d brought to the nearest
+// image, d - box * rint(d / box).  The product is exact (the factor is -1, 0 or 1), so the bits
+// are those of wrap() in three instructions instead of eight; only a difference that rounds
+// onto half a box may take the other image, which no pair within reach of a kernel has.
+__device__ __forceinline__ double wrap_near(double d, double box, double inv_box)
+{
+    return __builtin_fma(-__builtin_rint(d * inv_box), box, d);
+}
+
+// m = 2 m + (t <= lim): one candidate's bit into a lane's mask in two instructions
+__device__ __forceinline__ void mask_push(uint32_t &m, float t, float lim)
+{
+    __asm__("v_cmp_le_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(t), "v"(lim) : "vcc");
+}
+
+// ---------------------------------------------------------------------------------------
+// Cell walk's candidate window.  Most candidates a wavefront stages lie outside a given row's
+// radius (72 of 432 on a 64-neighbour lattice), so testing each of them with the pair body
+// behind the test runs the body for every candidate that any lane accepts: all of them.
+// Instead a tile of 64 culled candidates is tested first in FP32 (coordinates in units of the
+// cell side around the cell's centre: |x_j|^2 - 2 x_i.x_j against h_i^2 - |x_i|^2, four
+// instructions a candidate, with a slack that covers every rounding, so no partner is missed),
+// each lane keeping one bit per candidate; the lanes then take their own candidates one by one
+// through the exact test and the body.  The last kWinWords tiles stay in LDS, and a new one is
+// taken only when every lane is done with the oldest: lanes with few candidates in one tile
+// run ahead into the next ones, so the body runs nearly as often as the longest lane needs it
+// (78 times for rows of 77 partners among 432 culled candidates; 115 with a window of three
+// tiles, 203 with one).  Each lane takes its candidates in ascending order.
+// ---------------------------------------------------------------------------------------
+constexpr int kWinWords = 5;                     // tiles in the window
+constexpr int kWinRing = 64 * (kWinWords + 1);   // staged candidates: the window and the tile being filled
+// r^2 in units of the cell side squared: |x| <= 2 along each axis (a stencil cell and the
+// distance a particle may have moved, at most half a cell), |x|^2 <= 12, a dozen roundings of
+// 2^-24 each of at most 24: below 2e-5
+constexpr float kWinSlack = 3e-5f;
+
+// A lane's queue of masks: m[0] belongs to the tile at ring slot `at`, `behind` tiles before the
+// newest, the others to the tiles after it.
+struct Window {
+    unsigned long long m[kWinWords];
+    int at = 0, behind = -1;
+    __device__ __forceinline__ Window()
+    {
+        for (int w = 0; w < kWinWords; w++) m[w] = 0;
+    }
+    // a new tile's mask (behind < kWinWords - 1 in every lane)
+    __device__ __forceinline__ void push(unsigned long long mask)
+    {
+        behind++;
+        for (int w = 0; w < kWinWords; w++) m[w] = behind == w ? mask : m[w];
+    }
+    // on to the next tile when this lane is done with its oldest; whether it has a candidate now
+    __device__ __forceinline__ bool ready()
+    {
+        const bool done = m[0] == 0 && behind >= 0;
+        for (int w = 0; w + 1 < kWinWords; w++) m[w] = done ? m[w + 1] : m[w];
+        m[kWinWords - 1] = done ? 0 : m[kWinWords - 1];
+        behind -= done;
+        at += done ? 64 : 0;
+        at = at == kWinRing ? 0 : at;
+        return m[0] != 0;
+    }
+    // the ring slot of this lane's next candidate (ready() holds)
+    __device__ __forceinline__ int next()
+    {
+        const int slot = at + (int)__builtin_ctzll(m[0]);
+        m[0] &= m[0] - 1;
+        return slot;
+    }
+};
+
 // ---------------------------------------------------------------------------------------
 // density as a cell walk: one wavefront per occupied cell, its active particles one per lane;
-// the candidates of the cell's 27 neighbour ranges are staged through LDS 64 at a time (after
-// leaf culling) and every lane tests them in ascending order (the oracle's summation order).
-// need[r] marks the rows still iterating.  The 13 pair sums of DensitySpec::pair_kernel
-// (src/hydro/density_loop.h:1141-1385) go to acc[13*r]; k_density_after closes the round.
+// the candidates of the cell's 27 neighbour ranges are staged through LDS after leaf culling
+// and go through the candidate window above, every lane taking its own in ascending order (the
+// oracle's summation order).  need[r] marks the rows still iterating.  The 13 pair sums of
+// DensitySpec::pair_kernel (src/hydro/density_loop.h:1141-1385) go to acc[13*r];
+// k_density_after closes the round.  Bound by the body's VALU instructions (140 per candidate taken
+// in FP64, a third of them the square root and the division).  2M rows: FP64 3.45 -> 1.52 ms, FP32
+// 1.64 -> 1.11 ms against the body behind the test of every candidate; a window of three tiles
+// with branches around the sums (each copied all of them) took 2.12 and 1.45 ms.
 // ---------------------------------------------------------------------------------------
-template <int KERN, typename R>
+template <int KERN, typename R, bool FD>
 __global__ void __launch_bounds__(64) k_density_cells(DevParams P, GridView g, CellRows cr, const int *__restrict__ act,
                                                       const uint8_t *__restrict__ need, const double *__restrict__ X,
                                                       const double *__restrict__ Y, const double *__restrict__ Z,
@@ -492,7 +567,12 @@ __global__ void __launch_bounds__(64) k_density_cells(DevParams P, GridView g, C
                                                       const double *__restrict__ VZ, const double *__restrict__ M,
                                                       const double *__restrict__ hcur, double *__restrict__ accout)
 {
-    __shared__ double sx[64], sy[64], sz[64], svx[64], svy[64], svz[64], sm[64];
+    // the staged candidates: positions in FP64 (FP32 form on grids of 8 cells a side or more: as
+    // floats relative to the cell's origin, in the same memory), velocities and masses, and the
+    // tile being filled in cell units for the FP32 test
+    __shared__ double sx[kWinRing], sy[kWinRing], sz[kWinRing];
+    __shared__ R svx[kWinRing], svy[kWinRing], svz[kWinRing], sm[kWinRing];
+    __shared__ float4 st[64];
     const long cb = xcd_block();
     if (cb >= (cr.ncells_dev ? *cr.ncells_dev : cr.ncells)) return;
     int c, a0, a1, nst;
@@ -509,6 +589,12 @@ __global__ void __launch_bounds__(64) k_density_cells(DevParams P, GridView g, C
         c = cr.cells[cb]; a0 = cr.ca0[c]; a1 = cr.ca1[c]; nst = g.nsten[c]; sten = g.sten + (size_t)c * 27;
     }
     const int t = threadIdx.x;
+    const double inv_box = 1.0 / P.box;
+    // a lane without a candidate reads ring slots that may not be staged yet: zeros
+    for (int k = t; k < kWinRing; k += 64) {
+        sx[k] = sy[k] = sz[k] = 0;
+        svx[k] = svy[k] = svz[k] = sm[k] = 0;
+    }
     for (int base = a0; base < a1; base += 64) {
         const bool in = base + t < a1;
         const int r = in ? (cr.grow ? cr.grow[base + t] : base + t) : 0;
@@ -525,96 +611,155 @@ __global__ void __launch_bounds__(64) k_density_cells(DevParams P, GridView g, C
         }
         const LeafBox lb = leaf_box(g, c, on, xi, yi, zi);
         const double reach = wave_max(on ? h : 0.0);
-        // FP32 form on grids of at least 8 cells a side: positions relative to the home cell's
-        // origin (one FP64 difference and wrap per row and per staged candidate, rounded to
-        // FP32; every partner then lies within half a box of the origin), so the pair
-        // differences are FP32 subtractions
-        const bool rel = std::is_same<R, float>::value && (1 << g.level) >= 8;
+        // grids of at least 8 cells a side: every partner lies within half a box of the home
+        // cell's origin, so relative positions (one FP64 difference and wrap per row and per
+        // staged candidate) give the pairs' differences: the FP32 test of the window, and the
+        // FP32 form's pair differences
+        const bool small = (1 << g.level) >= 8;
+        const bool rel = std::is_same<R, float>::value && small;
         const R rxi = (R)wrap(xi - lb.ox, g.box, g.half), ryi = (R)wrap(yi - lb.oy, g.box, g.half),
                 rzi = (R)wrap(zi - lb.oz, g.box, g.half);
-        const bool fd = P.fd4alpha > 0;
-        R a[kDensSumsFD];
-        for (int q = 0; q < kDensSumsFD; q++) a[q] = 0;
+        const double inv_cell = 1.0 / g.cell;
+        float qx, qy, qz, lim;
+        {
+            const float ux = (float)(wrap(xi - lb.ox, g.box, g.half) * inv_cell - 0.5), uy = (float)(wrap(yi - lb.oy, g.box, g.half) * inv_cell - 0.5),
+                        uz = (float)(wrap(zi - lb.oz, g.box, g.half) * inv_cell - 0.5), uh = (float)(h * inv_cell);
+            qx = -2.0f * ux; qy = -2.0f * uy; qz = -2.0f * uz;
+            lim = on ? (uh * uh - (ux * ux + uy * uy + uz * uz)) + kWinSlack : -1e30f;
+        }
+        constexpr int nsum = FD ? kDensSumsFD : kDensSums;
+        R a[nsum];
+        for (int q = 0; q < nsum; q++) a[q] = 0;
         const R hR = (R)(on ? h : 1.0);
         const R h2 = hR * hR;
         R hinv, hinv3, hinv4;
         kernel_hinv(hR, hinv, hinv3, hinv4);
-        for (int q = 0; q < nst; q++) {
-            const int4 e = sten[q];
-            for (int ts = e.x; ts < e.y; ts += 64) {
-                const int j = ts + t;
-                bool keep = false;
-                double xj = 0, yj = 0, zj = 0;
-                if (j < e.y) {
+        Window win;
+        int head = 0;  // ring slot of the tile being filled
+        int q = 0, ts = nst > 0 ? sten[0].x : 0, te = nst > 0 ? sten[0].y : 0;  // the next candidates
+        int fill = 0;       // candidates in the tile being filled
+        bool keep = false;  // this lane holds a candidate for the next tile, at place pos
+        int pos = 0, j = 0;
+        double xj = 0, yj = 0, zj = 0;
+        bool more = nst > 0, left = false;
+        // a candidate into the tile being filled
+        auto stage = [&](int k) {
+            const int s = head + k;
+            const double ux = wrap(xj - lb.ox, g.box, g.half), uy = wrap(yj - lb.oy, g.box, g.half), uz = wrap(zj - lb.oz, g.box, g.half);
+            if (rel) {
+                ((float *)sx)[s] = (float)ux; ((float *)sy)[s] = (float)uy; ((float *)sz)[s] = (float)uz;
+            } else {
+                sx[s] = xj; sy[s] = yj; sz[s] = zj;
+            }
+            svx[s] = (R)VX[j]; svy[s] = (R)VY[j]; svz[s] = (R)VZ[j]; sm[s] = (R)M[j];
+            const float fx = (float)(ux * inv_cell - 0.5), fy = (float)(uy * inv_cell - 0.5), fz = (float)(uz * inv_cell - 0.5);
+            st[k] = make_float4(fx, fy, fz, fx * fx + fy * fy + fz * fz);
+        };
+        while (more || left) {
+            __syncthreads();  // the lanes are done with the tile before the last and its test values
+            if (keep) stage(pos);  // what the last tile had no room for
+            keep = false;
+            left = false;
+            while (more && fill < 64) {
+                j = ts + t;
+                if (j < te) {
                     xj = X[j]; yj = Y[j]; zj = Z[j];
                     keep = leaf_reach(g, lb, xj, yj, zj, reach);
                 }
                 int nt;
-                const int pos = kept_rank(keep, nt);
-                __syncthreads();
-                if (keep) {
-                    if (rel) {
-                        sx[pos] = (R)wrap(xj - lb.ox, g.box, g.half);
-                        sy[pos] = (R)wrap(yj - lb.oy, g.box, g.half);
-                        sz[pos] = (R)wrap(zj - lb.oz, g.box, g.half);
-                    } else {
-                        sx[pos] = xj; sy[pos] = yj; sz[pos] = zj;
-                    }
-                    svx[pos] = VX[j]; svy[pos] = VY[j]; svz[pos] = VZ[j]; sm[pos] = M[j];
+                pos = fill + kept_rank(keep, nt);
+                if (keep && pos < 64) {
+                    stage(pos);
+                    keep = false;
                 }
-                __syncthreads();
-                if (!on) continue;
-                for (int k = 0; k < nt; k++) {
-                    const double mj = sm[k];
-                    if (mj <= 0) continue;
-                    R dp0, dp1, dp2;
-                    if (rel) {
-                        dp0 = rxi - (R)sx[k]; dp1 = ryi - (R)sy[k]; dp2 = rzi - (R)sz[k];
-                    } else {
-                        double d0 = xi - sx[k], d1 = yi - sy[k], d2 = zi - sz[k];
-                        d1 = wrap(d1, P.box, P.half);
-                        d0 = wrap(d0, P.box, P.half);
-                        d2 = wrap(d2, P.box, P.half);
-                        dp0 = (R)d0; dp1 = (R)d1; dp2 = (R)d2;
-                    }
-                    const R r2 = dp0 * dp0 + dp1 * dp1 + dp2 * dp2;
-                    if (r2 >= h2) continue;
-                    const R rr = sqrt(r2);
-                    const R u = rr * hinv;
-                    R wk = 0, dwk = 0;
-                    kernel_main<KERN, 0>(u, hinv3, hinv4, wk, dwk);
-                    const R mj_wk = (R)mj * wk;
-                    a[0] += rounded(wk);
-                    a[1] += rounded(mj_wk);
-                    a[2] += rounded(-(R(3.0) * hinv * wk + u * dwk));
-                    if (rr > 0) {
-                        a[4] += rounded(wk * (dp0 * dp0));
-                        a[5] += rounded(wk * (dp1 * dp1));
-                        a[6] += rounded(wk * (dp2 * dp2));
-                        a[7] += rounded(wk * (dp0 * dp1));
-                        a[8] += rounded(wk * (dp1 * dp2));
-                        a[9] += rounded(wk * (dp0 * dp2));
-                        a[10] += rounded(wk * dp0);
-                        a[11] += rounded(wk * dp1);
-                        a[12] += rounded(wk * dp2);
-                        const R dv0 = vxi - (R)svx[k], dv1 = vyi - (R)svy[k], dv2 = vzi - (R)svz[k];
-                        a[3] -= rounded(dwk * (dp0 * dv0 + dp1 * dv1 + dp2 * dv2) / rr);
-                        if (fd) {  // GradH_numer, GradH_denom (src/hydro/density_loop.h:1281-1286)
-                            a[13] += rounded((dwk / rr) * dp0);
-                            a[14] += rounded((dwk / rr) * dp1);
-                            a[15] += rounded((dwk / rr) * dp2);
-                            a[16] += rounded(u * dwk);
-                        }
-                    }
+                fill += nt;
+                ts += 64;
+                if (ts >= te) {
+                    q++;
+                    more = q < nst;
+                    if (more) { ts = sten[q].x; te = sten[q].y; }
                 }
             }
+            const int nt = fill < 64 ? fill : 64;
+            fill -= nt;
+            left = fill > 0;
+            pos -= 64;
+            if (t >= nt) st[t] = make_float4(0.0f, 0.0f, 0.0f, 1e30f);  // no candidate
+            __syncthreads();
+            uint32_t mlo = 0, mhi = 0;
+            if (small) {
+#pragma unroll 4
+                for (int k = 31; k >= 0; k--) {
+                    const float4 u = st[k], v = st[k + 32];
+                    mask_push(mlo, __builtin_fmaf(qx, u.x, __builtin_fmaf(qy, u.y, __builtin_fmaf(qz, u.z, u.w))), lim);
+                    mask_push(mhi, __builtin_fmaf(qx, v.x, __builtin_fmaf(qy, v.y, __builtin_fmaf(qz, v.z, v.w))), lim);
+                }
+            } else {
+                // coarse grids: the test itself, in FP64
+                const double lim2 = on ? h * h * (1.0 + 1e-5) : -1.0;
+                for (int k = 63; k >= 0; k--) {
+                    const int s = head + k;
+                    const double d0 = wrap(xi - sx[s], g.box, g.half), d1 = wrap(yi - sy[s], g.box, g.half), d2 = wrap(zi - sz[s], g.box, g.half);
+                    const bool ok = k < nt && d0 * d0 + d1 * d1 + d2 * d2 <= lim2;
+                    mhi = (mhi << 1) | (mlo >> 31);
+                    mlo = (mlo << 1) | (ok ? 1u : 0u);
+                }
+            }
+            win.push(((unsigned long long)mhi << 32) | mlo);
+            head = head == kWinRing - 64 ? 0 : head + 64;
+            // until the next tile has room (the last tile: until every candidate is taken)
+            const int room = more || left ? kWinWords - 2 : -1;
+            do {
+                // one region without branches (a branch around the sums would copy all of them): a
+                // lane without a candidate, a candidate that is no partner, and the row itself
+                // (rr = 0) add zeros, which leave a sum that starts at +0 as it is bit for bit
+                const bool got = win.ready();
+                const int k = got ? win.next() : 0;
+                const R mj = sm[k];
+                R dp0, dp1, dp2;
+                if (rel) {
+                    dp0 = rxi - (R)((float *)sx)[k]; dp1 = ryi - (R)((float *)sy)[k]; dp2 = rzi - (R)((float *)sz)[k];
+                } else {
+                    dp0 = (R)wrap_near(xi - sx[k], P.box, inv_box);
+                    dp1 = (R)wrap_near(yi - sy[k], P.box, inv_box);
+                    dp2 = (R)wrap_near(zi - sz[k], P.box, inv_box);
+                }
+                const R r2 = dp0 * dp0 + dp1 * dp1 + dp2 * dp2;
+                const bool ok = got && !(mj <= 0) && !(r2 >= h2);
+                const R rr = sqrt(r2);
+                const R u = rr * hinv;
+                R wk = 0, dwk = 0;
+                kernel_main<KERN, 0>(u, hinv3, hinv4, wk, dwk);
+                wk = ok ? wk : R(0);
+                dwk = ok ? dwk : R(0);
+                const R mj_wk = mj * wk;
+                a[0] += rounded(wk);
+                a[1] += rounded(mj_wk);
+                a[2] += rounded(-(R(3.0) * hinv * wk + u * dwk));
+                a[4] += rounded(wk * (dp0 * dp0));
+                a[5] += rounded(wk * (dp1 * dp1));
+                a[6] += rounded(wk * (dp2 * dp2));
+                a[7] += rounded(wk * (dp0 * dp1));
+                a[8] += rounded(wk * (dp1 * dp2));
+                a[9] += rounded(wk * (dp0 * dp2));
+                a[10] += rounded(wk * dp0);
+                a[11] += rounded(wk * dp1);
+                a[12] += rounded(wk * dp2);
+                const R dv0 = vxi - svx[k], dv1 = vyi - svy[k], dv2 = vzi - svz[k];
+                const R rs = rr > 0 ? rr : R(1);
+                const R dwr = rounded(dwk * (dp0 * dv0 + dp1 * dv1 + dp2 * dv2) / rs);
+                a[3] -= ok && rr > 0 ? dwr : R(0);
+                if constexpr (FD) {  // GradH_numer, GradH_denom (src/hydro/density_loop.h:1281-1286)
+                    a[13] += rounded((dwk / rs) * dp0);
+                    a[14] += rounded((dwk / rs) * dp1);
+                    a[15] += rounded((dwk / rs) * dp2);
+                    a[16] += rounded(u * dwk);
+                }
+            } while (wave_any(win.behind > room));
         }
-        if (on) {
-            // static bounds: the sums stay in registers
-            for (int q = 0; q < kDensSums; q++) accout[(size_t)q * cr.nrows + r] = (double)a[q];
-            if (fd)
-                for (int q = kDensSums; q < kDensSumsFD; q++) accout[(size_t)q * cr.nrows + r] = (double)a[q];
-        }
+        __syncthreads();  // before the next rows' candidates take the ring
+        if (on)
+            for (int k = 0; k < nsum; k++) accout[(size_t)k * cr.nrows + r] = (double)a[k];
     }
 }
 

@@ -1,0 +1,61 @@
+"""The kernels of passes over many rows (cell walks, one lane per row) against the row kernels
+(a workgroup per row), at the sizes where their tiles, windows and queues can go wrong: grids of
+2-4 cells a side (no relative coordinates), cells of more than 64 rows, candidate counts that are
+no multiple of a tile, radii far below the cell side, partly active rows, strong shocks (every
+rung of the Riemann ladder).
+
+Both shapes add each row's terms in ascending partner order, so every field agrees bit for bit,
+in both arithmetic forms; the row kernels are held to the oracle in test_gpu_parity.py and
+test_gpu_riemann.py.
+"""
+import numpy as np
+import pytest
+
+from gizmo_amd import ics
+from gizmo_amd.hydro import GZ_FP32_MIXED, GZ_FP64, Hydro
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("h", "numngb", "rho", "press", "nvt", "nvt_fw", "cn", "fce", "drkern", "divvel", "grad_rho", "grad_p", "grad_v",
+          "accel", "dtu", "maxsig", "wakeup")
+
+BOXES = {
+    "two_cells": lambda: ics.lattice_box(8, 21, kernel=3, des_num_ngb=32.0, mach_sigma=0.3),
+    "four_cells": lambda: ics.lattice_box(13, 22, kernel=6, des_num_ngb=64.0, mach_sigma=1.0),
+    "eight_cells": lambda: ics.lattice_box(21, 23, kernel=6, des_num_ngb=64.0, mach_sigma=2.0),
+    "odd": lambda: ics.lattice_box(27, 24, kernel=3, des_num_ngb=32.0, mach_sigma=0.2),
+    # one grid sized by the largest radius: dense cells of hundreds of rows with radii of a
+    # fraction of the cell
+    "clustered": lambda: ics.lognormal_box(6000, 25, ng=16),
+    "blast": lambda: ics.sedov_box(18, 26, kernel=6, des_num_ngb=64.0),
+}
+
+
+def run(ic, few_rows, precision, active, fd):
+    g = Hydro(dict(ic["params"]), len(ic["mass"]), precision)
+    g.set_option("few_rows", few_rows)
+    if fd:
+        g.set_option("fd_correction", 1)
+    g.load({k: ic[k] for k in ("pos", "vel", "mass", "u", "h")})
+    g.hydro_pass()
+    if active < 1.0:
+        rng = np.random.Generator(np.random.Philox(7))
+        g.set_active(rng.random(len(ic["mass"])) < active)
+        g.hydro_pass()
+    out = g.store(FIELDS)
+    g.close()
+    return out
+
+
+@pytest.mark.parametrize("precision", [GZ_FP64, GZ_FP32_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("name,active,fd", [("two_cells", 1.0, False), ("four_cells", 0.3, False), ("eight_cells", 1.0, True),
+                                            ("eight_cells", 0.05, False), ("odd", 1.0, False), ("clustered", 1.0, False),
+                                            ("clustered", 0.4, False), ("blast", 1.0, False)])
+def test_many_rows_equal_row_kernels(name, active, fd, precision):
+    ic = BOXES[name]()
+    print(f"shapes: {name} n={len(ic['mass'])} active={active} fd={fd} precision={precision}", flush=True)
+    a = run(ic, 0, precision, active, fd)
+    b = run(ic, 10 ** 9, precision, active, fd)
+    for k in FIELDS:
+        same = a[k].view(np.int64 if a[k].dtype == np.float64 else a[k].dtype) == b[k].view(np.int64 if b[k].dtype == np.float64 else b[k].dtype)
+        assert np.isfinite(a[k]).all() and same.all(), (k, int((~same).sum()), same.size)
