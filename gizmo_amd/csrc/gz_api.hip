@@ -74,10 +74,7 @@ struct gz_context {
     bool speculate = false, spec = false;
     bool spec_enabled = true;  // option "speculate"
     bool fd = false;           // option "fd_correction": the first-derivative volume correction of the density
-    int force_split = -1;      // option "force_split": -1 by the last pass's rare share, 0 one kernel, 1 two kernels
-    int force_waves = 0;       // option "force_waves": the FP64 common force kernel's waves per SIMD (0: by wide_search)
-    double rare_share = 0;     // share of the rows the last two-kernel force pass left to k_force_rare
-    bool split_ran = false;
+    int force_split = -1;      // option "force_split": 0 leaves the rows with rare faces uncounted
     bool force_flags_clear = false;  // the last gradient launch cleared the force pass's flags
     bool in_run_steps = false;       // inside gz_run_steps' loop
     bool prepped = false;            // the last step's closing kick cleared this step's counters
@@ -109,12 +106,13 @@ struct gz_context {
     RowGroups grp;
     // the force pass's row order over the lanes (longest lists first within blocks of rows)
     int *sched = nullptr;
-    int *rare = nullptr;  // rows the force pass's common kernel leaves to the whole Riemann ladder
     // the rows still iterating in the density rounds of the row kernels: rl_a holds the coming
     // round's rows (hcounters[0] of them) when rl_valid, rl_b receives the next round's
     int *rl_a = nullptr, *rl_b = nullptr;
     bool rl_valid = false;
     unsigned long long *sched_part = nullptr;
+    void *flux = nullptr;     // the force pass's stored fluxes
+    size_t flux_bytes = 0;
     int sched_span = 2048;  // rows per sorted block (0: plain order)
     bool sched_valid = false;
 
@@ -424,7 +422,7 @@ void free_state(gz_context *c)
     dfree(c->wide_dev);
     {
         dfree(c->act_bits); dfree(c->act_bcount);
-        dfree(c->sched); dfree(c->sched_part); dfree(c->rare); dfree(c->rl_a); dfree(c->rl_b);
+        dfree(c->sched); dfree(c->sched_part); dfree(c->flux); c->flux_bytes = 0; dfree(c->rl_a); dfree(c->rl_b);
         c->sched_valid = false;
         c->rl_valid = false;
         RowGroups &G = c->grp;
@@ -1193,40 +1191,31 @@ int force_stage(gz_context *ctx)
                 ctx->all_active ? nullptr : ctx->ACT, ctx->TB, ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2,
                 ctx->counters + 4, ctx->nact <= kRowPairAtomics ? ctx->u64c + 65 : nullptr, BoxTable{}, gate);
         } else {
-            if (!ctx->rare) CHK(dalloc(ctx, &ctx->rare, ctx->cap));
-            const ForceRows a{ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->all_active ? nullptr : ctx->ACT, ctx->TB,
-                              ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2, ctx->counters + 4, nullptr,
-                              ctx->sched_valid ? ctx->sched : nullptr, ctx->rare};
-            const dim3 grid = xcd_grid(nblk(ctx->nact));
-            // one kernel with the whole ladder when most rows took a later rung in the last pass
-            // (the two kernels then evaluate most rows twice): by the option "force_split", or
-            // on its default by the last pass's share of such rows in the FP32 form (where the
-            // whole ladder costs few registers more; the FP64 whole-ladder kernel spills)
-            const bool single = ctx->force_split == 0 ||
-                                (ctx->force_split < 0 && std::is_same<R, float>::value && ctx->rare_share > kRareShareSingle);
-            ctx->split_ran = !ctx->rung_stats && !single;
-            if (ctx->rung_stats) {
-                k_force<KERN, R, false, true, false><<<grid, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
-            } else if (single) {
-                k_force<KERN, R, false, false, false><<<grid, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
-            } else {
-                // the rows whose faces all take the Riemann ladder's common case, then the others
-                // with the whole ladder
-                // FP64: two or three waves per SIMD by the option "force_waves" (default: three
-                // with the search over many levels, else two)
-                const int waves = ctx->force_waves ? ctx->force_waves : (ctx->wide ? 3 : 2);
-                if constexpr (std::is_same<R, double>::value) {
-                    if (waves == 3)
-                        k_force_w3<KERN><<<grid, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
-                    else
-                        k_force<KERN, R, false, false, true><<<grid, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a,
-                                                                                                BoxTable{});
+            // the stored fluxes: a buffer of their own, or (in a pool, or without memory for it) what
+            // is left of the pool or the density sums, which are free now
+            void *flux = ctx->flux;
+            ForcePlan plan = force_plan<R>(ctx->nact, ~(size_t)0);
+            if (ctx->flux_bytes < plan.bytes) {
+                const size_t sums = (size_t)kDensSumsFD * ctx->cap * sizeof(double);
+                if (ctx->pool) {
+                    const size_t at = (ctx->pool_used + 255) & ~(size_t)255;
+                    const size_t left = at < ctx->pool_size ? ctx->pool_size - at : 0;
+                    flux = left > sums ? (void *)(ctx->pool + at) : (void *)ctx->dacc;
+                    plan = force_plan<R>(ctx->nact, std::max(left, sums));
+                } else if (dalloc(ctx, (char **)&ctx->flux, plan.bytes) == 0) {
+                    flux = ctx->flux;
+                    ctx->flux_bytes = plan.bytes;
                 } else {
-                    k_force<KERN, R, false, false, true><<<grid, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
+                    ctx->flux_bytes = 0;
+                    flux = ctx->dacc;
+                    plan = force_plan<R>(ctx->nact, sums);
                 }
-                k_force_rare<KERN, R, false><<<std::min(nblk(ctx->nact), kRareBlocks), kBlock, 0, ctx->stream>>>(
-                    ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
             }
+            const ForceRows a{ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->all_active ? nullptr : ctx->ACT, ctx->TB,
+                              ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2, ctx->counters + 4,
+                              ctx->sched_valid ? ctx->sched : nullptr, flux, plan.segment, ctx->force_split != 0 && !ctx->rung_stats};
+            auto lanes_kernel = ctx->rung_stats ? k_force<KERN, R, false, true> : k_force<KERN, R, false, false>;
+            lanes_kernel<<<plan.blocks, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
         }
         // the pairs of the pass: each row's workgroup adds its own while a few hundred rows are
         // active (atomics on one address execute one after another)
@@ -1235,11 +1224,6 @@ int force_stage(gz_context *ctx)
         HIPCHK(hipGetLastError());
     }
     CHK(read_counters(ctx));
-    if (ctx->split_ran) {
-        // rows the common kernel left to k_force_rare (err[12] = counters[14])
-        ctx->rare_share = (double)ctx->hcounters[14] / (double)std::max(ctx->nact, 1);
-        ctx->split_ran = false;
-    }
     if (ctx->spec) {
         ctx->spec = false;
         const int g = ctx->hcounters[kPassGate];
@@ -1262,7 +1246,7 @@ int force_stage(gz_context *ctx)
             return rc;
         }
     }
-    // rows the common kernel left to the whole Riemann ladder (counters[14]: zero unless it ran)
+    // rows with a face past the Riemann ladder's common case (counters[14]: zero unless counted)
     if (ctx->nact > ctx->few_rows && !ctx->rung_stats) ctx->st.force_rare_rows += ctx->hcounters[14];
     if (ctx->lazy && ctx->hmax_bound > 0) {
         // the radii the passes' lazy drifts produced (u64c[75], read back with the counters)
@@ -2118,8 +2102,8 @@ int gz_set_option(gz_context *ctx, const char *name, double value)
         return 0;
     }
     if (k == "force_waves") {
+        // kept for callers of earlier versions: one kernel serves every setting
         if (value != 0 && value != 2 && value != 3) return fail(ctx, GZ_E_ARG, "force_waves must be 0, 2 or 3");
-        ctx->force_waves = (int)value;
         return 0;
     }
     if (k == "force_split") {

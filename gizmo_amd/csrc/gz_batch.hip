@@ -79,8 +79,9 @@ struct gz_batch {
     double *it_h = nullptr, *it_hb = nullptr, *it_l = nullptr, *it_r = nullptr, *it_cn = nullptr;
     int *it_ci = nullptr, *it_it = nullptr;
     void *rec_grad = nullptr, *rec_force = nullptr;
+    void *flux = nullptr;  // the force pass's stored fluxes
+    size_t flux_bytes = 0;
     int *ell = nullptr, *cnt = nullptr;
-    int *rare = nullptr;  // rows the force pass's common kernel leaves to the whole Riemann ladder
     int ell_cap = 0;
     void *tmp = nullptr;
     size_t tmp_bytes = 0;
@@ -225,13 +226,16 @@ int alloc_all(gz_batch *b)
     BCHK(balloc(b, &b->T, 6 * n)); BCHK(balloc(b, &b->FW, 3 * n)); BCHK(balloc(b, &b->GR, 3 * n)); BCHK(balloc(b, &b->GP, 3 * n));
     BCHK(balloc(b, &b->GV, 9 * n)); BCHK(balloc(b, &b->ACC, 3 * n)); BCHK(balloc(b, &b->stage, 9 * n)); BCHK(balloc(b, &b->dacc, kDensSumsFD * n));
     BCHK(balloc(b, &b->TIB, n)); BCHK(balloc(b, &b->DTS, n));
-    int **i1[] = {&b->TB, &b->WAKE, &b->BOX, &b->perm, &b->ival, &b->ival2, &b->act, &b->it_ci, &b->it_it, &b->cnt, &b->rare};
+    int **i1[] = {&b->TB, &b->WAKE, &b->BOX, &b->perm, &b->ival, &b->ival2, &b->act, &b->it_ci, &b->it_it, &b->cnt};
     for (auto p : i1) BCHK(balloc(b, p, n));
     BCHK(balloc(b, &b->iflag, n + 1)); BCHK(balloc(b, &b->iscan, n + 1));
     BCHK(balloc(b, &b->ACT, n)); BCHK(balloc(b, &b->need, n));
     BCHK(balloc(b, &b->key, n)); BCHK(balloc(b, &b->key64, n)); BCHK(balloc(b, &b->key64b, n));
     BCHK(balloc(b, (char **)&b->rec_grad, n * sizeof(GradRec<double>)));
     BCHK(balloc(b, (char **)&b->rec_force, n * sizeof(Cell<double>)));
+    // room for the force pass's stored fluxes of every row of the batch
+    b->flux_bytes = b->par.precision == GZ_FP64 ? force_plan<double>(b->cap, ~(size_t)0).bytes : force_plan<float>(b->cap, ~(size_t)0).bytes;
+    BCHK(balloc(b, (char **)&b->flux, b->flux_bytes));
     const size_t nbx = nbox_all(b);
     BCHK(balloc(b, &b->tab, nbx)); BCHK(balloc(b, &b->hist, 64 * nbx)); BCHK(balloc(b, &b->slot, kBoxSlots * nbx));
     BCHK(balloc(b, &b->sel, nbx)); BCHK(balloc(b, &b->due, nbx)); BCHK(balloc(b, &b->rank, nbx)); BCHK(balloc(b, &b->lim, 2 * nbx));
@@ -253,10 +257,10 @@ void free_all(gz_batch *c)
                      &c->ACC, &c->stage, &c->dacc, &c->chmax};
     for (auto p : d1) bfree(*p);
     int **i1[] = {&c->TB, &c->WAKE, &c->BOX, &c->perm, &c->ival, &c->ival2, &c->act, &c->it_ci, &c->it_it, &c->cnt, &c->iflag,
-                  &c->iscan, &c->rank, &c->lim, &c->counters, &c->ell, &c->cstart, &c->cend, &c->rare};
+                  &c->iscan, &c->rank, &c->lim, &c->counters, &c->ell, &c->cstart, &c->cend};
     for (auto p : i1) bfree(*p);
     bfree(c->TIB); bfree(c->DTS); bfree(c->ACT); bfree(c->need); bfree(c->sel); bfree(c->due);
-    bfree(c->key); bfree(c->key64); bfree(c->key64b); bfree(c->rec_grad); bfree(c->rec_force); bfree(c->tab);
+    bfree(c->key); bfree(c->key64); bfree(c->key64b); bfree(c->rec_grad); bfree(c->rec_force); bfree(c->flux); bfree(c->tab);
     bfree(c->hist); bfree(c->slot); bfree(c->u64);
     bfree(c->tmp);
     {
@@ -626,12 +630,10 @@ int gradients_force(gz_batch *b)
     else
         k_pack_force<R><<<nb(b->cap), kB, 0, b->stream>>>(b->par.gamma, F, rf, b->counters + 2, 1.0, bt);
     if (lanes) {
-        // the rows whose faces all take the Riemann ladder's common case, then the others with the
-        // whole ladder
+        const ForcePlan plan = force_plan<R>(na, b->flux_bytes);
         const ForceRows a{na, b->act, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV, b->WAKE, b->ACC, b->DTU, b->MSV, b->counters + 2,
-                          b->counters + 4, nullptr, nullptr, b->rare};
-        k_force<KERN, R, true, false, true><<<xcd_grid(nb(na)), kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);
-        k_force_rare<KERN, R, true><<<std::min(nb(na), kRareBlocks), kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);
+                          b->counters + 4, nullptr, b->flux, plan.segment, 0};
+        k_force<KERN, R, true><<<plan.blocks, kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);
     } else {
         k_force_rows<KERN, R><<<xcd_grid(na), kListThreads, 0, b->stream>>>(b->dp, G, na, b->act, F, rf, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV,
                                                                    b->WAKE, b->ACC, b->DTU, b->MSV, b->counters + 2, b->counters + 4,

@@ -118,17 +118,33 @@ __device__ __forceinline__ void kernel_main(R u, R hinv3, R hinv4, R &wk, R &dwk
     kernel_main_q<KERN, MODE, R>(u, R(1) - u, hinv3, hinv4, wk, dwk);
 }
 
+// a / b, correctly rounded in both forms (the FP32 form's plain division is approximate, and the
+// compiler makes it exact where it moves it out of a loop): for quantities of the row alone, whose
+// bits must not depend on where a kernel evaluates them
+template <typename R>
+__device__ __forceinline__ R exact_div(R a, R b)
+{
+    return (R)((double)a / (double)b);
+}
+
 // The kernel of a pair at distance r from a particle of radius h (wk, dwk left as they are
 // beyond h).  FP64 form: the reference's kernel_hinv and kernel_main at u = r / h.  FP32 form:
 // the edge factor 1 - u from the FP64 distance rd and radius h, the rest in FP32.  A partner
 // near the edge of h sits where the kernel is steep (W ~ (1 - u)^4), so the FP32 rounding of r
 // and h would enter its weight many times over: a hot partner at u = 0.993 of a cold particle
 // carries most of its pressure gradient, and an FP32 u moves that gradient by 5e-5.
-template <int KERN, int MODE, typename R>
+// ROW: h is the row's own radius (exact_div).
+template <int KERN, int MODE, typename R, bool ROW = false>
 __device__ __forceinline__ void pair_kernel(R r, double rd, double h, R &wk, R &dwk)
 {
     R hinv, hinv3, hinv4;
-    kernel_hinv((R)h, hinv, hinv3, hinv4);
+    if constexpr (ROW) {
+        hinv = exact_div(R(1.0), (R)h);
+        hinv3 = hinv * hinv * hinv;
+        hinv4 = hinv3 * hinv;
+    } else {
+        kernel_hinv((R)h, hinv, hinv3, hinv4);
+    }
     if constexpr (std::is_same<R, double>::value) {
         (void)rd;
         if (r < h) kernel_main<KERN, MODE>(r * hinv, hinv3, hinv4, wk, dwk);
@@ -608,6 +624,14 @@ __device__ inline R guess_p(const Gam<R> &G, const RState<R> &L, const RState<R>
     return x;
 }
 
+// (p / p_k)^((gamma - 1) / (2 gamma)) of a rarefaction, p <= p_k.  The logarithm times the exponent
+// is of order one, so the exponential's result is within an ulp or two of pow()'s, at a third of
+// its instructions; the wave's slope needs the power -(gamma + 1) / (2 gamma), this one over the
+// pressure ratio (the exponents add to -1).  A wavefront's Newton step costs ~350 instructions
+// instead of ~960 as soon as one of its lanes is in a rarefaction.
+template <typename R>
+__device__ __forceinline__ R rarefaction_power(const Gam<R> &G, R ratio) { return exp(G.G1 * log(ratio)); }
+
 template <typename R>
 __device__ inline int iterative_riemann(const Gam<R> &G, const RState<R> &L, const RState<R> &Rs, R vL, R vR, R csL, R csR, ROut<R> &o)
 {
@@ -643,18 +667,18 @@ __device__ inline int iterative_riemann(const Gam<R> &G, const RState<R> &L, con
             WL = (Pg - L.p) * a2;
             ZL = a2 * (R(1.0) - R(0.5) * (Pg - L.p) / (a1 + Pg));
         } else {
-            R pr = Pg / L.p;
-            WL = G.G4 * csL * (pow(pr, G.G1) - R(1));
-            ZL = R(1) / (L.rho * csL) * pow(Pg / L.p, -G.G2);
+            const R pr = Pg / L.p, w = rarefaction_power(G, pr);
+            WL = G.G4 * csL * (w - R(1));
+            ZL = R(1) / (L.rho * csL) * (w / pr);
         }
         if (Pg > Rs.p) {
             R a0 = G.G5 / Rs.rho, a1 = G.G6 * Rs.p, a2 = sqrt(a0 / (Pg + a1));
             WR = (Pg - Rs.p) * a2;
             ZR = a2 * (R(1.0) - R(0.5) * (Pg - Rs.p) / (a1 + Pg));
         } else {
-            R pr = Pg / Rs.p;
-            WR = G.G4 * csR * (pow(pr, G.G1) - R(1));
-            ZR = R(1) / (Rs.rho * csR) * pow(pr, -G.G2);
+            const R pr = Pg / Rs.p, w = rarefaction_power(G, pr);
+            WR = G.G4 * csR * (w - R(1));
+            ZR = R(1) / (Rs.rho * csR) * (w / pr);
         }
         if (it < 1000 / 2) Pg -= (WL + WR + dvel) / (ZL + ZR);
         else Pg -= R(0.5) * (WL + WR + dvel) / (ZL + ZR);
@@ -811,12 +835,14 @@ __device__ inline bool riemann_ladder(const Gam<T> &G, RState<T> L, RState<T> Rs
     o.P_M = o.S_M = o.f0 = o.f1 = o.f2 = o.fp = 0;
     rung |= riemann(G, L, Rs, n, ptl, o);
     if ((o.P_M < 0) || (isnan(o.P_M)) || (o.P_M > T(1.4) * ptl)) {
-        Rs.p = pI; L.p = pJ; Rs.rho = rhoI; L.rho = rhoJ;
+        // (rounded: the row's own state stays in this branch, where the FP32 form's divisions by it
+        // round alike in every kernel; moved out of a loop they would be exact)
+        Rs.p = rounded(pI); L.p = pJ; Rs.rho = rounded(rhoI); L.rho = rhoJ;
         Rs.v0 = vi0; Rs.v1 = vi1; Rs.v2 = vi2;
         L.v0 = vj0; L.v1 = vj1; L.v2 = vj2;
         rung |= kRungRetryFirstOrder | riemann(G, L, Rs, n, T(1.4) * ptl, o);
         if ((o.P_M < 0) || (isnan(o.P_M))) {
-            Rs.p = pI; L.p = pJ; Rs.rho = rhoI; L.rho = rhoJ;
+            Rs.p = rounded(pI); L.p = pJ; Rs.rho = rounded(rhoI); L.rho = rhoJ;
             Rs.v0 = Rs.v1 = Rs.v2 = 0; L.v0 = L.v1 = L.v2 = 0;
             rung |= kRungRetryZeroVel | riemann(G, L, Rs, n, T(2.0) * ptl, o);
             if ((o.P_M < 0) || (isnan(o.P_M))) { rung |= kRungFail; return false; }
@@ -828,8 +854,8 @@ __device__ inline bool riemann_ladder(const Gam<T> &G, RState<T> L, RState<T> Rs
 // The common case of the ladder alone: physical reconstructed states whose wave-speed estimate
 // (HLLC, Roe or PVRS) gives a positive pressure within the limiter.  The ladder then takes no
 // other rung, so the result is the ladder's, bit for bit.  false: the face needs the rest of the
-// ladder (KT, the exact solver or a retry), which a kernel that calls this leaves to a second
-// pass over its rows (the rare rungs' code then costs the common pass no registers).
+// ladder (KT, the exact solver or a retry), which a kernel that calls this takes with the whole
+// ladder later, together with other lanes' such faces.
 template <typename T>
 __device__ __forceinline__ bool riemann_common(const Gam<T> &G, const RState<T> &L, const RState<T> &Rs, const T *n, T ptl,
                                                ROut<T> &o, unsigned &rung)
@@ -847,27 +873,54 @@ __device__ __forceinline__ bool riemann_common(const Gam<T> &G, const RState<T> 
     return true;
 }
 
-// A row's force record with the fields of the reconstruction, the faces and the entropic switch
-// in LDS (ColdRec, 26 values: 208 B per lane in FP64, three workgroups of 256 per CU) and the
-// rest in registers: the record of i then costs a pair loop 12 registers instead of 64.
-template <typename R> struct ColdRec {
-    R m, p, cn, fce, drk, gr0, gr1, gr2, gp0, gp1, gp2;
-    R gv[9];
-    R t[6];
+// A force record staged in LDS by a quad of lanes (stage_records).  Its 16-byte pieces lie four
+// (one 64-byte block) by four, the blocks kBlock bytes apart; a last half block lies apart from
+// them (at half()), those of two lanes side by side.  The fields are read where the pair body
+// uses them, so the record of j costs a pair loop few registers.
+template <typename R> struct StagedRec {
+    static constexpr int kBytes = (int)sizeof(Cell<R>);
+    static constexpr int kBlocks = kBytes / 64;                          // whole blocks
+    static constexpr bool kHalf = kBytes % 64 != 0;
+    static_assert(kBytes % 64 == 0 || kBytes % 64 == 32, "whole and half blocks");
+    static constexpr int kBlock = 1024;                                  // one load instruction: 64 lanes x 16 B
+    static constexpr int kQuadRow = kBlocks * kBlock + 16;               // the quads' k-th rows (16: no bank conflicts among a quad's reads)
+    static constexpr int kHalfAt = 4 * kQuadRow;
+    static constexpr int kWave = kHalfAt + (kHalf ? 2 * kBlock : 0);     // LDS bytes of a wavefront
+    // LDS offset of a lane's record in its wavefront's area, and of its half block's pieces from there
+    __device__ static int lane_at(int lane) { return (lane & 3) * kQuadRow + (lane >> 2) * 64; }
+    __device__ static int half_at(int lane) { return kHalfAt + ((lane >> 1) & 1) * kBlock + (lane >> 2) * 64 + (lane & 1) * 32; }
 };
-template <typename R> struct SplitCell {
-    R h, rho, cs, v0, v1, v2;
-    const R &m, &p, &cn, &fce, &drk, &gr0, &gr1, &gr2, &gp0, &gp1, &gp2;
-    const R (&gv)[9];
-    const R (&t)[6];
+template <typename R, int OFF> struct StagedArr {
+    const unsigned char *b, *e;
+    __device__ __forceinline__ const R &operator[](int k) const
+    {
+        const int off = OFF + k * (int)sizeof(R), whole = StagedRec<R>::kBlocks * 64;
+        return *reinterpret_cast<const R *>(off < whole ? b + (off >> 6) * StagedRec<R>::kBlock + (off & 63) : e + (off - whole));
+    }
+};
+template <typename R> struct StagedCell {
+    static constexpr int H0 = std::is_same<R, float>::value ? 16 : 0, S0 = H0 + 8, W = (int)sizeof(R);
+    static_assert(sizeof(Cell<R>) == ((S0 + 31 * W + 15) & ~15), "the offsets below are the record's");
+    StagedArr<R, S0> s;
+    const double &h;
+    const R &m, &rho, &p, &cs, &cn, &fce, &drk, &v0, &v1, &v2, &gr0, &gr1, &gr2, &gp0, &gp1, &gp2;
+    StagedArr<R, S0 + 16 * W> gv;
+    StagedArr<R, S0 + 25 * W> t;
+    __device__ __forceinline__ StagedCell(const unsigned char *b, const unsigned char *e)
+        : s{b, e}, h(*reinterpret_cast<const double *>(b + H0)), m(s[0]), rho(s[1]), p(s[2]), cs(s[3]), cn(s[4]), fce(s[5]), drk(s[6]),
+          v0(s[7]), v1(s[8]), v2(s[9]), gr0(s[10]), gr1(s[11]), gr2(s[12]), gp0(s[13]), gp1(s[14]), gp2(s[15]), gv{b, e}, t{b, e}
+    {
+    }
+    // the fine position (FP32 form)
+    __device__ __forceinline__ const FinePos &fp() const { return *reinterpret_cast<const FinePos *>(s.b); }
 };
 
 // returns 0 skipped, 1 fluxes produced (maybe zero), -1 no Riemann solution (stop 1234), 2 (COMMON
 // only) the face needs a rare rung of the ladder; rung receives the RiemannRung bits of the face
 // (callers that do not count them leave it unused).  COMMON: the Riemann solve takes only the
-// ladder's common case (riemann_common).  IC: the record of i (Cell<R> or SplitCell<R>).
-template <int KERN, typename R, bool COMMON = false, typename IC = Cell<R>>
-__device__ inline int force_pair(const DevParams &P, const Gam<R> &G, const IC &I, const Cell<R> &J, R dp0, R dp1, R dp2, R r2,
+// ladder's common case (riemann_common).  JC: the record of j (Cell<R> or StagedCell<R>).
+template <int KERN, typename R, bool COMMON = false, typename JC = Cell<R>>
+__device__ inline int force_pair(const DevParams &P, const Gam<R> &G, const Cell<R> &I, const JC &J, R dp0, R dp1, R dp2, R r2,
                                  R &F0, R &F1, R &F2, R &Fp, R &vsig_ts, unsigned &rung)
 {
     rung = 0;
@@ -885,14 +938,14 @@ __device__ inline int force_pair(const DevParams &P, const Gam<R> &G, const IC &
     R wk_i = 0, dwk_i = 0, wk_j = 0, dwk_j = 0;
     {
         const double rd = std::is_same<R, double>::value ? 0.0 : sqrt(r2d);
-        pair_kernel<KERN, 0, R>(r, rd, I.h, wk_i, dwk_i);
+        pair_kernel<KERN, 0, R, true>(r, rd, I.h, wk_i, dwk_i);
         pair_kernel<KERN, 0, R>(r, rd, J.h, wk_j, dwk_j);
     }
     const R cnumcrit2 = R(kCnDanger) * R(kCnDanger) - I.cn * I.cn;
     const R vdotr2 = dp0 * dv0 + dp1 * dv1 + dp2 * dv2;
     if (vdotr2 < 0) vsig -= R(1.0) * vdotr2 * rinv;
     vsig_ts = vsig + fabs(I.cs - J.cs);
-    const R V_i = I.m / I.rho;
+    const R V_i = exact_div(I.m, I.rho);
     const R V_j = J.m / J.rho;
     const R leak = R(0.5) * (I.fce + J.fce);
     // faces
@@ -997,7 +1050,7 @@ __device__ inline int force_pair(const DevParams &P, const Gam<R> &G, const IC &
             R du_new = R(0.5) * (pdvi - pdvj + fpm * (fvi + fvj));
             R cnum2 = J.cn * J.cn;
             R ratio = R(1.001);
-            R toi = I.p / I.rho, toj = J.p / J.rho;
+            R toi = exact_div(I.p, I.rho), toj = J.p / J.rho;
             if (use && smc > R(1.e-3) && cnum2 < cnumcrit2) {
                 if (toi > ratio * toj) {
                     R dtoj = -du_old + fpm * fvj;

@@ -370,34 +370,50 @@ struct ForceRows {
     double *ACC, *DTU, *MSV;     // outputs
     int *err;                    // err[0] stop code; err[10], err[11] the first pair without a solution; err[12] rare rows
     int *need_wakeup;            // set when a neighbour is flagged (one box)
-    unsigned long long *pairs;   // the pass's pair count (nullptr: not counted)
     const int *sched;            // row order (nullptr: 0..nrows-1)
-    int *rare;                   // rows the common pass leaves to the whole ladder
+    void *flux;                  // scratch: a segment's fluxes of each workgroup (ForcePlan)
+    int segment;                 // list entries of a row between two rounds of queued faces
+    int count_rare;              // count the rows with a face past the Riemann ladder's common case into err[12]
 };
 
-// Lane per row.  STATS: count the faces' RiemannRung bits into F.rungs.  COMMON: every face takes
-// only the Riemann ladder's common case (riemann_common); a row with a face that needs more is
-// not written but appended to a.rare (count in a.err[12]), for k_force_rare.  The common pass
-// then carries no register cost of the rare rungs.
-template <int KERN, typename R, bool BOXES, bool STATS = false, bool COMMON = false>
+// Four lanes per row, kForceRowsPerBlock rows per workgroup at a time, on force_blocks() workgroups.
+// STATS: count the faces' RiemannRung bits into F.rungs.
+template <int KERN, typename R, bool BOXES, bool STATS = false>
 __global__ void k_force(DevParams P, Gam<R> G, ForceView F, const Cell<R> *rec, ForceRows a, BoxTable bt);
-// k_force<KERN, double, false, false, true> at three waves per SIMD instead of two (option "force_waves")
-template <int KERN>
-__global__ void k_force_w3(DevParams P, Gam<double> G, ForceView F, const Cell<double> *rec, ForceRows a, BoxTable bt);
-
-// the rows that k_force<..., COMMON> listed, each with the whole ladder (a fixed grid strides over
-// the count the device holds; the rows' results are the single-pass kernel's, bit for bit)
-constexpr unsigned kRareBlocks = 1024;  // workgroups of 256 at most that k_force_rare launches
-// FP32 force pass over many rows: above this share of rows left to k_force_rare by the last
-// pass, the next pass runs one kernel with the whole ladder (the two kernels would evaluate
-// most rows twice)
-constexpr double kRareShareSingle = 0.25;
+constexpr int kForceRowsPerBlock = 64;
+// at most this many list entries of a row between two rounds of queued faces: the lists of 64
+// neighbours (at most ~90 entries) in one segment, and a queue that leaves room for the LDS of
+// two workgroups on a CU
+constexpr int kForceSegment = 96;
+// workgroups of the fixed grid: two (FP64) or three (FP32) per CU of 256, by their LDS and registers
+template <typename R> constexpr int kForceBlocks = 2 * 256;
+// The launch of a pass over nrows rows with at most `room` bytes for the stored fluxes (a segment's
+// entries x rows x 4 per workgroup; the whole grid with whole segments takes up to 100 MB).  Less
+// room: shorter segments, at least eight entries, and then fewer workgroups.
+struct ForcePlan {
+    int blocks, segment;
+    size_t bytes;
+};
+template <typename R> inline ForcePlan force_plan(long nrows, size_t room)
+{
+    const long nrb = (nrows + kForceRowsPerBlock - 1) / kForceRowsPerBlock;
+    const size_t entry = (size_t)kForceRowsPerBlock * 4 * sizeof(R);
+    long blocks = (long)xcd_grid(nrb < kForceBlocks<R> ? nrb : kForceBlocks<R>);
+    long seg = (long)(room / ((size_t)blocks * entry));
+    if (seg > kForceSegment) seg = kForceSegment;
+    if (seg < 8) {
+        seg = 8;
+        blocks = (long)(room / (seg * entry)) / kXcds * kXcds;
+        if (blocks < kXcds) {
+            blocks = kXcds;
+            seg = (long)(room / (blocks * entry));
+        }
+    }
+    return ForcePlan{(int)blocks, (int)seg, (size_t)blocks * seg * entry};
+}
 // few-row force passes over at most this many rows make their records in the row kernel (its
 // MAKE form holds one wave per SIMD: this many rows of two wavefronts fill the chip once)
 constexpr int kMakeForceRows = 512;
-template <int KERN, typename R, bool BOXES>
-__global__ void k_force_rare(DevParams P, Gam<R> G, ForceView F, const Cell<R> *rec, ForceRows a, BoxTable bt);
-
 // the Riemann functions on given face states (diagnostic; layout of in/out at the definition)
 constexpr int kProbeIn = 24, kProbeOut = 8;
 template <typename R>

@@ -1248,151 +1248,296 @@ __device__ inline void force_tail(const DevParams &P, const ForceView &F, int i,
     MSV[i] = ms;
 }
 
-// the record of i a pair loop reads: the record itself, or its split over registers and LDS
-template <typename R>
-__device__ __forceinline__ Cell<R> make_irec(const Cell<R> &I, const ColdRec<R> &, std::false_type) { return I; }
-template <typename R>
-__device__ __forceinline__ SplitCell<R> make_irec(const Cell<R> &I, const ColdRec<R> &C, std::true_type)
+// The records of the lanes' partners into LDS: the four lanes of a quad load one record after the
+// other, 16 bytes per lane and instruction, straight into LDS (a lane loading its own record
+// would touch one cache line per lane and instruction).  Every lane of the wavefront calls it;
+// want: the lane's j is to be loaded.  The caller waits for the loads (wait_staged) before it
+// reads them, and has read what it needs of the area's last contents.
+__device__ __forceinline__ void lds_load16(const char *src, unsigned char *lds)
 {
-    return SplitCell<R>{I.h, I.rho, I.cs, I.v0, I.v1, I.v2, C.m, C.p, C.cn, C.fce, C.drk, C.gr0, C.gr1, C.gr2, C.gp0, C.gp1, C.gp2,
-                        C.gv, C.t};
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
+}
+template <typename R, int K>
+__device__ __forceinline__ void stage_quad_row(const Cell<R> *__restrict__ rec, int j, int want, unsigned char *wave_lds)
+{
+    using S = StagedRec<R>;
+    const int jk = __builtin_amdgcn_mov_dpp(j, K * 0x55, 0xf, 0xf, true);  // lane K of the quad
+    const int wk = __builtin_amdgcn_mov_dpp(want, K * 0x55, 0xf, 0xf, true);
+    const char *src = (const char *)(rec + jk) + (threadIdx.x & 3) * 16;
+    if (wk) {
+#pragma unroll
+        for (int b = 0; b < S::kBlocks; b++) lds_load16(src + b * 64, wave_lds + K * S::kQuadRow + b * S::kBlock);
+    }
+}
+// the half blocks of the quad's rows 2 K (lanes 0 and 1) and 2 K + 1 (lanes 2 and 3)
+template <typename R, int K>
+__device__ __forceinline__ void stage_quad_half(const Cell<R> *__restrict__ rec, int j, int want, unsigned char *wave_lds)
+{
+    using S = StagedRec<R>;
+    constexpr int perm = 2 * K | (2 * K) << 2 | (2 * K + 1) << 4 | (2 * K + 1) << 6;
+    const int jk = __builtin_amdgcn_mov_dpp(j, perm, 0xf, 0xf, true);
+    const int wk = __builtin_amdgcn_mov_dpp(want, perm, 0xf, 0xf, true);
+    if (wk) lds_load16((const char *)(rec + jk) + S::kBlocks * 64 + (threadIdx.x & 1) * 16, wave_lds + S::kHalfAt + K * S::kBlock);
+}
+template <typename R>
+__device__ __forceinline__ void stage_records(const Cell<R> *__restrict__ rec, int j, bool want, unsigned char *wave_lds)
+{
+    // reads and writes of the area's last contents are done
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    stage_quad_row<R, 0>(rec, j, want, wave_lds);
+    stage_quad_row<R, 1>(rec, j, want, wave_lds);
+    stage_quad_row<R, 2>(rec, j, want, wave_lds);
+    stage_quad_row<R, 3>(rec, j, want, wave_lds);
+    if constexpr (StagedRec<R>::kHalf) {
+        stage_quad_half<R, 0>(rec, j, want, wave_lds);
+        stage_quad_half<R, 1>(rec, j, want, wave_lds);
+    }
+}
+__device__ __forceinline__ void wait_staged() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// the difference of a pair's positions from the staged record of j (FP32 form) or the position
+// arrays (FP64 form)
+template <typename R>
+__device__ __forceinline__ void staged_dp(const DevParams &P, const Cell<R> &I, const StagedCell<R> &J, double xi, double yi, double zi,
+                                          double xj, double yj, double zj, R &dp0, R &dp1, R &dp2)
+{
+    if constexpr (std::is_same<R, float>::value) {
+        fine_dp(I.fp, J.fp(), (float)(P.box * (1.0 / 1024.0)), dp0, dp1, dp2);
+    } else {
+        const double inv_box = 1.0 / P.box;
+        dp0 = wrap_near(xi - xj, P.box, inv_box);
+        dp1 = wrap_near(yi - yj, P.box, inv_box);
+        dp2 = wrap_near(zi - zj, P.box, inv_box);
+    }
 }
 
-// One row of the lane-per-row force kernels; false (COMMON only): a face of the row needs a rare
-// rung of the Riemann ladder, and nothing of the row was written but its neighbours' wake-up
-// flags (which the whole-ladder pass over the row sets again, to the same values)
-template <int KERN, typename R, bool BOXES, bool STATS, bool COMMON>
-__device__ __forceinline__ bool force_row(const DevParams &P0, const Gam<R> &G, const ForceView &F, const Cell<R> *__restrict__ rec,
-                                          const ForceRows &a, const BoxTable &bt, int r)
+// What a pair's fluxes leave besides the sums: a failed solve, and the wake-up of an inactive
+// neighbour (rc, vts: force_pair's)
+template <bool BOXES, typename R>
+__device__ __forceinline__ void pair_flags(const ForceRows &a, const BoxTable &bt, int i, int j, int rc, R vts)
 {
-    DevParams P = P0;
-    const int i = a.act[r];
-    if (BOXES) {
-        GridView g{};
-        resolve_box(bt, i, P, g);
+    if (rc < 0) {
+        atomicMax(a.err, 1234);
+        if (atomicCAS(a.err + 10, -1, i) == -1) a.err[11] = j;
     }
-    // hydro_force_initial_operations_preloop (src/hydro/hydro_toplevel.cc:457-565): an active
-    // particle's own flag is cleared; only inactive neighbours are flagged below
-    if (a.wakeup) a.wakeup[i] = 0;
-    const double mi = F.M[i], rhoi = F.RHO[i];
-    double A0 = 0, A1 = 0, A2 = 0, dE = 0, msv = 0;
-    // effective_soundspeed of i, src/declarations/cell_data.h:703-712 (floor of MaxSignalVel)
-    double sound_i = (rhoi > 0) ? sqrt(P.gamma * F.PR[i] / rhoi) : sqrt(P.gamma * (P.gamma - 1.) * F.U[i]);
-    const bool enabled = (mi > 0 && rhoi > 0);
-    if (enabled) {
-        const Cell<R> I0 = rec[i];
-        // the FP64 common pass keeps most of i's record in LDS (SplitCell); the other kernels
-        // hold it in registers
-        constexpr bool split = COMMON && std::is_same<R, double>::value;
-        __shared__ ColdRec<R> cold[split ? 256 : 1];
-        ColdRec<R> &C = cold[split ? threadIdx.x : 0];
-        if constexpr (split) {
-            C.m = I0.m; C.p = I0.p; C.cn = I0.cn; C.fce = I0.fce; C.drk = I0.drk;
-            C.gr0 = I0.gr0; C.gr1 = I0.gr1; C.gr2 = I0.gr2; C.gp0 = I0.gp0; C.gp1 = I0.gp1; C.gp2 = I0.gp2;
-            for (int k = 0; k < 9; k++) C.gv[k] = I0.gv[k];
-            for (int k = 0; k < 6; k++) C.t[k] = I0.t[k];
+    if (rc == 1 && a.active && !a.active[j] && a.wakeup) {
+        if ((double)vts > kWakeup * a.msv_in[j]) {
+            atomicMax(&a.wakeup[j], (a.timebin ? a.timebin[i] : 0) + 1);
+            if (BOXES) bt.b[bt.BOX[i]].need_wakeup = 1;
+            else *a.need_wakeup = 1;
         }
-        using IC = typename std::conditional<split, SplitCell<R>, Cell<R>>::type;
-        const IC I = make_irec<R>(I0, C, std::integral_constant<bool, split>{});
-        const double xi = F.X[i], yi = F.Y[i], zi = F.Z[i];
-        const int tbi = a.timebin ? a.timebin[i] : 0;
-        const int c = a.cnt[r];
-        CSum<R> a0, a1, a2, ae;
+    }
+}
+
+// The force pass over many rows: four lanes (a quad) per row, 64 rows per workgroup, the quad's
+// lanes on four consecutive list entries at a time.  A fixed number of workgroups (kForceBlocks)
+// walks the rows, each XCD through its own contiguous part, so that the rows in flight on an XCD
+// are consecutive and few (4096) and their partners' records (2.6 MB FP64) stay in its L2; one
+// lane per row had 16K rows in flight, whose records (7 MB) did not.
+//
+// The fluxes are added in list order: the quad's four entries go through LDS, and lane t of the
+// quad keeps sum t (momentum, energy) and adds the four in turn.  A face past the Riemann ladder's
+// common case (riemann_common; one in 14 to 300 on moving gas, but nearly every row has some) is
+// not taken where it comes up, where it would hold the other 63 lanes through the exact solver:
+// it goes to the workgroup's queue, and from there on its row's fluxes go to the workgroup's part
+// of `flux` instead of the sums.  After a segment of every row's list the queued faces are
+// taken together, 256 at a time, with the whole ladder, and the rows that wait for them add the
+// stored fluxes in list order.  Each row's sums are those of one loop over its list, bit for bit.
+// STATS: the faces' RiemannRung bits are counted.
+//
+// 2M rows of a box at Mach 0.3 (7% of the faces past the common case, 97% of the rows): FP64 22.7
+// -> 11.4 ms, FP32 12.3 -> 8.5 ms; 1M rows of a lognormal field (0.3% of the faces) FP64 10.4 ->
+// 5.4 ms; 15,625 rows FP32 1,120 -> 130 us (one lane per row left most of the chip idle).  The two
+// kernels before took a row again from its start at its first such face.  Waiting lanes in one
+// lane per row's loop (until 8, 24, 40 of 64 waited) took 18.9, 24.9, 36.9 ms: rows with many such
+// faces hold their wavefront.  Two wavefronts per SIMD: the record of the row and the whole
+// ladder take 256 registers (FP32 at three: spills, 10.8 ms).  Bound now by its VALU instructions
+// (half of the time) and the wait for the records between them.
+template <int KERN, typename R, bool BOXES, bool STATS>
+__global__ void __launch_bounds__(256, 2)
+    k_force(DevParams P0, Gam<R> G, ForceView F, const Cell<R> *__restrict__ rec, ForceRows a, BoxTable bt)
+{
+    using S = StagedRec<R>;
+    __shared__ __align__(16) unsigned char staged[4][S::kWave];
+    __shared__ unsigned short queue[kForceRowsPerBlock * kForceSegment];  // (list entry in the segment) * rows + row
+    __shared__ unsigned long long mrow[kForceRowsPerBlock];               // signal speeds of the queued faces (bits)
+    __shared__ int nqueue, cwave[2][4];  // (two: a wavefront may be one row block ahead)
+    const int tid = threadIdx.x, lane = tid & 63, t = tid & 3;
+    unsigned char *wave_lds = staged[tid >> 6];
+    const StagedCell<R> J(wave_lds + S::lane_at(lane), wave_lds + S::half_at(lane));
+    R(*flux)[kForceRowsPerBlock][4] = (R(*)[kForceRowsPerBlock][4])a.flux + (size_t)blockIdx.x * a.segment;
+    // the row blocks of this workgroup: one of every (grid / 8) of its XCD's contiguous eighth, its
+    // place among them shifted each turn (the row order repeats from long lists to short ones)
+    const int nrb = (a.nrows + kForceRowsPerBlock - 1) / kForceRowsPerBlock;
+    const int per = (nrb + kXcds - 1) / kXcds, xcd = blockIdx.x % kXcds, nx = gridDim.x / kXcds;
+    int rare_rows = 0;
+    if (tid == 0) nqueue = 0;
+    for (int b0 = 0, place = blockIdx.x / kXcds, turn = 0; b0 < per; b0 += nx, turn ^= 1) {
+        const int b = b0 + place, rb = xcd * per + b;
+        place += 13;
+        while (place >= nx) place -= nx;
+        if (b >= per || rb >= nrb) continue;
+        const int k = rb * kForceRowsPerBlock + (tid >> 2);
+        const bool row = k < a.nrows;
+        const int r = row ? (a.sched ? a.sched[k] : k) : 0;
+        const int i = row ? a.act[r] : 0;
+        DevParams P = P0;
+        if (BOXES && row) {
+            GridView g{};
+            resolve_box(bt, i, P, g);
+        }
+        // hydro_force_initial_operations_preloop (src/hydro/hydro_toplevel.cc:457-565): an active
+        // particle's own flag is cleared; only inactive neighbours are flagged below
+        if (row && t == 0 && a.wakeup) a.wakeup[i] = 0;
+        const double mi = row ? F.M[i] : 0, rhoi = row ? F.RHO[i] : 0;
+        const bool enabled = row && mi > 0 && rhoi > 0;
+        const int c = enabled ? a.cnt[r] : 0;
+        {
+            int cm = c;
+            for (int o = 32; o >= 4; o >>= 1) cm = max(cm, __shfl_xor(cm, o, 64));
+            if (lane == 0) cwave[turn][tid >> 6] = cm;
+        }
+        if (t == 0) mrow[tid >> 2] = 0;
+        __syncthreads();
+        const int cmax = max(max(cwave[turn][0], cwave[turn][1]), max(cwave[turn][2], cwave[turn][3]));
+        CSum<R> sum;
         R m = 0;
-        for (int q = 0; q < c; q++) {
-            // LDS reads of i's record stay inside the loop (not hoisted into registers)
-            if constexpr (split) __asm__ volatile("" ::: "memory");
-            const int j = a.ell[ell_at(a.ld, r, q)];
-            if (m < I.cs) m = I.cs;
-            const Cell<R> J = rec[j];
-            R dp0, dp1, dp2;
-            record_dp<R>(P, I0, J, xi, yi, zi, F.X, F.Y, F.Z, j, dp0, dp1, dp2);
-            const R r2 = dp0 * dp0 + dp1 * dp1 + dp2 * dp2;
-            R f0, f1, f2, fp, vts;
-            unsigned rung;
-            int rc = force_pair<KERN, R, COMMON>(P, G, I, J, dp0, dp1, dp2, r2, f0, f1, f2, fp, vts, rung);
-            if constexpr (STATS) count_rungs(F.rungs, rung);
-            if constexpr (COMMON) {
-                if (rc == 2) return false;
-            }
-            if (rc < 0) {
-                atomicMax(a.err, 1234);
-                if (atomicCAS(a.err + 10, -1, i) == -1) a.err[11] = j;
-                continue;
-            }
-            if (rc == 0) continue;
-            a0.add(rounded(f0)); a1.add(rounded(f1)); a2.add(rounded(f2)); ae.add(rounded(fp));
-            if (vts > m) m = vts;
-            if (a.active && !a.active[j] && a.wakeup) {
-                if ((double)vts > kWakeup * a.msv_in[j]) {
-                    atomicMax(&a.wakeup[j], tbi + 1);
-                    if (BOXES) bt.b[bt.BOX[i]].need_wakeup = 1;
-                    else *a.need_wakeup = 1;
+        bool had_rare = false;
+        for (int seg = 0; seg < cmax; seg += a.segment) {
+            const int cs = min(c - seg, a.segment);  // this row's entries of the segment
+            int first_rare = -1;                         // the first queued entry of the row
+            {
+                const Cell<R> I = rec[i];
+                const double xi = F.X[i], yi = F.Y[i], zi = F.Z[i];
+                if (cs > 0 && m < I.cs) m = I.cs;
+                int jn = t < cs ? a.ell[ell_at(a.ld, r, seg + t)] : 0;
+                for (int q0 = 0; __any(q0 < cs); q0 += 4) {
+                    const int q = q0 + t, j = jn;
+                    const bool go = q < cs;
+                    stage_records<R>(rec, j, go, wave_lds);
+                    double xj = 0, yj = 0, zj = 0;
+                    if (go) {
+                        if constexpr (std::is_same<R, double>::value) { xj = F.X[j]; yj = F.Y[j]; zj = F.Z[j]; }
+                        if (q + 4 < cs) jn = a.ell[ell_at(a.ld, r, seg + q + 4)];
+                    }
+                    wait_staged();
+                    int rc = 0;
+                    R f0 = 0, f1 = 0, f2 = 0, fp = 0;
+                    if (go) {
+                        R dp0, dp1, dp2, vts;
+                        unsigned rung;
+                        staged_dp<R>(P, I, J, xi, yi, zi, xj, yj, zj, dp0, dp1, dp2);
+                        rc = force_pair<KERN, R, true>(P, G, I, J, dp0, dp1, dp2, dp0 * dp0 + dp1 * dp1 + dp2 * dp2, f0, f1, f2, fp, vts, rung);
+                        if constexpr (STATS) {
+                            if (rc != 2) count_rungs(F.rungs, rung);
+                        }
+                        if (rc == 1 && vts > m) m = vts;
+                        pair_flags<BOXES>(a, bt, i, j, rc, vts);
+                    }
+                    // faces of this round that wait; the quad's first one closes its row
+                    const unsigned long long waits = __ballot(rc == 2);
+                    if (waits) {
+                        int base = 0;
+                        const int lead = __ffsll((long long)waits) - 1;
+                        if (lane == lead) base = atomicAdd(&nqueue, (int)__popcll(waits));
+                        base = __shfl(base, lead, 64);
+                        if (rc == 2) queue[base + __popcll(waits & ((1ull << lane) - 1ull))] = (unsigned short)(q * kForceRowsPerBlock + (tid >> 2));
+                        const unsigned mine = (unsigned)(waits >> (lane & ~3)) & 15u;
+                        if (first_rare < 0 && mine) first_rare = q0 + __ffs((int)mine) - 1;
+                    }
+                    const bool open = first_rare < 0 || q < first_rare;
+                    if (go && !open && rc != 2) {
+                        R *w = flux[q][tid >> 2];
+                        w[0] = rounded(f0); w[1] = rounded(f1); w[2] = rounded(f2); w[3] = rounded(fp);
+                    }
+                    // lane t adds component t of the quad's entries, in order (an entry that is not
+                    // added here counts as zeros, which leave a sum as it is)
+                    R *w = (R *)(wave_lds + (lane >> 2) * (16 * (int)sizeof(R) + 16)) + 4 * t;
+                    const bool add = rc == 1 && open;
+                    w[0] = add ? rounded(f0) : R(0); w[1] = add ? rounded(f1) : R(0);
+                    w[2] = add ? rounded(f2) : R(0); w[3] = add ? rounded(fp) : R(0);
+                    __builtin_amdgcn_wave_barrier();
+                    const R *v = (const R *)(wave_lds + (lane >> 2) * (16 * (int)sizeof(R) + 16)) + t;
+                    const R x0 = v[0], x1 = v[4], x2 = v[8], x3 = v[12];
+                    __builtin_amdgcn_wave_barrier();
+                    sum.add(x0); sum.add(x1); sum.add(x2); sum.add(x3);
                 }
             }
+            __syncthreads();  // the queue and the stored fluxes are written
+            const int nq = nqueue;
+            __syncthreads();  // before a wavefront goes on to queue the next segment's faces
+            if (nq) {
+                // the queued faces with the whole ladder
+                for (int e0 = 0; e0 < nq; e0 += 256) {
+                    const bool go = e0 + tid < nq;
+                    const int e = go ? queue[e0 + tid] : 0, er = e % kForceRowsPerBlock, q = e / kForceRowsPerBlock;
+                    const int ek = min(rb * kForceRowsPerBlock + er, a.nrows - 1);
+                    const int rr = a.sched ? a.sched[ek] : ek, ii = a.act[rr];
+                    const int j = go ? a.ell[ell_at(a.ld, rr, seg + q)] : 0;
+                    stage_records<R>(rec, j, go, wave_lds);
+                    if (!__any(go)) break;
+                    const Cell<R> I = rec[ii];
+                    wait_staged();
+                    if (go) {
+                        DevParams Q = P0;
+                        if (BOXES) {
+                            GridView g{};
+                            resolve_box(bt, ii, Q, g);
+                        }
+                        R dp0, dp1, dp2, f0, f1, f2, fp, vts;
+                        unsigned rung;
+                        double xi = 0, yi = 0, zi = 0, xj = 0, yj = 0, zj = 0;
+                        if constexpr (std::is_same<R, double>::value) {
+                            xi = F.X[ii]; yi = F.Y[ii]; zi = F.Z[ii];
+                            xj = F.X[j]; yj = F.Y[j]; zj = F.Z[j];
+                        }
+                        staged_dp<R>(Q, I, J, xi, yi, zi, xj, yj, zj, dp0, dp1, dp2);
+                        const int rc = force_pair<KERN, R, false>(Q, G, I, J, dp0, dp1, dp2, dp0 * dp0 + dp1 * dp1 + dp2 * dp2, f0, f1, f2, fp, vts, rung);
+                        if constexpr (STATS) count_rungs(F.rungs, rung);
+                        const bool add = rc == 1;
+                        R *w = flux[q][er];
+                        w[0] = add ? rounded(f0) : R(0); w[1] = add ? rounded(f1) : R(0);
+                        w[2] = add ? rounded(f2) : R(0); w[3] = add ? rounded(fp) : R(0);
+                        if (add && vts > 0) atomicMax(&mrow[er], (unsigned long long)__double_as_longlong((double)vts));
+                        pair_flags<BOXES>(a, bt, ii, j, rc, vts);
+                    }
+                }
+                __syncthreads();
+                if (tid == 0) nqueue = 0;
+                // the rows that waited: the rest of the segment in list order
+                if (first_rare >= 0) {
+                    had_rare = true;
+                    const R *f = &flux[0][tid >> 2][t];
+                    int q = first_rare;
+                    for (; q + 4 <= cs; q += 4) {
+                        const R x0 = f[(size_t)q * 4 * kForceRowsPerBlock], x1 = f[(size_t)(q + 1) * 4 * kForceRowsPerBlock],
+                                x2 = f[(size_t)(q + 2) * 4 * kForceRowsPerBlock], x3 = f[(size_t)(q + 3) * 4 * kForceRowsPerBlock];
+                        sum.add(x0); sum.add(x1); sum.add(x2); sum.add(x3);
+                    }
+                    for (; q < cs; q++) sum.add(f[(size_t)q * 4 * kForceRowsPerBlock]);
+                }
+                __syncthreads();  // the next segment's entries take the queue and the flux rows
+            }
         }
-        A0 = a0.value(); A1 = a1.value(); A2 = a2.value(); dE = ae.value(); msv = m;
+        // lane 0 of the quad closes the row: the quad's sums and its largest signal speed
+        const double v = sum.value();
+        const int l0 = lane & ~3;
+        const double A0 = __shfl(v, l0, 64), A1 = __shfl(v, l0 + 1, 64), A2 = __shfl(v, l0 + 2, 64), dE = __shfl(v, l0 + 3, 64);
+        m = dmax(m, __shfl_xor(m, 1, 64));
+        m = dmax(m, __shfl_xor(m, 2, 64));
+        if (row && t == 0) {
+            const double mq = __longlong_as_double((long long)mrow[tid >> 2]);
+            // effective_soundspeed of i, src/declarations/cell_data.h:703-712 (floor of MaxSignalVel)
+            const double sound_i = (rhoi > 0) ? sqrt(P.gamma * F.PR[i] / rhoi) : sqrt(P.gamma * (P.gamma - 1.) * F.U[i]);
+            force_tail(P, F, i, enabled, sound_i, A0, A1, A2, dE, dmax((double)m, mq), a.ACC, a.DTU, a.MSV);
+            rare_rows += had_rare;
+        }
     }
-    force_tail(P, F, i, enabled, sound_i, A0, A1, A2, dE, msv, a.ACC, a.DTU, a.MSV);
-    return true;
-}
-
-// one lane per row of k_force and k_force_w3 (the kernels differ in their launch bounds only)
-template <int KERN, typename R, bool BOXES, bool STATS, bool COMMON>
-__device__ __forceinline__ void force_lanes(const DevParams &P, const Gam<R> &G, const ForceView &F, const Cell<R> *__restrict__ rec,
-                                            const ForceRows &a, const BoxTable &bt)
-{
-    const int k = (int)(xcd_block() * blockDim.x + threadIdx.x);
-    const int r = k < a.nrows ? (a.sched ? a.sched[k] : k) : a.nrows;
-    // pairs of this launch when asked (wave sum, one atomic per wave; a launch of k_sum_counts
-    // after the pass costs fewer atomics on the one address)
-    if (a.pairs) {
-        unsigned long long c = (r < a.nrows) ? (unsigned long long)a.cnt[r] : 0ull;
-        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-        if ((threadIdx.x & 63) == 0 && c) atomicAdd(a.pairs, c);
+    // rows with a face past the common case (one atomic per wavefront of the fixed grid)
+    if (a.count_rare) {
+        for (int o = 32; o > 0; o >>= 1) rare_rows += __shfl_xor(rare_rows, o, 64);
+        if (lane == 0 && rare_rows) atomicAdd(a.err + 12, rare_rows);
     }
-    const bool done = (r >= a.nrows) || force_row<KERN, R, BOXES, STATS, COMMON>(P, G, F, rec, a, bt, r);
-    // rows left to the whole ladder: appended a wavefront at a time (one atomic per wavefront, the
-    // wavefront's rows kept together and in lane order)
-    const unsigned long long left = __ballot(!done);
-    if (!left) return;
-    const int lane = threadIdx.x & 63, lead = __ffsll((long long)left) - 1;
-    int base = 0;
-    if (lane == lead) base = atomicAdd(a.err + 12, __popcll(left));
-    base = __shfl(base, lead, 64);
-    if (!done) a.rare[base + __popcll(left & ((1ull << lane) - 1ull))] = r;
-}
-
-// the FP64 common pass of one box at two waves per SIMD (172 registers, no scratch; its LDS
-// record: 52 KB per workgroup); with the box table it takes 178 (two waves, no spill)
-template <int KERN, typename R, bool BOXES, bool STATS, bool COMMON>
-__global__ void __launch_bounds__(256, (COMMON && !BOXES && std::is_same<R, double>::value) ? 2 : 1) k_force(DevParams P, Gam<R> G, ForceView F, const Cell<R> *__restrict__ rec, ForceRows a,
-                                               BoxTable bt)
-{
-    force_lanes<KERN, R, BOXES, STATS, COMMON>(P, G, F, rec, a, bt);
-}
-
-// the FP64 common pass of one box at three waves per SIMD (166 registers).  Which is faster
-// depends on the field: on a 2M-row lattice pass the rows resident at three waves outgrow the
-// L2 with their neighbour records (7.3 ms against 6.7 at two); on the 4M lognormal field of
-// radii over many levels three waves hide more of the loads' latency (20.2 ms against 23.8)
-template <int KERN>
-__global__ void __launch_bounds__(256, 3) k_force_w3(DevParams P, Gam<double> G, ForceView F, const Cell<double> *__restrict__ rec,
-                                                     ForceRows a, BoxTable bt)
-{
-    force_lanes<KERN, double, false, false, true>(P, G, F, rec, a, bt);
-}
-
-// two waves per SIMD: the whole ladder then spills a few registers (FP64 ~300 wanted) but hides
-// more latency than one wave of the unspilled kernel (4M lognormal pass: FP64 93.4 -> 88.0 ms,
-// FP32 68.9 -> 64.5 ms)
-template <int KERN, typename R, bool BOXES>
-__global__ void __launch_bounds__(256, 2) k_force_rare(DevParams P, Gam<R> G, ForceView F, const Cell<R> *__restrict__ rec, ForceRows a,
-                                                    BoxTable bt)
-{
-    const int count = a.err[12];
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < count; k += gridDim.x * blockDim.x)
-        force_row<KERN, R, BOXES, false, false>(P, G, F, rec, a, bt, a.rare[k]);
 }
 
 // ---------------------------------------------------------------------------------------

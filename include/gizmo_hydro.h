@@ -127,8 +127,7 @@ int gz_synchronize(gz_context *ctx);
    "pairs_symmetric", "ngb_rebuilds", "n_active", "ell_widen"), and totals since the last
    gz_timing_reset ("active_updates": active particles through the hot path, "resorts",
    "force_pairs_total": neighbour pairs of every force launch, "force_rare_rows": rows of
-   lane-per-row force passes that a face past the Riemann ladder's common case sent to the
-   pass's second kernel).  With the option
+   force passes over many rows with a face past the Riemann ladder's common case).  With the option
    "riemann_stats" set to 1, the force passes of a single box also count, per face, the rungs of
    the Riemann ladder it took (each at most once per face) since the option was last set:
    "riemann_faces" (faces that reached the Riemann solve), "riemann_hllc", "riemann_vacuum",
@@ -231,13 +230,9 @@ int gz_drift_all(gz_context *ctx);
    (the force kernels, whose wake-up flags and pair counts a second run would not undo, wait on
    a device flag: the round converged every row and no radius outgrew the list's grid); one
    read of the counters after the force pass then settles the step, and when the flag says no,
-   the rounds go on and the three passes run again; "force_split" (default -1) -- the force pass
-   over more than few_rows rows runs in two kernels, the first evaluating every face through the
-   Riemann ladder's common case and leaving rows with a face that needs a later rung to the
-   second (1), in one kernel with the whole ladder (0), or (-1) in two unless it is the FP32 form
-   and more than a quarter of the rows took the second kernel in the last two-kernel pass;
-   "force_waves" (default 0; 2 or 3) -- the FP64 form's first force kernel of those two runs at
-   this many waves per SIMD (0: three with wide_search, else two).
+   the rounds go on and the three passes run again; "force_split" (default -1; 0 or 1) --
+   0: the force pass does not count the rows of "force_rare_rows" (the pass itself is the same);
+   "force_waves" (default 0; 2 or 3) -- accepted for callers of earlier versions, without effect.
    None of these changes a neighbour set or a
    sum, and none has a counterpart in the reference (tuning knobs of this library).
    One option selects physics, the reference's compile-time HYDRO_PARTITION_UNITY_IMPROVE_FD
