@@ -717,27 +717,28 @@ __device__ inline unsigned exact_riemann(const Gam<R> &G, const RState<R> &L, co
 // the sound speeds, enthalpies and normal velocities Riemann_solver derives from the face states
 // (src/hydro/reimann.h:313-339, no EOS_GENERAL)
 template <typename R> struct RPrep { R csL, csR, hL, hR, vL, vR; };
-template <typename R>
+// ROW: the right state's density and pressure are the row's own (exact_div)
+template <typename R, bool ROW = false>
 __device__ __forceinline__ RPrep<R> riemann_prep(const Gam<R> &G, const RState<R> &L, const RState<R> &Rs, const R *n)
 {
     RPrep<R> q;
     q.csL = sqrt(G.G0 * L.p / L.rho);
-    q.csR = sqrt(G.G0 * Rs.p / Rs.rho);
+    q.csR = ROW ? (R)sqrt((double)exact_div(G.G0 * Rs.p, Rs.rho)) : sqrt(G.G0 * Rs.p / Rs.rho);
     R uL = L.p / (G.G9 * L.rho);
-    R uR = Rs.p / (G.G9 * Rs.rho);
+    R uR = ROW ? exact_div(Rs.p, G.G9 * Rs.rho) : Rs.p / (G.G9 * Rs.rho);
     q.hL = L.p / L.rho + uL + R(0.5) * (L.v0 * L.v0 + L.v1 * L.v1 + L.v2 * L.v2);
-    q.hR = Rs.p / Rs.rho + uR + R(0.5) * (Rs.v0 * Rs.v0 + Rs.v1 * Rs.v1 + Rs.v2 * Rs.v2);
+    q.hR = (ROW ? exact_div(Rs.p, Rs.rho) : Rs.p / Rs.rho) + uR + R(0.5) * (Rs.v0 * Rs.v0 + Rs.v1 * Rs.v1 + Rs.v2 * Rs.v2);
     q.vL = L.v0 * n[0] + L.v1 * n[1] + L.v2 * n[2];
     q.vR = Rs.v0 * n[0] + Rs.v1 * n[1] + Rs.v2 * n[2];
     return q;
 }
 
 // Riemann_solver (:282-370) with HLLC_Riemann_solver (:382-396, MFM fluxes); returns the rungs taken
-template <typename R>
+template <typename R, bool ROW = false>
 __device__ inline unsigned riemann(const Gam<R> &G, const RState<R> &L, const RState<R> &Rs, const R *n, R ptl, ROut<R> &o)
 {
     if ((L.p < 0 && Rs.p < 0) || (L.rho < 0) || (Rs.rho < 0)) { o.P_M = 0; return kRungUnphysical; }
-    const RPrep<R> q = riemann_prep(G, L, Rs, n);
+    const RPrep<R> q = riemann_prep<R, ROW>(G, L, Rs, n);
     unsigned rung = wavespeeds(G, L, Rs, n, q.vL, q.vR, q.csL, q.csR, q.hL, q.hR, o, ptl);
     o.f0 = o.P_M * n[0];
     o.f1 = o.P_M * n[1];
@@ -835,16 +836,14 @@ __device__ inline bool riemann_ladder(const Gam<T> &G, RState<T> L, RState<T> Rs
     o.P_M = o.S_M = o.f0 = o.f1 = o.f2 = o.fp = 0;
     rung |= riemann(G, L, Rs, n, ptl, o);
     if ((o.P_M < 0) || (isnan(o.P_M)) || (o.P_M > T(1.4) * ptl)) {
-        // (rounded: the row's own state stays in this branch, where the FP32 form's divisions by it
-        // round alike in every kernel; moved out of a loop they would be exact)
-        Rs.p = rounded(pI); L.p = pJ; Rs.rho = rounded(rhoI); L.rho = rhoJ;
+        Rs.p = pI; L.p = pJ; Rs.rho = rhoI; L.rho = rhoJ;
         Rs.v0 = vi0; Rs.v1 = vi1; Rs.v2 = vi2;
         L.v0 = vj0; L.v1 = vj1; L.v2 = vj2;
-        rung |= kRungRetryFirstOrder | riemann(G, L, Rs, n, T(1.4) * ptl, o);
+        rung |= kRungRetryFirstOrder | riemann<T, true>(G, L, Rs, n, T(1.4) * ptl, o);
         if ((o.P_M < 0) || (isnan(o.P_M))) {
-            Rs.p = rounded(pI); L.p = pJ; Rs.rho = rounded(rhoI); L.rho = rhoJ;
+            Rs.p = pI; L.p = pJ; Rs.rho = rhoI; L.rho = rhoJ;
             Rs.v0 = Rs.v1 = Rs.v2 = 0; L.v0 = L.v1 = L.v2 = 0;
-            rung |= kRungRetryZeroVel | riemann(G, L, Rs, n, T(2.0) * ptl, o);
+            rung |= kRungRetryZeroVel | riemann<T, true>(G, L, Rs, n, T(2.0) * ptl, o);
             if ((o.P_M < 0) || (isnan(o.P_M))) { rung |= kRungFail; return false; }
         }
     }
