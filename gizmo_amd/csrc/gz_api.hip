@@ -98,6 +98,7 @@ struct gz_context {
     int wide = 0;
     WideGrid wide_h{};
     WideGrid *wide_dev = nullptr;
+    float4 *wboxes = nullptr;  // bounding boxes of 64 consecutive particles each
     int *wstart = nullptr, *wend = nullptr, *wlstart = nullptr, *wlend = nullptr, *lidx = nullptr, *plev = nullptr, *lcount = nullptr;
     long long wcells_alloc = 0;
     long wide_key_version = -1;
@@ -420,6 +421,7 @@ void free_state(gz_context *c)
     dfree(c->TB); dfree(c->WAKE); dfree(c->ACT); dfree(c->perm); dfree(c->key); dfree(c->key2);
     dfree(c->wstart); dfree(c->wend); dfree(c->wlstart); dfree(c->wlend); dfree(c->lidx); dfree(c->plev); dfree(c->lcount);
     dfree(c->wide_dev);
+    dfree(c->wboxes);
     {
         dfree(c->act_bits); dfree(c->act_bcount);
         dfree(c->sched); dfree(c->sched_part); dfree(c->flux); c->flux_bytes = 0; dfree(c->rl_a); dfree(c->rl_b);
@@ -706,13 +708,16 @@ int build_wide(gz_context *ctx, bool lists)
     }
     if (!ctx->lidx) {
         CHK(dalloc(ctx, &ctx->lidx, ctx->cap)); CHK(dalloc(ctx, &ctx->plev, ctx->cap)); CHK(dalloc(ctx, &ctx->lcount, kFineLevel + 2));
-        CHK(dalloc(ctx, &ctx->wide_dev, 1));
+        CHK(dalloc(ctx, &ctx->wide_dev, 1)); CHK(dalloc(ctx, &ctx->wboxes, 2 * ((ctx->cap + 63) / 64)));
     }
     W.key = ctx->key;
     W.n = (int)n;
     W.lmax = lmax;
     W.start = ctx->wstart; W.end = ctx->wend; W.lidx = ctx->lidx; W.lstart = ctx->wlstart; W.lend = ctx->wlend;
+    W.boxes = ctx->wboxes;
     Timed t(ctx, "ngb_build");
+    k_block_boxes<<<nblk(n), kBlock, 0, ctx->stream>>>((int)n, ctx->X, ctx->Y, ctx->Z, ctx->H, ctx->wboxes);
+    HIPCHK(hipGetLastError());
     if (ctx->wide_key_version != ctx->key_version || lmax > ctx->wide_lmax) {
         k_wide_bounds<<<nblk(n), kBlock, 0, ctx->stream>>>(W);
         HIPCHK(hipGetLastError());
@@ -1076,7 +1081,7 @@ int ensure_sym(gz_context *ctx)
         {
             Timed t(ctx, "ngb_build");
             if (wide && !few)
-                k_build_sym_cells<<<xcd_grid(ctx->grp.ngroups), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
+                k_build_sym_groups<<<xcd_grid(ctx->grp.ngroups), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
                                                                                        ctx->X, ctx->Y, ctx->Z, ctx->H, ctx->ell_s, ctx->ld_s,
                                                                                        ctx->cap_s, ctx->cnt_s, ctx->counters + 3);
             else if (wide)
@@ -1088,7 +1093,7 @@ int ensure_sym(gz_context *ctx)
                                                                                ctx->Z, ctx->H, ctx->ell_s, ctx->ld_s, ctx->cap_s, ctx->cnt_s,
                                                                                ctx->counters + 3, BoxTable{});
             else
-                k_build_sym_cells<<<xcd_grid(ctx->ncells), 64, 0, ctx->stream>>>(grid_view(ctx), cell_rows(ctx), ctx->act, ctx->X, ctx->Y,
+                sym_kernel(ctx->nact, ctx->ncells)<<<xcd_grid(ctx->ncells), 64, 0, ctx->stream>>>(grid_view(ctx), cell_rows(ctx), ctx->act, ctx->X, ctx->Y,
                                                                                   ctx->Z, ctx->H, ctx->ell_s, ctx->ld_s, ctx->cap_s,
                                                                                   ctx->cnt_s, ctx->counters + 3);
             HIPCHK(hipGetLastError());
@@ -2204,7 +2209,7 @@ long gz_neighbors(gz_context *ctx, int symmetric, long *offsets, int *nbr, long 
             ctx->overflow_clear = false;
             if (hipMemsetAsync(ctx->counters + 3, 0, sizeof(int), ctx->stream) != hipSuccess) { rc = GZ_E_HIP; break; }
             if (ctx->nact > ctx->few_rows)
-                k_build_sym_cells<<<xcd_grid(ctx->grp.ngroups), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
+                k_build_sym_groups<<<xcd_grid(ctx->grp.ngroups), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
                                                                                        ctx->X, ctx->Y, ctx->Z, ctx->H, ell, ld, capl, cnt,
                                                                                        ctx->counters + 3);
             else

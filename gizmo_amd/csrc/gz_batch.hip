@@ -574,7 +574,7 @@ int sym_list(gz_batch *b, const std::vector<uint8_t> &in_pass)
         BHIP(hipMemsetAsync(b->counters + 3, 0, sizeof(int), b->stream));
         if (na > b->few_rows) {
             BCHK(build_groups(b));
-            k_build_sym_cells<<<xcd_grid(b->grp.ngroups), 64, 0, b->stream>>>(gview(b), b->grp.view(bt), b->act, b->X, b->Y, b->Z, b->H,
+            sym_kernel(na, b->grp.ngroups)<<<xcd_grid(b->grp.ngroups), 64, 0, b->stream>>>(gview(b), b->grp.view(bt), b->act, b->X, b->Y, b->Z, b->H,
                                                                                b->ell, ld, b->ell_cap, b->cnt, b->counters + 3);
         } else {
             k_build_sym_rows<<<xcd_grid(na), kRowThreads, 0, b->stream>>>(gview(b), na, b->act, b->key, b->X, b->Y, b->Z, b->H, b->ell, ld,

@@ -17,6 +17,13 @@ __device__ __forceinline__ long xcd_block()
     const long b = blockIdx.x, q = gridDim.x / kXcds;
     return (b % kXcds) * q + b / kXcds;
 }
+// The same in runs of 64 workgroups, dealt to the XCDs in turn: for work whose cost drifts along the
+// logical order (an XCD's contiguous eighth could take several times another's)
+__device__ __forceinline__ long xcd_block_dealt()
+{
+    const long b = blockIdx.x, l = b / kXcds, q = gridDim.x / kXcds, whole = q / 64 * 64;
+    return l < whole ? (l / 64 * kXcds + b % kXcds) * 64 + l % 64 : whole * kXcds + (b % kXcds) * (q - whole) + (l - whole);
+}
 inline unsigned xcd_grid(long nblocks) { return (unsigned)(((nblocks + kXcds - 1) / kXcds) * kXcds); }
 
 // Search over kernel radii that span many grid levels.  Every cell of every level 0..lmax is a
@@ -35,6 +42,7 @@ struct WideGrid {
     int *lstart, *lend;
     long long loff[kFineLevel + 1];
     int lofs[kFineLevel + 2];
+    const float4 *boxes;       // per 64 particles of the order: lowest corner and largest radius, highest corner
 };
 
 struct GridView {
@@ -283,6 +291,14 @@ __global__ void k_cell_rows_list(int nact, const int *act, const uint32_t *key, 
                                  int *cells);
 __global__ void k_build_sym_cells(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
                                   const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
+__global__ void k_block_boxes(int n, const double *X, const double *Y, const double *Z, const double *H, float4 *boxes);
+__global__ void k_build_sym_groups(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
+                                   const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
+// cells of at most this many rows on average: one candidate per lane (k_build_sym_groups), whose
+// time grows with the rows of a cell (4 of 31: 218 us against 524 with a row per lane) where the
+// other's does not
+constexpr int kSymFewRows = 16;
+inline auto sym_kernel(long nrows, long ncells) { return nrows <= kSymFewRows * ncells ? k_build_sym_groups : k_build_sym_cells; }
 
 // FD: with the sums of the first-derivative volume correction
 template <int KERN, typename R, bool FD>

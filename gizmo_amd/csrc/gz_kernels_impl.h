@@ -438,6 +438,11 @@ __device__ __forceinline__ double wave_min(double v)
     for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
     return v;
 }
+__device__ __forceinline__ float wave_minf(float v)
+{
+    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+    return v;
+}
 __device__ __forceinline__ double wave_max(double v)
 {
     for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
@@ -466,6 +471,14 @@ __device__ __forceinline__ bool leaf_reach(const GridView &g, const LeafBox &b, 
     const double ez = fmax(fmax(b.lo[2] - rz, rz - b.hi[2]), 0.0);
     const double rr = reach * (1.0 + 1e-9) + 1e-12 * g.box;
     return ex * ex + ey * ey + ez * ez <= rr * rr;
+}
+
+// a lane's value in every lane (a: the same lane for all)
+__device__ __forceinline__ int lane_value(int v, int a) { return __builtin_amdgcn_readlane(v, a); }
+__device__ __forceinline__ float lane_value(float v, int a) { return __int_as_float(lane_value(__float_as_int(v), a)); }
+__device__ __forceinline__ double lane_value(double v, int a)
+{
+    return __hiloint2double(lane_value(__double2hiint(v), a), lane_value(__double2loint(v), a));
 }
 
 // position of this lane among the kept lanes below it (stable compaction)

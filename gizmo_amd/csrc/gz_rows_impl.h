@@ -170,6 +170,67 @@ __device__ __forceinline__ void row_stencil_wide(const GridView &g, const WideGr
     stencil_finish(rs, code, st, en);
 }
 
+// ---------------------------------------------------------------------------------------
+// Long walks over many levels.  The cells of a coarse level next to a clump hold up to a tenth of all
+// particles (1M lognormal particles: 100K candidates for the rows of one cell), and one
+// wavefront walks them.  The bounding box and the largest radius of every 64 consecutive particles
+// let a lane drop 64 candidates at once.  Density rounds of 1M lognormal rows FP64 2.5 -> 1.9 ms,
+// of 4M rows FP32 5.7 -> 4.3 ms.
+// ---------------------------------------------------------------------------------------
+#ifdef GZ_DEFINE_COMMON_KERNELS
+__global__ void __launch_bounds__(256) k_block_boxes(int n, const double *__restrict__ X, const double *__restrict__ Y,
+                                                     const double *__restrict__ Z, const double *__restrict__ H, float4 *__restrict__ boxes)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool on = j < n;
+    // rounded outwards by the caller's slack (2^-23 of the box)
+    const float x = on ? (float)X[j] : 0.0f, y = on ? (float)Y[j] : 0.0f, z = on ? (float)Z[j] : 0.0f, h = on ? (float)H[j] : 0.0f;
+    const float lx = wave_minf(on ? x : 1e30f), ly = wave_minf(on ? y : 1e30f), lz = wave_minf(on ? z : 1e30f);
+    const float mx = -wave_minf(on ? -x : 1e30f), my = -wave_minf(on ? -y : 1e30f), mz = -wave_minf(on ? -z : 1e30f), hm = -wave_minf(-h);
+    if (on && (j & 63) == 0) {
+        boxes[2 * (j >> 6)] = make_float4(lx, ly, lz, hm);
+        boxes[2 * (j >> 6) + 1] = make_float4(mx, my, mz, 0.0f);
+    }
+}
+#endif
+
+// what a block's particles are tested against: the rows' bounding box (centre, half extents) and radius
+struct BlockReach {
+    float cx, cy, cz, ex, ey, ez, h, box;
+    // whether a pair of a row and a particle of block b may lie within the larger radius (SYM) or the
+    // row's; the slack covers the FP32 rounding of the positions and the boxes
+    template <bool SYM> __device__ __forceinline__ bool hits(const float4 *__restrict__ boxes, int b) const
+    {
+        const float4 lo = boxes[2 * b], hi = boxes[2 * b + 1];
+        const float half = 0.5f * box;
+        auto gap = [&](float c, float e, float l, float m) {
+            float d = fabsf(c - 0.5f * (l + m));
+            d = d > half ? box - d : d;
+            return fmaxf(d - e - 0.5f * (m - l) - 2e-6f * box, 0.0f);
+        };
+        const float gx = gap(cx, ex, lo.x, hi.x), gy = gap(cy, ey, lo.y, hi.y), gz = gap(cz, ez, lo.z, hi.z);
+        const float r = (SYM ? fmaxf(h, lo.w) : h) * (1.0f + 1e-5f);
+        return gx * gx + gy * gy + gz * gz <= r * r;
+    }
+};
+
+// Of 64 runs of RUN candidates from v0 on (at(v): candidate v's particle, negative: not from the
+// order), the ones that may hold a partner, as a bit per run.  A run whose particles are
+// consecutive covers few blocks; any other run is kept.
+template <bool SYM, int RUN, typename At>
+__device__ __forceinline__ unsigned long long live_runs(const BlockReach &reach, const float4 *__restrict__ boxes, int v0, int total, At at)
+{
+    const int a = v0 + RUN * (int)(threadIdx.x & 63);
+    bool live = false;
+    if (a < total) {
+        const int last = min(a + RUN, total) - 1, j0 = at(a), j1 = at(last);
+        live = j0 < 0 || j1 - j0 != last - a;
+        for (int b = j0 >> 6; !live && b <= j1 >> 6; b++) live = reach.hits<SYM>(boxes, b);
+    }
+    return __ballot(live);
+}
+constexpr int kLongWalk = 1024;  // candidates from which a walk asks for its live runs first
+
 // The place of this thread's entry among the flagged entries of its workgroup, in thread order
 // (total: the flagged entries of the workgroup).  One barrier: smask[TPB / 64] must not be read
 // by another round of the caller before the caller's next barrier.
@@ -264,7 +325,16 @@ __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, i
     const int nsum = fd ? kDensSumsFD : kDensSums;
     R acc = 0;  // thread q < nsum keeps sum q
     int accepted = 0;  // thread 17: the row's pairs (the pass's work, counted when npairs is given)
-    for (int base = 0; base < total; base += TPB) {
+    const bool long_walk = g.wide && total > kLongWalk;
+    const BlockReach reach{(float)xi, (float)yi, (float)zi, 0.0f, 0.0f, 0.0f, (float)h, (float)g.box};
+    unsigned long long live = ~0ull;
+    for (int base = 0, run = 0; base < total; base += TPB, run++) {
+        if (long_walk) {
+            // (every wavefront of the workgroup finds the same bits)
+            if ((run & 63) == 0)
+                live = live_runs<false, TPB>(reach, g.wide->boxes, base, total, [&](int v) { return row_candidate(rs, v); });
+            if (!((live >> (run & 63)) & 1ull)) continue;
+        }
         const int v = base + tid;
         bool ok = false;
         R t[kDensSumsFD];
@@ -536,21 +606,215 @@ __global__ void __launch_bounds__(64) k_build_sym_wide(GridView g, int nrows, co
 #endif
 
 // ---------------------------------------------------------------------------------------
-// symmetric list as a cell walk (one wavefront per occupied cell, culled LDS-staged candidates):
-// rows r2 < max(h_i,h_j)^2, self excluded, ascending (src/mesh/sfc_tiles_functions.h:83-102);
-// with row groups (CellRows.gsten) a group is one cell of one grid level or of one box
+// symmetric list as a cell walk (one wavefront per occupied cell): rows r2 < max(h_i,h_j)^2, self
+// excluded, ascending (src/mesh/sfc_tiles_functions.h:83-102); with row groups (CellRows.gsten) a
+// group is one cell of one grid level or of one box.  Two kernels with the same lists:
+// k_build_sym_cells, a row per lane, where the cells hold rows enough to fill a wavefront, and
+// k_build_sym_groups, a candidate per lane, where they do not (kSymFewRows) and for the search
+// over many levels.
+// Before, one kernel with the exact FP64 test behind every staged candidate and a lane per row
+// for both.  2M rows, 64 to a cell: 1.47 -> 1.00 ms (of cells, a row per lane); 128K rows, 4 to a
+// cell: 700 -> 218 us; search over many levels (a dozen rows to a cell) 1M rows 6.3 -> 5.0 ms, 4M
+// rows 23.1 -> 9.1 ms.  Candidates laid end to end (as the groups' ranges are) made the walk of
+// full cells slower (1.00 -> 1.25 ms: the search for a lane's range).
 // ---------------------------------------------------------------------------------------
 #ifdef GZ_DEFINE_COMMON_KERNELS
+// Candidates are culled against the rows' bounding box and staged 64 at a time; each lane masks the
+// tile with the FP32 test of the candidate window (k_density_cells), against the larger of the two
+// radii, and takes its own candidates through the exact test.
 __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr, const int *__restrict__ act,
                                                         const double *__restrict__ X, const double *__restrict__ Y,
                                                         const double *__restrict__ Z, const double *__restrict__ H,
                                                         int *__restrict__ ell, long ld, int cap, int *__restrict__ cnt,
                                                         int *__restrict__ overflow)
 {
-    __shared__ double sx[64], sy[64], sz[64], sh[64];
-    __shared__ int sj[64];
-    __shared__ RowStencil rs;
+    __shared__ double sx[kWinRing], sy[kWinRing], sz[kWinRing], sh[kWinRing];
+    __shared__ int sj[kWinRing];
+    __shared__ float4 st[64];
+    __shared__ float sth[64];
     const long cb = xcd_block();
+    if (cb >= (cr.ncells_dev ? *cr.ncells_dev : cr.ncells)) return;
+    int c, a0, a1, nst;
+    const int4 *sten;
+    if (cr.gsten) {
+        c = cr.gcode[cb]; a0 = cr.gstart[cb]; a1 = cr.gstart[cb + 1]; nst = cr.gnst[cb]; sten = cr.gsten + (size_t)27 * cb;
+        DevParams P{};
+        resolve_box(cr.bt, act[cr.grow ? cr.grow[a0] : a0], P, g);
+    } else {
+        c = cr.cells[cb]; a0 = cr.ca0[c]; a1 = cr.ca1[c]; nst = g.nsten[c]; sten = g.sten + (size_t)c * 27;
+    }
+    const int t = threadIdx.x;
+    for (int base = a0; base < a1; base += 64) {
+        const bool on = base + t < a1;
+        const int r = on ? (cr.grow ? cr.grow[base + t] : base + t) : 0;
+        int i = -1;
+        double xi = 0, yi = 0, zi = 0, hi = 0;
+        if (on) { i = act[r]; xi = X[i]; yi = Y[i]; zi = Z[i]; hi = H[i]; }
+        const LeafBox lb = leaf_box(g, c, on, xi, yi, zi);
+        const double hleaf = wave_max(on ? hi : 0.0);
+        const bool small = (1 << g.level) >= 8;
+        const double inv_cell = 1.0 / g.cell;
+        float qx, qy, qz, qh, lim;
+        {
+            const float ux = (float)(wrap(xi - lb.ox, g.box, g.half) * inv_cell - 0.5), uy = (float)(wrap(yi - lb.oy, g.box, g.half) * inv_cell - 0.5),
+                        uz = (float)(wrap(zi - lb.oz, g.box, g.half) * inv_cell - 0.5), uh = (float)(hi * inv_cell);
+            qx = -2.0f * ux; qy = -2.0f * uy; qz = -2.0f * uz;
+            qh = uh * uh;
+            lim = on ? kWinSlack - (ux * ux + uy * uy + uz * uz) : -1e30f;
+        }
+        Window win;
+        int head = 0, fill = 0, n = 0;
+        int q = 0, ts = nst > 0 ? sten[0].x : 0, te = nst > 0 ? sten[0].y : 0;  // the next candidates
+        bool more = nst > 0, left = false, keep = false;
+        int pos = 0, j = 0;
+        double xj = 0, yj = 0, zj = 0, hj = 0;
+        auto stage = [&](int k) {
+            const int s = head + k;
+            sx[s] = xj; sy[s] = yj; sz[s] = zj; sh[s] = hj; sj[s] = j;
+            const float fx = (float)(wrap(xj - lb.ox, g.box, g.half) * inv_cell - 0.5), fy = (float)(wrap(yj - lb.oy, g.box, g.half) * inv_cell - 0.5),
+                        fz = (float)(wrap(zj - lb.oz, g.box, g.half) * inv_cell - 0.5), fh = (float)(hj * inv_cell);
+            st[k] = make_float4(fx, fy, fz, fx * fx + fy * fy + fz * fz);
+            sth[k] = fh * fh;
+        };
+        while (more || left) {
+            __syncthreads();  // the lanes are done with the tile before the last and its test values
+            if (keep) stage(pos);  // what the last tile had no room for
+            keep = false;
+            left = false;
+            while (more && fill < 64) {
+                j = ts + t;
+                if (j < te) {
+                    xj = X[j]; yj = Y[j]; zj = Z[j]; hj = H[j];
+                    keep = leaf_reach(g, lb, xj, yj, zj, fmax(hleaf, hj));
+                }
+                int nt;
+                pos = fill + kept_rank(keep, nt);
+                if (keep && pos < 64) {
+                    stage(pos);
+                    keep = false;
+                }
+                fill += nt;
+                ts += 64;
+                if (ts >= te) {
+                    q++;
+                    more = q < nst;
+                    if (more) { ts = sten[q].x; te = sten[q].y; }
+                }
+            }
+            const int nt = fill < 64 ? fill : 64;
+            fill -= nt;
+            left = fill > 0;
+            pos -= 64;
+            if (t >= nt) { st[t] = make_float4(0.0f, 0.0f, 0.0f, 1e30f); sth[t] = 0.0f; }  // no candidate
+            __syncthreads();
+            uint32_t mlo = 0, mhi = 0;
+            if (small) {
+#pragma unroll 4
+                for (int k = 31; k >= 0; k--) {
+                    const float4 u = st[k], v = st[k + 32];
+                    mask_push(mlo, __builtin_fmaf(qx, u.x, __builtin_fmaf(qy, u.y, __builtin_fmaf(qz, u.z, u.w))) - fmaxf(qh, sth[k]), lim);
+                    mask_push(mhi, __builtin_fmaf(qx, v.x, __builtin_fmaf(qy, v.y, __builtin_fmaf(qz, v.z, v.w))) - fmaxf(qh, sth[k + 32]), lim);
+                }
+            } else {
+                // coarse grids: every candidate takes the exact test
+                const unsigned long long all = on ? (nt == 64 ? ~0ull : (1ull << nt) - 1ull) : 0ull;
+                mlo = (uint32_t)all;
+                mhi = (uint32_t)(all >> 32);
+            }
+            win.push(((unsigned long long)mhi << 32) | mlo);
+            head = head == kWinRing - 64 ? 0 : head + 64;
+            const int room = more || left ? kWinWords - 2 : -1;
+            do {
+                if (win.ready()) {
+                    const int k = win.next();
+                    const int jj = sj[k];
+                    if (jj != i && accept_pair<true>(xi, yi, zi, sx[k], sy[k], sz[k], hi, sh[k], g.box, g.half)) {
+                        if (n < cap) ell[ell_at(ld, r, n)] = jj;
+                        n++;
+                    }
+                }
+            } while (wave_any(win.behind > room));
+        }
+        __syncthreads();  // before the next rows' candidates take the ring
+        if (on) {
+            cnt[r] = min(n, cap);  // readers stay inside the list; the overflow carries the full length
+            if (n > cap) atomicMax(overflow, n);
+        }
+    }
+}
+
+// The candidates of a cell walk: up to kMaxRanges index ranges in ascending order, laid end to end, so
+// that 64 candidates are taken at a time whatever the ranges' lengths (cells of a dozen particles
+// would leave most lanes of a range-by-range walk idle).  Candidate v is start[k] + v - pref[k]
+// of the last range k with pref[k] <= v.
+constexpr int kMaxRanges = 56;
+struct CellRanges {
+    int start[kMaxRanges];
+    int pref[kMaxRanges];
+    int n, total;
+    __device__ __forceinline__ int at(int v) const
+    {
+        int lo = 0, hi = n - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (pref[mid] <= v) lo = mid;
+            else hi = mid - 1;
+        }
+        return start[lo] + (v - pref[lo]);
+    }
+};
+
+// the ranges of a stencil (one wavefront; nst <= 27 entries, one lane each)
+__device__ __forceinline__ void stencil_ranges(CellRanges &cr, const int4 *__restrict__ sten, int nst)
+{
+    const int lane = threadIdx.x & 63;
+    const int4 e = lane < nst ? sten[lane] : make_int4(0, 0, 0, 0);
+    const int len = e.y - e.x;
+    int sum = len;
+    for (int o = 1; o < 32; o <<= 1) {
+        const int up = __shfl_up(sum, o, 64);
+        if (lane >= o) sum += up;
+    }
+    if (lane < nst) {
+        cr.start[lane] = e.x;
+        cr.pref[lane] = sum - len;
+    }
+    if (lane == 31) {
+        cr.n = nst;
+        cr.total = sum;
+    }
+    __syncthreads();
+}
+
+// One candidate per lane and the rows of the group in turn: no lane is idle however few rows a cell
+// holds (a dozen in the search over many levels, whose cells are sized by the rows' own radii),
+// and a ballot gives each accepted candidate its place.  The test is FP32 in units of the cell
+// side (|x_i|^2 + |x_j|^2 - 2 x_i.x_j against the larger radius squared) with a bound on its
+// rounding error; only a pair within that bound of the radius takes the exact test.
+//
+// The search over many levels adds the particles of each coarser level L in the 27 cells of
+// level L around the group's cell that lie outside the 27 cells of the group's level (part B, as
+// k_build_sym_wide).  They are collected first, sorted, and laid between the group's own ranges,
+// so that the walk meets every candidate in ascending order; more than kMaxCoarse of them are
+// inserted into the finished rows one by one.
+constexpr int kMaxCoarse = 768;
+// bound on the FP32 test's rounding error, per unit of |x_j|^2 + h_j^2 + 13 (|x_i|^2 <= 12 in cells):
+// a dozen roundings of 2^-24 each of at most twice that
+constexpr float kSymSlack = 2e-6f;
+constexpr int kCoarseRange = 1 << 30;
+__global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr, const int *__restrict__ act,
+                                                         const double *__restrict__ X, const double *__restrict__ Y,
+                                                         const double *__restrict__ Z, const double *__restrict__ H,
+                                                         int *__restrict__ ell, long ld, int cap, int *__restrict__ cnt,
+                                                         int *__restrict__ overflow)
+{
+    __shared__ RowStencil rs;
+    __shared__ CellRanges cells;
+    __shared__ int coarse[kMaxCoarse], sorted[kMaxCoarse], runs[kFineLevel + 2];
+    __shared__ float4 st[64];  // a tile of candidates: position in cells, radius squared
+    __shared__ int sj[64];
+    // (the groups of the search over many levels come level by level, at very different costs)
+    const long cb = xcd_block_dealt();
     if (cb >= (cr.ncells_dev ? *cr.ncells_dev : cr.ncells)) return;
     int c, a0, a1, nst;
     const int4 *sten;
@@ -569,78 +833,210 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
     // the search over many levels adds part B (its groups are cells of the rows' own levels)
     const bool wide = cr.gsten && !cr.bt.b && g.wide;
     const int t = threadIdx.x;
+    const int nci = 1 << g.level;
+    const int hx = compact10((uint32_t)c >> 2), hy = compact10((uint32_t)c >> 1), hz = compact10((uint32_t)c);
+    const int si = 3 * (kFineLevel - g.level);
+    // the FP32 test: grids of at least 8 cells a side (a partner then lies within half a box of the
+    // cell's origin); 16 over many levels, whose coarse partners lie up to box / 2.6 from the row
+    const bool small = nci >= (wide ? 16 : 8);
+    const double inv_cell = 1.0 / g.cell, inv_box = 1.0 / g.box;
+    // a coordinate relative to the centre of the group's cell (index h along its axis), in cells
+    auto rel = [&](double x, int h) { return (float)(wrap_near(x - h * g.cell, g.box, inv_box) * inv_cell - 0.5); };
+    // a particle of a coarser level that the group's own cells do not hold
+    auto outside = [&](int j) {
+        const uint32_t cj = g.wide->key[j] >> si;
+        return !(periodic_adjacent((int)compact10(cj >> 2), hx, nci) && periodic_adjacent((int)compact10(cj >> 1), hy, nci) &&
+                 periodic_adjacent((int)compact10(cj), hz, nci));
+    };
+    if (!wide) stencil_ranges(cells, sten, nst);
     for (int base = a0; base < a1; base += 64) {
         const bool on = base + t < a1;
         const int r = on ? (cr.grow ? cr.grow[base + t] : base + t) : 0;
         int i = -1;
         double xi = 0, yi = 0, zi = 0, hi = 0;
         if (on) { i = act[r]; xi = X[i]; yi = Y[i]; zi = Z[i]; hi = H[i]; }
-        const LeafBox lb = leaf_box(g, c, on, xi, yi, zi);
-        const double hleaf = wave_max(on ? hi : 0.0);
-        int n = 0;
-        for (int q = 0; q < nst; q++) {
-            const int4 e = sten[q];
-            for (int ts = e.x; ts < e.y; ts += 64) {
-                const int j = ts + t;
-                bool keep = false;
-                double xj = 0, yj = 0, zj = 0, hj = 0;
-                if (j < e.y) {
-                    xj = X[j]; yj = Y[j]; zj = Z[j]; hj = H[j];
-                    keep = leaf_reach(g, lb, xj, yj, zj, fmax(hleaf, hj));
-                }
-                int nt;
-                const int pos = kept_rank(keep, nt);
-                __syncthreads();
-                if (keep) { sx[pos] = xj; sy[pos] = yj; sz[pos] = zj; sh[pos] = hj; sj[pos] = j; }
-                __syncthreads();
-                if (!on) continue;
-                for (int k = 0; k < nt; k++) {
-                    const int jj = sj[k];
-                    if (jj == i) continue;
-                    if (accept_pair<true>(xi, yi, zi, sx[k], sy[k], sz[k], hi, sh[k], g.box, g.half)) {
-                        if (n < cap) ell[ell_at(ld, r, n)] = jj;
-                        n++;
+        // the rows in units of the cell side around the cell's centre, and their bounding box
+        const float ux = rel(xi, hx), uy = rel(yi, hy), uz = rel(zi, hz), uh = (float)(hi * inv_cell);
+        const float qx = -2.0f * ux, qy = -2.0f * uy, qz = -2.0f * uz, qn = ux * ux + uy * uy + uz * uz, qh = uh * uh;
+        const float lx = wave_minf(on ? ux : 1e30f), ly = wave_minf(on ? uy : 1e30f), lz = wave_minf(on ? uz : 1e30f);
+        const float mx = -wave_minf(on ? -ux : 1e30f), my = -wave_minf(on ? -uy : 1e30f), mz = -wave_minf(on ? -uz : 1e30f);
+        const float hleaf = -wave_minf(on ? -uh : 0.0f);
+        // a candidate that no row can reach (conservative: the slack covers the rounding)
+        auto culled = [&](float fx, float fy, float fz, float fh) {
+            const float ex = fmaxf(fmaxf(lx - fx, fx - mx), 0.0f), ey = fmaxf(fmaxf(ly - fy, fy - my), 0.0f),
+                        ez = fmaxf(fmaxf(lz - fz, fz - mz), 0.0f), hm = fmaxf(fh, hleaf);
+            return small && ex * ex + ey * ey + ez * ez > hm * hm + kSymSlack * (fx * fx + fy * fy + fz * fz + hm * hm + 12.0f);
+        };
+        int ncoarse = 0;  // part B's particles (above kMaxCoarse: not collected)
+        if (wide) {
+            const WideGrid &W = *g.wide;
+            for (int L = 0; L < g.level && ncoarse <= kMaxCoarse; L++) {
+                if (t == 0) runs[L] = ncoarse;
+                if (W.lofs[L + 1] == W.lofs[L]) continue;  // no particle of this level
+                __syncthreads();  // every lane is done with rs before it is built again
+                row_stencil_wide<true>(g, W, L, (uint32_t)c >> (3 * (g.level - L)), 0.0, 0.0, 0.0, -1.0, rs);
+                const int total = rs.pref[rs.nst];
+                for (int v0 = 0; v0 < total; v0 += 64) {
+                    bool keep = false;
+                    int j = 0;
+                    if (v0 + t < total) {
+                        j = W.lidx[row_candidate(rs, v0 + t)];
+                        keep = outside(j) && !culled(rel(X[j], hx), rel(Y[j], hy), rel(Z[j], hz), (float)(H[j] * inv_cell));
                     }
+                    int nt;
+                    const int pos = ncoarse + kept_rank(keep, nt);
+                    if (keep && pos < kMaxCoarse) coarse[pos] = j;
+                    ncoarse += nt;
                 }
             }
+            __syncthreads();
+            const int nb = ncoarse <= kMaxCoarse ? ncoarse : 0;
+            if (t == 0 && nb) runs[g.level] = nb;
+            __syncthreads();
+            // merged: each level's particles ascend, so a particle's place is the sum of its places
+            // among every level's
+            for (int k = t; k < nb; k += 64) {
+                const int e = coarse[k];
+                int rank = 0;
+                for (int L = 0; L < g.level; L++) {
+                    const int first = runs[L];
+                    int lo = first, hi2 = runs[L + 1];
+                    while (lo < hi2) {
+                        const int mid = (lo + hi2) >> 1;
+                        if (coarse[mid] < e) lo = mid + 1;
+                        else hi2 = mid;
+                    }
+                    rank += lo - first;
+                }
+                sorted[rank] = e;
+            }
+            __syncthreads();
+            // ranges 2 q + 1: the stencil's cells, 2 q: the coarse particles before them (as their
+            // places in `sorted`, less kCoarseRange), 2 nst: those after the last
+            const int4 e = t < nst ? sten[t] : make_int4(0x7fffffff, 0x7fffffff, 0, 0);
+            int before = 0, above = nb;  // coarse particles below e.x
+            while (before < above) {
+                const int mid = (before + above) >> 1;
+                if (sorted[mid] < e.x) before = mid + 1;
+                else above = mid;
+            }
+            const int prev = __shfl_up(before, 1, 64), bcount = before - (t ? prev : 0), len = e.y - e.x;
+            const int mine = t <= nst ? bcount + len : 0;
+            int sum = mine;
+            for (int o = 1; o < 32; o <<= 1) {
+                const int up = __shfl_up(sum, o, 64);
+                if (t >= o) sum += up;
+            }
+            if (t <= nst) {
+                cells.start[2 * t] = before - bcount - kCoarseRange;
+                cells.pref[2 * t] = sum - mine;
+                if (t < nst) {
+                    cells.start[2 * t + 1] = e.x;
+                    cells.pref[2 * t + 1] = sum - mine + bcount;
+                }
+            }
+            if (t == nst) {
+                cells.n = 2 * nst + 1;
+                cells.total = sum;
+            }
+            __syncthreads();
         }
-        if (wide) {
-            // Part B of the search over many levels (as k_build_sym_wide): the particles of each
-            // coarser level L in the 27 cells of level L around the group's cell that lie outside
-            // the 27 cells of the group's level, each accepted one inserted in ascending place
-            const int nci = 1 << g.level;
-            const int hx = compact10((uint32_t)c >> 2), hy = compact10((uint32_t)c >> 1), hz = compact10((uint32_t)c);
-            const int si = 3 * (kFineLevel - g.level);
+        const int rows = min(a1 - base, 64);
+        int n = 0, fill = 0, v0 = 0, pos = 0, j = 0;
+        bool more = cells.total > 0, left = false, keep = false;
+        const bool long_walk = wide && small && cells.total > kLongWalk;
+        const float side = (float)g.cell;
+        const BlockReach reach{(float)(hx * g.cell) + (0.5f * (lx + mx) + 0.5f) * side, (float)(hy * g.cell) + (0.5f * (ly + my) + 0.5f) * side,
+                               (float)(hz * g.cell) + (0.5f * (lz + mz) + 0.5f) * side, 0.5f * (mx - lx) * side, 0.5f * (my - ly) * side,
+                               0.5f * (mz - lz) * side, hleaf * side, (float)g.box};
+        unsigned long long live = ~0ull;
+        int run = 0;
+        float fx = 0, fy = 0, fz = 0, fh = 0;
+        auto stage = [&](int k) {
+            st[k] = make_float4(fx, fy, fz, fh * fh);
+            sj[k] = j;
+        };
+        while (more || left) {
+            __syncthreads();  // the lanes have read the last tile
+            if (keep) stage(pos);  // what the last tile had no room for
+            keep = false;
+            left = false;
+            while (more && fill < 64) {
+                if (long_walk) {
+                    if ((run & 63) == 0)
+                        live = live_runs<true, 64>(reach, g.wide->boxes, v0, cells.total, [&](int v) { return cells.at(v); });
+                    const bool skip = !((live >> (run++ & 63)) & 1ull);
+                    if (skip) {
+                        v0 += 64;
+                        more = v0 < cells.total;
+                        continue;
+                    }
+                }
+                if (v0 + t < cells.total) {
+                    j = cells.at(v0 + t);
+                    if (j < 0) j = sorted[j + kCoarseRange];
+                    fx = rel(X[j], hx); fy = rel(Y[j], hy); fz = rel(Z[j], hz); fh = (float)(H[j] * inv_cell);
+                    keep = !culled(fx, fy, fz, fh);
+                }
+                int nt;
+                pos = fill + kept_rank(keep, nt);
+                if (keep && pos < 64) {
+                    stage(pos);
+                    keep = false;
+                }
+                fill += nt;
+                v0 += 64;
+                more = v0 < cells.total;
+            }
+            const int nt = fill < 64 ? fill : 64;
+            fill -= nt;
+            left = fill > 0;
+            pos -= 64;
+            __syncthreads();
+            const bool mine = t < nt;
+            const float4 u = mine ? st[t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const int cj = mine ? sj[t] : -1;
+            const float w = u.x * u.x + u.y * u.y + u.z * u.z;
+            const float slack = kSymSlack * (w + u.w + 13.0f);  // (a row's radius is at most the cell side)
+            for (int a = 0; a < rows; a++) {
+                const float d = __builtin_fmaf(lane_value(qx, a), u.x, __builtin_fmaf(lane_value(qy, a), u.y, __builtin_fmaf(lane_value(qz, a), u.z, w))) +
+                                lane_value(qn, a) - fmaxf(u.w, lane_value(qh, a));
+                const bool other = mine && cj != lane_value(i, a);
+                bool acc = other && d < -slack;
+                const bool close = other && (!small || fabsf(d) <= slack);
+                if (wave_any(close)) {
+                    if (close)
+                        acc = accept_pair<true>(lane_value(xi, a), lane_value(yi, a), lane_value(zi, a), X[cj], Y[cj], Z[cj], lane_value(hi, a), H[cj],
+                                                g.box, g.half);
+                }
+                int na;
+                const int place = lane_value(n, a) + kept_rank(acc, na);
+                if (acc && place < cap) ell[ell_at(ld, lane_value(r, a), place)] = cj;
+                if (t == a) n += na;
+            }
+        }
+        if (ncoarse > kMaxCoarse) {
+            // too many to collect: each accepted one inserted in ascending place of its row
             const WideGrid &W = *g.wide;
             for (int L = 0; L < g.level; L++) {
                 if (W.lofs[L + 1] == W.lofs[L]) continue;  // no particle of this level
                 __syncthreads();  // every lane is done with rs before it is built again
                 row_stencil_wide<true>(g, W, L, (uint32_t)c >> (3 * (g.level - L)), 0.0, 0.0, 0.0, -1.0, rs);
                 const int total = rs.pref[rs.nst];
-                for (int base2 = 0; base2 < total; base2 += 64) {
-                    const int v = base2 + t;
-                    bool keep = false;
-                    int j = -1;
+                for (v0 = 0; v0 < total; v0 += 64) {
+                    keep = false;
                     double xj = 0, yj = 0, zj = 0, hj = 0;
-                    if (v < total) {
-                        j = W.lidx[row_candidate(rs, v)];
-                        const uint32_t cj = W.key[j] >> si;
-                        const bool in_a = periodic_adjacent((int)compact10(cj >> 2), hx, nci) &&
-                                          periodic_adjacent((int)compact10(cj >> 1), hy, nci) && periodic_adjacent((int)compact10(cj), hz, nci);
-                        if (!in_a) {
+                    if (v0 + t < total) {
+                        j = W.lidx[row_candidate(rs, v0 + t)];
+                        if (outside(j)) {
                             xj = X[j]; yj = Y[j]; zj = Z[j]; hj = H[j];
-                            keep = leaf_reach(g, lb, xj, yj, zj, fmax(hleaf, hj));
+                            keep = !culled(rel(xj, hx), rel(yj, hy), rel(zj, hz), (float)(hj * inv_cell));
                         }
                     }
-                    int nt;
-                    const int pos = kept_rank(keep, nt);
-                    __syncthreads();
-                    if (keep) { sx[pos] = xj; sy[pos] = yj; sz[pos] = zj; sh[pos] = hj; sj[pos] = j; }
-                    __syncthreads();
-                    if (!on) continue;
-                    for (int k = 0; k < nt; k++) {
-                        const int jj = sj[k];
-                        if (jj == i || !accept_pair<true>(xi, yi, zi, sx[k], sy[k], sz[k], hi, sh[k], g.box, g.half)) continue;
+                    for (unsigned long long m = __ballot(keep); m; m &= m - 1) {
+                        const int k = __ffsll((long long)m) - 1, jj = lane_value(j, k);
+                        const double xk = lane_value(xj, k), yk = lane_value(yj, k), zk = lane_value(zj, k), hk = lane_value(hj, k);
+                        if (!on || jj == i || !accept_pair<true>(xi, yi, zi, xk, yk, zk, hi, hk, g.box, g.half)) continue;
                         if (n < cap) {
                             int q = n;
                             while (q > 0 && ell[ell_at(ld, r, q - 1)] > jj) { ell[ell_at(ld, r, q)] = ell[ell_at(ld, r, q - 1)]; q--; }
@@ -655,6 +1051,7 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
             cnt[r] = min(n, cap);  // readers stay inside the list; the overflow carries the full length
             if (n > cap) atomicMax(overflow, n);
         }
+        __syncthreads();  // before the next rows' ranges
     }
 }
 #endif
