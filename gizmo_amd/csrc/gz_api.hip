@@ -943,7 +943,7 @@ int density_rounds(gz_context *ctx, int iters, bool speculate)
                         ctx->M, ctx->it_h, ctx->dacc, BoxTable{}, npairs, rows, nround);
                 else {
                     auto cells_kernel = ctx->fd ? k_density_cells<KERN, R, true> : k_density_cells<KERN, R, false>;
-                    cells_kernel<<<xcd_grid(ctx->ncells), 64, 0, ctx->stream>>>(
+                    cells_kernel<<<dim3(xcd_grid(ctx->ncells), walk_parts(na, ctx->ncells)), 64, 0, ctx->stream>>>(
                         ctx->dp, grid_view(ctx), cell_rows(ctx), ctx->act, ctx->need, ctx->X, ctx->Y, ctx->Z, ctx->VX, ctx->VY, ctx->VZ,
                         ctx->M, ctx->it_h, ctx->dacc);
                 }
@@ -1093,7 +1093,7 @@ int ensure_sym(gz_context *ctx)
                                                                                ctx->Z, ctx->H, ctx->ell_s, ctx->ld_s, ctx->cap_s, ctx->cnt_s,
                                                                                ctx->counters + 3, BoxTable{});
             else
-                sym_kernel(ctx->nact, ctx->ncells)<<<xcd_grid(ctx->ncells), 64, 0, ctx->stream>>>(grid_view(ctx), cell_rows(ctx), ctx->act, ctx->X, ctx->Y,
+                sym_launch(ctx->nact, ctx->ncells).kernel<<<sym_launch(ctx->nact, ctx->ncells).grid, 64, 0, ctx->stream>>>(grid_view(ctx), cell_rows(ctx), ctx->act, ctx->X, ctx->Y,
                                                                                   ctx->Z, ctx->H, ctx->ell_s, ctx->ld_s, ctx->cap_s,
                                                                                   ctx->cnt_s, ctx->counters + 3);
             HIPCHK(hipGetLastError());

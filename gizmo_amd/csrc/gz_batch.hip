@@ -525,7 +525,7 @@ int density(gz_batch *b)
         if (na > b->few_rows) {
             BCHK(build_groups(b));
             auto cells_kernel = b->dp.fd4alpha > 0 ? k_density_cells<KERN, R, true> : k_density_cells<KERN, R, false>;
-            cells_kernel<<<xcd_grid(b->grp.ngroups), 64, 0, b->stream>>>(b->dp, gview(b), b->grp.view(bt), b->act, b->need, b->X, b->Y,
+            cells_kernel<<<dim3(xcd_grid(b->grp.ngroups), walk_parts(na, b->grp.ngroups)), 64, 0, b->stream>>>(b->dp, gview(b), b->grp.view(bt), b->act, b->need, b->X, b->Y,
                                                                          b->Z, b->VX, b->VY, b->VZ, b->M, b->it_h, b->dacc);
         } else {
             k_density_rows<KERN, R, kRowThreads><<<xcd_grid(na), kRowThreads, 0, b->stream>>>(b->dp, gview(b), na, b->act, b->need, b->key, b->X, b->Y, b->Z,
@@ -574,7 +574,7 @@ int sym_list(gz_batch *b, const std::vector<uint8_t> &in_pass)
         BHIP(hipMemsetAsync(b->counters + 3, 0, sizeof(int), b->stream));
         if (na > b->few_rows) {
             BCHK(build_groups(b));
-            sym_kernel(na, b->grp.ngroups)<<<xcd_grid(b->grp.ngroups), 64, 0, b->stream>>>(gview(b), b->grp.view(bt), b->act, b->X, b->Y, b->Z, b->H,
+            sym_launch(na, b->grp.ngroups).kernel<<<sym_launch(na, b->grp.ngroups).grid, 64, 0, b->stream>>>(gview(b), b->grp.view(bt), b->act, b->X, b->Y, b->Z, b->H,
                                                                                b->ell, ld, b->ell_cap, b->cnt, b->counters + 3);
         } else {
             k_build_sym_rows<<<xcd_grid(na), kRowThreads, 0, b->stream>>>(gview(b), na, b->act, b->key, b->X, b->Y, b->Z, b->H, b->ell, ld,

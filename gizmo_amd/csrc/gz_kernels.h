@@ -298,7 +298,23 @@ __global__ void k_build_sym_groups(GridView g, CellRows cr, const int *act, cons
 // time grows with the rows of a cell (4 of 31: 218 us against 524 with a row per lane) where the
 // other's does not
 constexpr int kSymFewRows = 16;
-inline auto sym_kernel(long nrows, long ncells) { return nrows <= kSymFewRows * ncells ? k_build_sym_groups : k_build_sym_cells; }
+// workgroups along y of the cell walks: enough for the rows of a cell, 64 each, when the cells hold
+// that many on average (a wavefront that walks a cell's candidates again for its next 64 rows
+// takes as long again; small boxes have fewer cells than the chip has wavefronts)
+inline unsigned walk_parts(long nrows, long ncells)
+{
+    const long p = (nrows + 48 * ncells - 1) / (48 * (ncells > 0 ? ncells : 1));
+    return (unsigned)(p < 1 ? 1 : (p > 16 ? 16 : p));
+}
+struct SymLaunch {
+    decltype(&k_build_sym_cells) kernel;
+    dim3 grid;
+};
+inline SymLaunch sym_launch(long nrows, long ncells)
+{
+    if (nrows <= kSymFewRows * ncells) return {k_build_sym_groups, dim3(xcd_grid(ncells))};
+    return {k_build_sym_cells, dim3(xcd_grid(ncells), walk_parts(nrows, ncells))};
+}
 
 // FD: with the sums of the first-derivative volume correction
 template <int KERN, typename R, bool FD>

@@ -644,8 +644,11 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
         c = cr.cells[cb]; a0 = cr.ca0[c]; a1 = cr.ca1[c]; nst = g.nsten[c]; sten = g.sten + (size_t)c * 27;
     }
     const int t = threadIdx.x;
-    for (int base = a0; base < a1; base += 64) {
-        const bool on = base + t < a1;
+    // a cell's rows in equal parts of at most 64, dealt to the workgroups along y
+    const int parts = (a1 - a0 + 63) / 64, part_rows = (a1 - a0 + parts - 1) / parts;
+    for (int part = blockIdx.y; part < parts; part += gridDim.y) {
+        const int base = a0 + part * part_rows;
+        const bool on = t < part_rows && base + t < a1;
         const int r = on ? (cr.grow ? cr.grow[base + t] : base + t) : 0;
         int i = -1;
         double xi = 0, yi = 0, zi = 0, hi = 0;
@@ -654,18 +657,23 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
         const double hleaf = wave_max(on ? hi : 0.0);
         const bool small = (1 << g.level) >= 8;
         const double inv_cell = 1.0 / g.cell;
-        float qx, qy, qz, qh, lim;
-        {
-            const float ux = (float)(wrap(xi - lb.ox, g.box, g.half) * inv_cell - 0.5), uy = (float)(wrap(yi - lb.oy, g.box, g.half) * inv_cell - 0.5),
-                        uz = (float)(wrap(zi - lb.oz, g.box, g.half) * inv_cell - 0.5), uh = (float)(hi * inv_cell);
-            qx = -2.0f * ux; qy = -2.0f * uy; qz = -2.0f * uz;
-            qh = uh * uh;
-            lim = on ? kWinSlack - (ux * ux + uy * uy + uz * uz) : -1e30f;
-        }
+        const float ux = (float)(wrap(xi - lb.ox, g.box, g.half) * inv_cell - 0.5), uy = (float)(wrap(yi - lb.oy, g.box, g.half) * inv_cell - 0.5),
+                    uz = (float)(wrap(zi - lb.oz, g.box, g.half) * inv_cell - 0.5), uh = (float)(hi * inv_cell);
+        const float qx = -2.0f * ux, qy = -2.0f * uy, qz = -2.0f * uz, qh = uh * uh;
+        const float lim = on ? (small ? kWinSlack - (ux * ux + uy * uy + uz * uz) : kWinSlack) : -1e30f;
         Window win;
         int head = 0, fill = 0, n = 0;
         int q = 0, ts = nst > 0 ? sten[0].x : 0, te = nst > 0 ? sten[0].y : 0;  // the next candidates
         bool more = nst > 0, left = false, keep = false;
+        // the next 64 candidates, loaded while the last are tested and staged (with the walk in
+        // parts along y: twelve boxes of 16^3 to 64^3 796 -> 704 us; 128^3 990 either way)
+        double xn = 0, yn = 0, zn = 0, hn = 0;
+        auto load_next = [&]() {
+            if (ts + t < te) {
+                xn = X[ts + t]; yn = Y[ts + t]; zn = Z[ts + t]; hn = H[ts + t];
+            }
+        };
+        load_next();
         int pos = 0, j = 0;
         double xj = 0, yj = 0, zj = 0, hj = 0;
         auto stage = [&](int k) {
@@ -682,11 +690,17 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
             keep = false;
             left = false;
             while (more && fill < 64) {
+                const bool in_range = ts + t < te;
                 j = ts + t;
-                if (j < te) {
-                    xj = X[j]; yj = Y[j]; zj = Z[j]; hj = H[j];
-                    keep = leaf_reach(g, lb, xj, yj, zj, fmax(hleaf, hj));
+                xj = xn; yj = yn; zj = zn; hj = hn;
+                ts += 64;
+                if (ts >= te) {
+                    q++;
+                    more = q < nst;
+                    if (more) { ts = sten[q].x; te = sten[q].y; }
                 }
+                if (more) load_next();
+                keep = in_range && leaf_reach(g, lb, xj, yj, zj, fmax(hleaf, hj));
                 int nt;
                 pos = fill + kept_rank(keep, nt);
                 if (keep && pos < 64) {
@@ -694,12 +708,6 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
                     keep = false;
                 }
                 fill += nt;
-                ts += 64;
-                if (ts >= te) {
-                    q++;
-                    more = q < nst;
-                    if (more) { ts = sten[q].x; te = sten[q].y; }
-                }
             }
             const int nt = fill < 64 ? fill : 64;
             fill -= nt;
@@ -716,10 +724,15 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
                     mask_push(mhi, __builtin_fmaf(qx, v.x, __builtin_fmaf(qy, v.y, __builtin_fmaf(qz, v.z, v.w))) - fmaxf(qh, sth[k + 32]), lim);
                 }
             } else {
-                // coarse grids: every candidate takes the exact test
-                const unsigned long long all = on ? (nt == 64 ? ~0ull : (1ull << nt) - 1ull) : 0ull;
-                mlo = (uint32_t)all;
-                mhi = (uint32_t)(all >> 32);
+                // coarse grids: the nearest image of each difference
+                const float nc = (float)(1 << g.level), inv_nc = 1.0f / nc;
+                for (int k = 31; k >= 0; k--) {
+                    mask_push(mlo, wrapped_r2(ux, uy, uz, st[k], nc, inv_nc) - fmaxf(qh, sth[k]), lim);
+                    mask_push(mhi, wrapped_r2(ux, uy, uz, st[k + 32], nc, inv_nc) - fmaxf(qh, sth[k + 32]), lim);
+                }
+                const unsigned long long valid = nt == 64 ? ~0ull : (1ull << nt) - 1ull;
+                mlo &= (uint32_t)valid;
+                mhi &= (uint32_t)(valid >> 32);
             }
             win.push(((unsigned long long)mhi << 32) | mlo);
             head = head == kWinRing - 64 ? 0 : head + 64;
