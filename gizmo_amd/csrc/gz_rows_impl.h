@@ -14,45 +14,75 @@ namespace gz {
 // code (cells are consecutive ranges of the Morton order, so this is ascending start: the
 // candidates come in ascending particle index whatever the grid level), laid end to end.
 // Virtual index v maps to the particle of range k with pref[k] <= v < pref[k+1].
+constexpr int kMarked = 1024;  // candidates whose range is found by counting bits (row_candidate_marked)
 struct RowStencil {
     int start[27];
     int pref[28];
-    int code[27];
     int len[27];
     int nst;
+    int shift[27];           // start - pref
+    unsigned long long first[kMarked / 64];  // a bit per candidate below kMarked: the first of its range
+    int range[kMarked / 64];                 // for each word: the range of the word's first candidate, less bit 0 of the word
 };
 
-// of equal codes (grids under 3 cells a side) the first lane stays; ranks by code; prefix of
-// the lengths.  Lanes below 27 bring their cell's code (0x7fffffff: dropped) and range, and
-// have stored the code in rs.code.
-__device__ __forceinline__ void stencil_finish(RowStencil &rs, int code, int st, int en)
+// the sum of the values of lanes 0 .. lane, for lanes below 32
+__device__ __forceinline__ int scan32(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    return x;
+}
+
+// The ranges in ascending code, of a grid of nc cells a side.  The lanes of the first wavefront bring
+// their cell's code (0x7fffffff: dropped, all lanes from 27 on) and range; of equal codes (grids under
+// 3 cells a side) the first lane stays.  The ranks come from 27 lane broadcasts and the prefix of
+// the lengths from a scan in registers: loops over LDS words here were a chain of 80 dependent
+// reads (about 5000 cycles), a third of the time of a row.
+__device__ __forceinline__ void stencil_finish(RowStencil &rs, int nc, int code, int st, int en)
 {
     const int lane = threadIdx.x;
-    __syncthreads();
-    bool first = false;
-    if (lane < 27 && code != 0x7fffffff) {
-        first = true;
-        for (int q = 0; q < lane; q++)
-            if (rs.code[q] == code) { first = false; break; }
+    int m = 0;
+    if (lane < 64) {
+        if (nc < 3) {
+            for (int q = 0; q < 26; q++) {
+                const int cq = lane_value(code, q);
+                if (lane > q && code == cq) code = 0x7fffffff;
+            }
+        }
+        const bool kept = code != 0x7fffffff;
+        int rank = 0;  // kept codes below this one
+#pragma unroll
+        for (int q = 0; q < 27; q++) rank += lane_value(code, q) < code;
+        m = __popcll(__ballot(kept));
+        if (kept) {
+            rs.start[rank] = st;
+            rs.len[rank] = en - st;
+        }
+        if (lane < kMarked / 64) rs.first[lane] = 0;
     }
-    const unsigned long long firsts = __ballot(first);
-    if (first) {
-        int rank = 0;  // distinct kept codes below this one
-        for (int q = 0; q < 27; q++)
-            if (((firsts >> q) & 1ull) && rs.code[q] < code) rank++;
-        rs.start[rank] = st;
-        rs.len[rank] = en - st;
+    __syncthreads();
+    if (lane < 64) {
+        const int len = lane < m ? rs.len[lane] : 0;
+        const int upto = scan32(len), pref = upto - len;
+        if (lane <= m) rs.pref[lane] = pref;
+        if (lane < m) {
+            rs.shift[lane] = rs.start[lane] - pref;
+            if (pref < kMarked) atomicOr(&rs.first[pref >> 6], 1ull << (pref & 63));
+        }
+        if (lane == 0) rs.nst = m;
     }
     __syncthreads();
-    if (lane == 0) {
-        const int m = __popcll(firsts);
-        int acc = 0;
-        for (int k = 0; k < m; k++) { rs.pref[k] = acc; acc += rs.len[k]; }
-        rs.pref[m] = acc;
-        rs.nst = m;
+    if (lane < 64) {
+        const unsigned long long word = lane < kMarked / 64 ? rs.first[lane] : 0ull;
+        const int marks = __popcll(word), upto = scan32(marks);
+        if (lane < kMarked / 64) rs.range[lane] = upto - marks + (int)(word & 1ull) - 1;
     }
     __syncthreads();
 }
+
 
 // The stencil of the row's home cell, built by 27 lanes (one per neighbour cell): periodic
 // neighbours, duplicates of small grids dropped, cells beyond reach dropped (the row lies
@@ -69,7 +99,7 @@ __device__ __forceinline__ void row_stencil(const GridView &g, uint32_t home, do
     int code = 0x7fffffff, st = 0, en = 0;
     if (lane < 27) {
         const int dx = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
-        const int a = (cx + dx + nc) % nc, b = (cy + dy + nc) % nc, d = (cz + dz + nc) % nc;
+        const int a = (cx + dx) & (nc - 1), b = (cy + dy) & (nc - 1), d = (cz + dz) & (nc - 1);
         const int c = (int)((spread10(a) << 2) | (spread10(b) << 1) | spread10(d));
         st = g.cstart[g.cell_off + c];
         en = g.cend[g.cell_off + c];
@@ -87,9 +117,8 @@ __device__ __forceinline__ void row_stencil(const GridView &g, uint32_t home, do
             if (gx * gx + gy * gy + gz * gz > rr * rr) keep = false;
         }
         if (keep) code = c;
-        rs.code[lane] = code;
     }
-    stencil_finish(rs, code, st, en);
+    stencil_finish(rs, nc, code, st, en);
 }
 
 // (v < the total; the range k with pref[k] <= v < pref[k+1], the last such k when empty ranges
@@ -105,6 +134,15 @@ __device__ __forceinline__ int row_candidate(const RowStencil &rs, int v)
     return rs.start[lo] + (v - rs.pref[lo]);
 }
 
+// the same for v < kMarked and below the total, where the wavefront's lanes hold 64 consecutive v
+// from a multiple of 64: the marks up to this lane's in its word
+__device__ __forceinline__ int row_candidate_marked(const RowStencil &rs, int v)
+{
+    const unsigned long long word = rs.first[v >> 6] >> 1;
+    const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(word >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)word, 0));
+    return v + rs.shift[rs.range[v >> 6] + below];
+}
+
 // ---------------------------------------------------------------------------------------
 // search over many grid levels (WideGrid)
 // ---------------------------------------------------------------------------------------
@@ -113,7 +151,11 @@ __device__ __forceinline__ int row_candidate(const RowStencil &rs, int v)
 __device__ __forceinline__ int wide_level(double box, int lmax, double reach)
 {
     int L = 0;
-    while (L < lmax && box / (double)(1 << (L + 1)) >= reach * (1.0 + 1e-6)) L++;
+    double side = 0.5 * box;  // of level L + 1 (halving is exact)
+    while (L < lmax && side >= reach * (1.0 + 1e-6)) {
+        L++;
+        side *= 0.5;
+    }
     return L;
 }
 
@@ -144,12 +186,12 @@ __device__ __forceinline__ void row_stencil_wide(const GridView &g, const WideGr
     const int lane = threadIdx.x;
     const int nc = 1 << L;
     const int s = 3 * (kFineLevel - L);
-    const double cell = g.box / (double)nc;
+    const double cell = ldexp(g.box, -L);
     const int cx = compact10(home >> 2), cy = compact10(home >> 1), cz = compact10(home);
     int code = 0x7fffffff, st = 0, en = 0;
     if (lane < 27) {
         const int dx = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
-        const int a = (cx + dx + nc) % nc, b = (cy + dy + nc) % nc, d = (cz + dz + nc) % nc;
+        const int a = (cx + dx) & (nc - 1), b = (cy + dy) & (nc - 1), d = (cz + dz) & (nc - 1);
         const uint32_t c = (spread10(a) << 2) | (spread10(b) << 1) | spread10(d);
         const long long e = W.loff[L] + c;
         bool keep = LIST ? wide_range(W.lstart, W.lend, e, W.key, W.lidx, W.lofs[L], W.lofs[L + 1], s, c, st, en)
@@ -165,9 +207,8 @@ __device__ __forceinline__ void row_stencil_wide(const GridView &g, const WideGr
         }
         if (!keep) { st = 0; en = 0; }
         if (keep) code = (int)c;
-        rs.code[lane] = code;
     }
-    stencil_finish(rs, code, st, en);
+    stencil_finish(rs, nc, code, st, en);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -232,13 +273,18 @@ __device__ __forceinline__ unsigned long long live_runs(const BlockReach &reach,
 constexpr int kLongWalk = 1024;  // candidates from which a walk asks for its live runs first
 
 // The place of this thread's entry among the flagged entries of its workgroup, in thread order
-// (total: the flagged entries of the workgroup).  One barrier: smask[TPB / 64] must not be read
-// by another round of the caller before the caller's next barrier.
+// (total: the flagged entries of the workgroup).  One barrier for several wavefronts, none for one:
+// smask[TPB / 64] must not be read by another round of the caller before the caller's next
+// barrier (two buffers in turn will do).
 template <int TPB>
 __device__ __forceinline__ int flagged_rank(bool flag, unsigned long long *smask, int &total)
 {
     const unsigned long long mask = __ballot(flag);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (TPB == 64) {
+        total = __popcll(mask);
+        return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+    }
     if (lane == 0) smask[w] = mask;
     __syncthreads();
     int before = 0;
@@ -270,7 +316,14 @@ __device__ __forceinline__ R ordered_sum(R acc, const R *s, int n, bool neg)
 }
 
 // density sums of the rows still iterating (DensitySpec::pair_kernel,
-// src/hydro/density_loop.h:1141-1385), the terms in k_density_cells' order
+// src/hydro/density_loop.h:1141-1385), the terms in k_density_cells' order.
+// Two phases: the candidates' distances find the partners (one in five to twenty), which a ring in LDS
+// collects in order; whenever it holds a workgroup's worth, each thread computes one partner's terms
+// and one thread per sum adds them in order.  The terms (about 150 instructions) thus run once per row
+// on full wavefronts where they ran for every candidate chunk that held a partner.  Bound by
+// latencies (the stencil, the candidates' gathers) and the 450 instructions of the stencil.
+// 1M lognormal rows FP64 1.90 -> 1.35 ms (mean of a pass's rounds), 4M FP32 4.3 -> 3.0 ms; 4 wavefronts per row for a few
+// hundred rows 19.2 -> 10.0 us.
 template <int KERN, typename R, int TPB>
 __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, int nrows, const int *__restrict__ act,
                                                      const uint8_t *__restrict__ need, const uint32_t *__restrict__ key,
@@ -282,8 +335,9 @@ __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, i
                                                      const int *__restrict__ rows, int nlist)
 {
     __shared__ RowStencil rs;
-    __shared__ R sc[kDensSumsFD][TPB + 1];  // the accepted candidates' terms, in candidate order (padded: no bank conflicts)
-    __shared__ unsigned long long smask[TPB / 64];
+    __shared__ R sc[kDensSumsFD][TPB + 1];  // the partners' terms, in candidate order (padded: no bank conflicts)
+    __shared__ int list[2 * TPB];           // a ring of partners found
+    __shared__ unsigned long long smask[2][TPB / 64];
     // workgroup b takes row b, or the b-th row of the list of rows still iterating; the pair
     // count goes to npairs[b]
     const long b = xcd_block();
@@ -323,88 +377,120 @@ __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, i
     const int total = rs.pref[rs.nst];
     const bool fd = P.fd4alpha > 0;
     const int nsum = fd ? kDensSumsFD : kDensSums;
+    const double inv_box = 1.0 / P.box;
     R acc = 0;  // thread q < nsum keeps sum q
-    int accepted = 0;  // thread 17: the row's pairs (the pass's work, counted when npairs is given)
-    const bool long_walk = g.wide && total > kLongWalk;
-    const BlockReach reach{(float)xi, (float)yi, (float)zi, 0.0f, 0.0f, 0.0f, (float)h, (float)g.box};
-    unsigned long long live = ~0ull;
-    for (int base = 0, run = 0; base < total; base += TPB, run++) {
-        if (long_walk) {
-            // (every wavefront of the workgroup finds the same bits)
-            if ((run & 63) == 0)
-                live = live_runs<false, TPB>(reach, g.wide->boxes, base, total, [&](int v) { return row_candidate(rs, v); });
-            if (!((live >> (run & 63)) & 1ull)) continue;
+    int accepted = 0;  // this wavefront's share of the row's pairs (the pass's work, counted when npairs is given)
+    // the separation from particle j; both uses below compute the same bits
+    auto separation = [&](int j, R &dp0, R &dp1, R &dp2) {
+        if (rel) {
+            dp0 = rxi - (R)wrap_near(X[j] - ox, P.box, inv_box);
+            dp1 = ryi - (R)wrap_near(Y[j] - oy, P.box, inv_box);
+            dp2 = rzi - (R)wrap_near(Z[j] - oz, P.box, inv_box);
+        } else {
+            dp0 = (R)wrap_near(xi - X[j], P.box, inv_box);
+            dp1 = (R)wrap_near(yi - Y[j], P.box, inv_box);
+            dp2 = (R)wrap_near(zi - Z[j], P.box, inv_box);
         }
-        const int v = base + tid;
-        bool ok = false;
-        R t[kDensSumsFD];
-        if (v < total) {
-            const int j = row_candidate(rs, v);
+    };
+    // the terms of the first nt partners of the list, side by side in LDS, and the sums over them
+    auto add_partners = [&](int first, int nt) {
+        __syncthreads();  // the list is whole
+        bool counted = false;
+        if (tid < nt) {
+            const int j = list[(first + tid) & (2 * TPB - 1)];
             const double mj = M[j];
-            if (mj > 0) {
-                R dp0, dp1, dp2;
-                if (rel) {
-                    dp0 = rxi - (R)wrap(X[j] - ox, g.box, g.half);
-                    dp1 = ryi - (R)wrap(Y[j] - oy, g.box, g.half);
-                    dp2 = rzi - (R)wrap(Z[j] - oz, g.box, g.half);
-                } else {
-                    double d0 = xi - X[j], d1 = yi - Y[j], d2 = zi - Z[j];
-                    d1 = wrap(d1, P.box, P.half);
-                    d0 = wrap(d0, P.box, P.half);
-                    d2 = wrap(d2, P.box, P.half);
-                    dp0 = (R)d0; dp1 = (R)d1; dp2 = (R)d2;
-                }
+            const R vxj = (R)VX[j], vyj = (R)VY[j], vzj = (R)VZ[j];
+            R dp0, dp1, dp2;
+            separation(j, dp0, dp1, dp2);
+            R t[kDensSumsFD];
+            // a retired particle adds zeros, and so does the particle itself (rr = 0) to all but the
+            // first three sums: sums that start at +0 stay the same bit for bit
+            for (int q = 0; q < kDensSumsFD; q++) t[q] = 0;
+            counted = mj > 0;
+            if (counted) {
                 const R r2 = dp0 * dp0 + dp1 * dp1 + dp2 * dp2;
-                if (r2 < h2) {
-                    const R rr = sqrt(r2);
-                    const R u = rr * hinv;
-                    R wk = 0, dwk = 0;
-                    kernel_main<KERN, 0>(u, hinv3, hinv4, wk, dwk);
-                    t[0] = wk;
-                    t[1] = (R)mj * wk;
-                    t[2] = -(R(3.0) * hinv * wk + u * dwk);
-                    ok = true;
-                    // the particle itself (rr = 0) adds to the first three sums only: its other
-                    // terms are +0, which leave a sum that starts at +0 unchanged bit for bit
-                    for (int q = 3; q < kDensSumsFD; q++) t[q] = 0;
-                    if (rr > 0) {
-                        t[4] = wk * (dp0 * dp0);
-                        t[5] = wk * (dp1 * dp1);
-                        t[6] = wk * (dp2 * dp2);
-                        t[7] = wk * (dp0 * dp1);
-                        t[8] = wk * (dp1 * dp2);
-                        t[9] = wk * (dp0 * dp2);
-                        t[10] = wk * dp0;
-                        t[11] = wk * dp1;
-                        t[12] = wk * dp2;
-                        const R dv0 = vxi - (R)VX[j], dv1 = vyi - (R)VY[j], dv2 = vzi - (R)VZ[j];
-                        t[3] = dwk * (dp0 * dv0 + dp1 * dv1 + dp2 * dv2) / rr;
-                        if (fd) {  // GradH_numer, GradH_denom (src/hydro/density_loop.h:1281-1286)
-                            t[13] = (dwk / rr) * dp0;
-                            t[14] = (dwk / rr) * dp1;
-                            t[15] = (dwk / rr) * dp2;
-                            t[16] = u * dwk;
-                        }
+                const R rr = sqrt(r2);
+                const R u = rr * hinv;
+                R wk = 0, dwk = 0;
+                kernel_main<KERN, 0>(u, hinv3, hinv4, wk, dwk);
+                t[0] = wk;
+                t[1] = (R)mj * wk;
+                t[2] = -(R(3.0) * hinv * wk + u * dwk);
+                if (rr > 0) {
+                    t[4] = wk * (dp0 * dp0);
+                    t[5] = wk * (dp1 * dp1);
+                    t[6] = wk * (dp2 * dp2);
+                    t[7] = wk * (dp0 * dp1);
+                    t[8] = wk * (dp1 * dp2);
+                    t[9] = wk * (dp0 * dp2);
+                    t[10] = wk * dp0;
+                    t[11] = wk * dp1;
+                    t[12] = wk * dp2;
+                    const R dv0 = vxi - vxj, dv1 = vyi - vyj, dv2 = vzi - vzj;
+                    t[3] = dwk * (dp0 * dv0 + dp1 * dv1 + dp2 * dv2) / rr;
+                    if (fd) {  // GradH_numer, GradH_denom (src/hydro/density_loop.h:1281-1286)
+                        t[13] = (dwk / rr) * dp0;
+                        t[14] = (dwk / rr) * dp1;
+                        t[15] = (dwk / rr) * dp2;
+                        t[16] = u * dwk;
                     }
                 }
             }
-        }
-        // the accepted candidates' terms packed in candidate order; threads 0-12 then add them
-        int nok;
-        const int pos = flagged_rank<TPB>(ok, smask, nok);
-        if (ok) {
             // static bounds: the terms stay in registers
-            for (int q = 0; q < kDensSums; q++) sc[q][pos] = t[q];
+            for (int q = 0; q < kDensSums; q++) sc[q][tid] = t[q];
             if (fd)
-                for (int q = kDensSums; q < kDensSumsFD; q++) sc[q][pos] = t[q];
+                for (int q = kDensSums; q < kDensSumsFD; q++) sc[q][tid] = t[q];
         }
+        accepted += __popcll(__ballot(counted));
         __syncthreads();
-        if (tid < nsum) acc = ordered_sum(acc, sc[tid], nok, tid == 3);
-        else if (tid == kDensSumsFD) accepted += nok;
-        __syncthreads();
+        if (tid < nsum) acc = ordered_sum(acc, sc[tid], nt, tid == 3);
+    };
+    const bool long_walk = g.wide && total > kLongWalk;
+    const bool marked = total <= kMarked;
+    const BlockReach reach{(float)xi, (float)yi, (float)zi, 0.0f, 0.0f, 0.0f, (float)h, (float)g.box};
+    unsigned long long live = ~0ull;
+    int head = 0, fill = 0;  // the partners found and not yet added: list places head .. head + fill - 1
+    for (int base = 0, run = 0; base < total || fill > 0; base += TPB, run++) {
+        bool walk = base < total;
+        if (walk && long_walk) {
+            // (every wavefront of the workgroup finds the same bits)
+            if ((run & 63) == 0)
+                live = live_runs<false, TPB>(reach, g.wide->boxes, base, total, [&](int v) { return row_candidate(rs, v); });
+            walk = (live >> (run & 63)) & 1ull;
+        }
+        if (walk) {
+            const int v = base + tid;
+            bool ok = false;
+            int j = 0;
+            if (v < total) {
+                j = marked ? row_candidate_marked(rs, v) : row_candidate(rs, v);
+                R dp0, dp1, dp2;
+                separation(j, dp0, dp1, dp2);
+                ok = dp0 * dp0 + dp1 * dp1 + dp2 * dp2 < h2;
+            }
+            int nok;
+            const int pos = flagged_rank<TPB>(ok, smask[run & 1], nok);
+            if (ok) list[(head + fill + pos) & (2 * TPB - 1)] = j;
+            fill += nok;
+        }
+        if (fill >= TPB || (base + TPB >= total && fill > 0)) {
+            const int nt = min(fill, TPB);
+            add_partners(head, nt);
+            head += nt;
+            fill -= nt;
+        }
     }
     if (tid < nsum) accout[(size_t)tid * nrows + r] = (double)acc;
-    if (tid == kDensSumsFD && npairs) npairs[b] = accepted;
+    if (npairs) {
+        __syncthreads();
+        if ((tid & 63) == 0) smask[0][tid >> 6] = (unsigned long long)accepted;
+        __syncthreads();
+        if (tid == 0) {
+            int all = 0;
+            for (int w = 0; w < TPB / 64; w++) all += (int)smask[0][w];
+            npairs[b] = all;
+        }
+    }
 }
 
 // the symmetric list of few rows (the same entries, in the same order, as k_build_sym_cells)
