@@ -99,6 +99,8 @@ struct gz_context {
     WideGrid wide_h{};
     WideGrid *wide_dev = nullptr;
     float4 *wboxes = nullptr;  // bounding boxes of 64 consecutive particles each
+    float4 *wlpos = nullptr;   // rounded positions and radii in the order of lidx
+    uint32_t *wlkey = nullptr; // keys in the order of lidx
     int *wstart = nullptr, *wend = nullptr, *wlstart = nullptr, *wlend = nullptr, *lidx = nullptr, *plev = nullptr, *lcount = nullptr;
     long long wcells_alloc = 0;
     long wide_key_version = -1;
@@ -422,6 +424,8 @@ void free_state(gz_context *c)
     dfree(c->wstart); dfree(c->wend); dfree(c->wlstart); dfree(c->wlend); dfree(c->lidx); dfree(c->plev); dfree(c->lcount);
     dfree(c->wide_dev);
     dfree(c->wboxes);
+    dfree(c->wlpos);
+    dfree(c->wlkey);
     {
         dfree(c->act_bits); dfree(c->act_bcount);
         dfree(c->sched); dfree(c->sched_part); dfree(c->flux); c->flux_bytes = 0; dfree(c->rl_a); dfree(c->rl_b);
@@ -709,12 +713,15 @@ int build_wide(gz_context *ctx, bool lists)
     if (!ctx->lidx) {
         CHK(dalloc(ctx, &ctx->lidx, ctx->cap)); CHK(dalloc(ctx, &ctx->plev, ctx->cap)); CHK(dalloc(ctx, &ctx->lcount, kFineLevel + 2));
         CHK(dalloc(ctx, &ctx->wide_dev, 1)); CHK(dalloc(ctx, &ctx->wboxes, 2 * ((ctx->cap + 63) / 64)));
+        CHK(dalloc(ctx, &ctx->wlpos, ctx->cap)); CHK(dalloc(ctx, &ctx->wlkey, ctx->cap));
     }
     W.key = ctx->key;
     W.n = (int)n;
     W.lmax = lmax;
     W.start = ctx->wstart; W.end = ctx->wend; W.lidx = ctx->lidx; W.lstart = ctx->wlstart; W.lend = ctx->wlend;
     W.boxes = ctx->wboxes;
+    W.lpos = ctx->wlpos;
+    W.lkey = ctx->wlkey;
     Timed t(ctx, "ngb_build");
     k_block_boxes<<<nblk(n), kBlock, 0, ctx->stream>>>((int)n, ctx->X, ctx->Y, ctx->Z, ctx->H, ctx->wboxes);
     HIPCHK(hipGetLastError());
@@ -741,7 +748,7 @@ int build_wide(gz_context *ctx, bool lists)
             W.lofs[L] = acc;
             if (L <= kFineLevel) acc += counts[L];
         }
-        k_wide_list_bounds<<<nblk(n), kBlock, 0, ctx->stream>>>(W, ctx->plev);
+        k_wide_list_bounds<<<nblk(n), kBlock, 0, ctx->stream>>>(W, ctx->plev, ctx->X, ctx->Y, ctx->Z, ctx->H);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipMemcpyAsync(ctx->wide_dev, &W, sizeof W, hipMemcpyHostToDevice, ctx->stream));

@@ -44,10 +44,12 @@ struct DevParams {
 // touch 64 lines per load and fetch them again as the gathered records evict them (measured on
 // the 2M all-active pass: list writes 3.8 -> 1.1 GB, gradient and force fetches up to 10x, the
 // pass 0.7 ms slower; the list build was no faster).
-constexpr int kEllChunk = 1;
+constexpr int kEllChunk = 4;
 __host__ __device__ __forceinline__ size_t ell_at(long ld, long r, int q)
 {
-    return ((size_t)(q / kEllChunk) * (size_t)ld + (size_t)r) * kEllChunk + (size_t)(q % kEllChunk);
+    // (ld < 2^31, q >= 0: one 32 x 32 bit product)
+    const unsigned k = (unsigned)q / kEllChunk;
+    return ((unsigned long long)k * (unsigned)ld + (size_t)r) * kEllChunk + ((unsigned)q - k * kEllChunk);
 }
 // entries to allocate per row for a list of width cap
 __host__ __device__ __forceinline__ int ell_width(int cap) { return (cap + kEllChunk - 1) / kEllChunk * kEllChunk; }

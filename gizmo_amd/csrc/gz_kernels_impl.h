@@ -418,7 +418,7 @@ __global__ void k_cell_rows_list(int nact, const int *__restrict__ act, const ui
 #endif
 
 
-__device__ __forceinline__ bool wave_any(bool v) { return __any(v ? 1 : 0) != 0; }
+__device__ __forceinline__ bool wave_any(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
 
 // ---------------------------------------------------------------------------------------
 // leaf culling for the cell walks.  A wavefront's particles (one leaf) have a bounding box in

@@ -15,16 +15,6 @@ namespace gz {
 // candidates come in ascending particle index whatever the grid level), laid end to end.
 // Virtual index v maps to the particle of range k with pref[k] <= v < pref[k+1].
 constexpr int kMarked = 1024;  // candidates whose range is found by counting bits (row_candidate_marked)
-struct RowStencil {
-    int start[27];
-    int pref[28];
-    int len[27];
-    int nst;
-    int shift[27];           // start - pref
-    unsigned long long first[kMarked / 64];  // a bit per candidate below kMarked: the first of its range
-    int range[kMarked / 64];                 // for each word: the range of the word's first candidate, less bit 0 of the word
-};
-
 // the sum of the values of lanes 0 .. lane, for lanes below 32
 __device__ __forceinline__ int scan32(int x)
 {
@@ -35,6 +25,41 @@ __device__ __forceinline__ int scan32(int x)
     x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
     return x;
 }
+
+struct RangeMarks {
+    unsigned long long first[kMarked / 64];  // a bit per candidate: the first of its range
+    int range[kMarked / 64];                 // for each word: the range of the word's first candidate, less bit 0 of the word
+    // candidate v's range, where the wavefront's lanes hold 64 consecutive v from a multiple of 64:
+    // the marks up to this lane's in its word
+    __device__ __forceinline__ int range_of(int v) const
+    {
+        const unsigned long long word = first[v >> 6] >> 1;
+        return range[v >> 6] + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(word >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)word, 0));
+    }
+    // built by one wavefront: cleared, each range's first candidate marked (no range is empty), counted
+    __device__ __forceinline__ void clear(int lane)
+    {
+        if (lane < kMarked / 64) first[lane] = 0;
+    }
+    __device__ __forceinline__ void mark(int pref)
+    {
+        if (pref < kMarked) atomicOr(&first[pref >> 6], 1ull << (pref & 63));
+    }
+    __device__ __forceinline__ void count(int lane)
+    {
+        const unsigned long long word = lane < kMarked / 64 ? first[lane] : 0ull;
+        const int marks = __popcll(word), upto = scan32(marks);
+        if (lane < kMarked / 64) range[lane] = upto - marks + (int)(word & 1ull) - 1;
+    }
+};
+struct RowStencil {
+    int start[27];
+    int pref[28];
+    int len[27];
+    int nst;
+    int shift[27];  // start - pref
+    RangeMarks marks;
+};
 
 // The ranges in ascending code, of a grid of nc cells a side.  The lanes of the first wavefront bring
 // their cell's code (0x7fffffff: dropped, all lanes from 27 on) and range; of equal codes (grids under
@@ -61,7 +86,7 @@ __device__ __forceinline__ void stencil_finish(RowStencil &rs, int nc, int code,
             rs.start[rank] = st;
             rs.len[rank] = en - st;
         }
-        if (lane < kMarked / 64) rs.first[lane] = 0;
+        rs.marks.clear(lane);
     }
     __syncthreads();
     if (lane < 64) {
@@ -70,16 +95,12 @@ __device__ __forceinline__ void stencil_finish(RowStencil &rs, int nc, int code,
         if (lane <= m) rs.pref[lane] = pref;
         if (lane < m) {
             rs.shift[lane] = rs.start[lane] - pref;
-            if (pref < kMarked) atomicOr(&rs.first[pref >> 6], 1ull << (pref & 63));
+            rs.marks.mark(pref);
         }
         if (lane == 0) rs.nst = m;
     }
     __syncthreads();
-    if (lane < 64) {
-        const unsigned long long word = lane < kMarked / 64 ? rs.first[lane] : 0ull;
-        const int marks = __popcll(word), upto = scan32(marks);
-        if (lane < kMarked / 64) rs.range[lane] = upto - marks + (int)(word & 1ull) - 1;
-    }
+    if (lane < 64) rs.marks.count(lane);
     __syncthreads();
 }
 
@@ -134,14 +155,8 @@ __device__ __forceinline__ int row_candidate(const RowStencil &rs, int v)
     return rs.start[lo] + (v - rs.pref[lo]);
 }
 
-// the same for v < kMarked and below the total, where the wavefront's lanes hold 64 consecutive v
-// from a multiple of 64: the marks up to this lane's in its word
-__device__ __forceinline__ int row_candidate_marked(const RowStencil &rs, int v)
-{
-    const unsigned long long word = rs.first[v >> 6] >> 1;
-    const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(word >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)word, 0));
-    return v + rs.shift[rs.range[v >> 6] + below];
-}
+// the same for totals up to kMarked, as RangeMarks::range_of
+__device__ __forceinline__ int row_candidate_marked(const RowStencil &rs, int v) { return v + rs.shift[rs.marks.range_of(v)]; }
 
 // ---------------------------------------------------------------------------------------
 // search over many grid levels (WideGrid)
@@ -160,20 +175,18 @@ __device__ __forceinline__ int wide_level(double box, int lmax, double reach)
 }
 
 // the range [a, b) of the cell with code c (key >> s) from table entry e, if the entry is
-// exactly a maximal run of that code among positions [lo, hi) (map: position -> particle,
-// nullptr for the order itself); otherwise the cell is empty
+// exactly a maximal run of that code among positions [lo, hi) (key: of each position); otherwise
+// the cell is empty
 __device__ __forceinline__ bool wide_range(const int *__restrict__ start, const int *__restrict__ end, long long e,
-                                           const uint32_t *__restrict__ key, const int *__restrict__ map, int lo, int hi, int s,
+                                           const uint32_t *__restrict__ key, int lo, int hi, int s,
                                            uint32_t c, int &a, int &b)
 {
     a = start[e];
     b = end[e];
     if (!(a >= lo && a < b && b <= hi)) return false;
-    auto code = [&](int p) { return key[map ? map[p] : p] >> s; };
-    if (code(a) != c || code(b - 1) != c) return false;
-    if (a > lo && code(a - 1) == c) return false;
-    if (b < hi && code(b) == c) return false;
-    return true;
+    // (all four at once: one wait)
+    const uint32_t first = key[a] >> s, last = key[b - 1] >> s, before = key[max(a - 1, lo)] >> s, after = key[min(b, hi - 1)] >> s;
+    return first == c && last == c && !(a > lo && before == c) && !(b < hi && after == c);
 }
 
 // The 27-cell stencil at level L around the row (home = the row's key >> s), from the tables
@@ -194,8 +207,8 @@ __device__ __forceinline__ void row_stencil_wide(const GridView &g, const WideGr
         const int a = (cx + dx) & (nc - 1), b = (cy + dy) & (nc - 1), d = (cz + dz) & (nc - 1);
         const uint32_t c = (spread10(a) << 2) | (spread10(b) << 1) | spread10(d);
         const long long e = W.loff[L] + c;
-        bool keep = LIST ? wide_range(W.lstart, W.lend, e, W.key, W.lidx, W.lofs[L], W.lofs[L + 1], s, c, st, en)
-                         : wide_range(W.start, W.end, e, W.key, nullptr, 0, W.n, s, c, st, en);
+        bool keep = LIST ? wide_range(W.lstart, W.lend, e, W.lkey, W.lofs[L], W.lofs[L + 1], s, c, st, en)
+                         : wide_range(W.start, W.end, e, W.key, 0, W.n, s, c, st, en);
         if (keep && nc >= 4 && reach > 0) {
             const double ox = cx * cell, oy = cy * cell, oz = cz * cell;
             const double rx = wrap(xi - ox, g.box, g.half), ry = wrap(yi - oy, g.box, g.half), rz = wrap(zi - oz, g.box, g.half);
@@ -240,9 +253,8 @@ struct BlockReach {
     float cx, cy, cz, ex, ey, ez, h, box;
     // whether a pair of a row and a particle of block b may lie within the larger radius (SYM) or the
     // row's; the slack covers the FP32 rounding of the positions and the boxes
-    template <bool SYM> __device__ __forceinline__ bool hits(const float4 *__restrict__ boxes, int b) const
+    template <bool SYM> __device__ __forceinline__ bool hits(const float4 &lo, const float4 &hi) const
     {
-        const float4 lo = boxes[2 * b], hi = boxes[2 * b + 1];
         const float half = 0.5f * box;
         auto gap = [&](float c, float e, float l, float m) {
             float d = fabsf(c - 0.5f * (l + m));
@@ -256,17 +268,31 @@ struct BlockReach {
 };
 
 // Of 64 runs of RUN candidates from v0 on (at(v): candidate v's particle, negative: not from the
-// order), the ones that may hold a partner, as a bit per run.  A run whose particles are
-// consecutive covers few blocks; any other run is kept.
-template <bool SYM, int RUN, typename At>
-__device__ __forceinline__ unsigned long long live_runs(const BlockReach &reach, const float4 *__restrict__ boxes, int v0, int total, At at)
+// order), the ones that may hold a partner, as a bit per run.  hit(lowest corner and largest
+// radius, highest corner) tells whether a block may hold one; all lanes call it together.  A run
+// whose particles are consecutive covers few blocks; any other run is kept.
+template <int RUN, typename At, typename Hit>
+__device__ __forceinline__ unsigned long long live_runs(const float4 *__restrict__ boxes, int v0, int total, At at, Hit hit)
 {
     const int a = v0 + RUN * (int)(threadIdx.x & 63);
     bool live = false;
+    int b = 1, e = 0;  // the blocks still to look at
     if (a < total) {
         const int last = min(a + RUN, total) - 1, j0 = at(a), j1 = at(last);
         live = j0 < 0 || j1 - j0 != last - a;
-        for (int b = j0 >> 6; !live && b <= j1 >> 6; b++) live = reach.hits<SYM>(boxes, b);
+        if (!live) {
+            b = j0 >> 6;
+            e = j1 >> 6;
+        }
+    }
+    while (wave_any(b <= e)) {
+        const bool look = b <= e;
+        const float4 lo = boxes[look ? 2 * b : 0], hi = boxes[look ? 2 * b + 1 : 0];
+        if (hit(lo, hi) && look) {
+            live = true;
+            e = -1;
+        }
+        b++;
     }
     return __ballot(live);
 }
@@ -455,7 +481,8 @@ __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, i
         if (walk && long_walk) {
             // (every wavefront of the workgroup finds the same bits)
             if ((run & 63) == 0)
-                live = live_runs<false, TPB>(reach, g.wide->boxes, base, total, [&](int v) { return row_candidate(rs, v); });
+                live = live_runs<TPB>(g.wide->boxes, base, total, [&](int v) { return row_candidate(rs, v); },
+                                      [&](const float4 &lo, const float4 &hi) { return reach.hits<false>(lo, hi); });
             walk = (live >> (run & 63)) & 1ull;
         }
         if (walk) {
@@ -581,7 +608,9 @@ __global__ void __launch_bounds__(256) k_particle_level(int n, const double *__r
 }
 
 // the range of every cell of level L among the particles of level L (positions in lidx)
-__global__ void __launch_bounds__(256) k_wide_list_bounds(WideGrid W, const int *__restrict__ plev)
+__global__ void __launch_bounds__(256) k_wide_list_bounds(WideGrid W, const int *__restrict__ plev, const double *__restrict__ X,
+                                                          const double *__restrict__ Y, const double *__restrict__ Z,
+                                                          const double *__restrict__ H)
 {
     const long p = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (p >= W.n) return;
@@ -592,12 +621,14 @@ __global__ void __launch_bounds__(256) k_wide_list_bounds(WideGrid W, const int 
     const int lo = W.lofs[L], hi = W.lofs[L + 1];
     if (p == lo || (W.key[W.lidx[p - 1]] >> s) != c) W.lstart[W.loff[L] + c] = (int)p;
     if (p + 1 == hi || (W.key[W.lidx[p + 1]] >> s) != c) W.lend[W.loff[L] + c] = (int)(p + 1);
+    W.lkey[p] = W.key[j];
+    W.lpos[p] = make_float4((float)X[j], (float)Y[j], (float)Z[j], (float)H[j]);
 }
 
 __device__ __forceinline__ bool periodic_adjacent(int a, int b, int nc)
 {
-    const int d = ((a - b) % nc + nc) % nc;
-    return d <= 1 || d >= nc - 1;
+    const int d = (a - b + 1) & (nc - 1);  // (nc is a power of two)
+    return d <= 2 || nc < 3;
 }
 
 // Symmetric rows r2 < max(h_i,h_j)^2 (src/mesh/sfc_tiles_functions.h:83-102) over many levels.
@@ -848,9 +879,10 @@ __global__ void __launch_bounds__(64) k_build_sym_cells(GridView g, CellRows cr,
 // of the last range k with pref[k] <= v.
 constexpr int kMaxRanges = 56;
 struct CellRanges {
-    int start[kMaxRanges];
+    int shift[kMaxRanges];  // start - pref
     int pref[kMaxRanges];
     int n, total;
+    RangeMarks marks;
     __device__ __forceinline__ int at(int v) const
     {
         int lo = 0, hi = n - 1;
@@ -859,7 +891,38 @@ struct CellRanges {
             if (pref[mid] <= v) lo = mid;
             else hi = mid - 1;
         }
-        return start[lo] + (v - pref[lo]);
+        return v + shift[lo];
+    }
+    // 64 consecutive v from a multiple of 64
+    __device__ __forceinline__ int at_lanes(int v) const { return total <= kMarked ? v + shift[marks.range_of(v)] : at(v); }
+    // laid out by one wavefront: lane k < 28 brings range 2 k (starting at a0, of len0 candidates) and
+    // range 2 k + 1; empty ones are dropped
+    __device__ __forceinline__ void lay(int a0, int len0, int a1, int len1)
+    {
+        const int lane = threadIdx.x & 63;
+        const int upto = scan32(len0 + len1), pref0 = upto - len0 - len1, pref1 = upto - len1;
+        const unsigned long long some0 = __ballot(len0 > 0), some1 = __ballot(len1 > 0), below = (1ull << lane) - 1;
+        const int k = __popcll(some0 & below) + __popcll(some1 & below);
+        marks.clear(lane);
+        __syncthreads();
+        if (len0 > 0) {
+            pref[k] = pref0;
+            shift[k] = a0 - pref0;
+            marks.mark(pref0);
+        }
+        if (len1 > 0) {
+            const int k1 = k + (len0 > 0);
+            pref[k1] = pref1;
+            shift[k1] = a1 - pref1;
+            marks.mark(pref1);
+        }
+        if (lane == 31) {
+            n = __popcll(some0) + __popcll(some1);
+            total = upto;
+        }
+        __syncthreads();
+        marks.count(lane);
+        __syncthreads();
     }
 };
 
@@ -868,21 +931,7 @@ __device__ __forceinline__ void stencil_ranges(CellRanges &cr, const int4 *__res
 {
     const int lane = threadIdx.x & 63;
     const int4 e = lane < nst ? sten[lane] : make_int4(0, 0, 0, 0);
-    const int len = e.y - e.x;
-    int sum = len;
-    for (int o = 1; o < 32; o <<= 1) {
-        const int up = __shfl_up(sum, o, 64);
-        if (lane >= o) sum += up;
-    }
-    if (lane < nst) {
-        cr.start[lane] = e.x;
-        cr.pref[lane] = sum - len;
-    }
-    if (lane == 31) {
-        cr.n = nst;
-        cr.total = sum;
-    }
-    __syncthreads();
+    cr.lay(0, 0, e.x, e.y - e.x);
 }
 
 // One candidate per lane and the rows of the group in turn: no lane is idle however few rows a cell
@@ -901,7 +950,7 @@ constexpr int kMaxCoarse = 768;
 // a dozen roundings of 2^-24 each of at most twice that
 constexpr float kSymSlack = 2e-6f;
 constexpr int kCoarseRange = 1 << 30;
-__global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr, const int *__restrict__ act,
+__global__ void __launch_bounds__(64, 4) k_build_sym_groups(GridView g, CellRows cr, const int *__restrict__ act,
                                                          const double *__restrict__ X, const double *__restrict__ Y,
                                                          const double *__restrict__ Z, const double *__restrict__ H,
                                                          int *__restrict__ ell, long ld, int cap, int *__restrict__ cnt,
@@ -935,15 +984,16 @@ __global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr
     const int nci = 1 << g.level;
     const int hx = compact10((uint32_t)c >> 2), hy = compact10((uint32_t)c >> 1), hz = compact10((uint32_t)c);
     const int si = 3 * (kFineLevel - g.level);
-    // the FP32 test: grids of at least 8 cells a side (a partner then lies within half a box of the
-    // cell's origin); 16 over many levels, whose coarse partners lie up to box / 2.6 from the row
-    const bool small = nci >= (wide ? 16 : 8);
+    // the FP32 tests relative to the cell: grids of at least 8 cells a side, where a partner lies
+    // within half a box of the cell's centre; 16 where particles of levels 0 and 1 may be partners,
+    // up to box / 2.6 from the row (those of level 2 reach a quarter)
+    const bool small = nci >= 16 || (nci == 8 && !(wide && g.wide->lofs[2] > 0));
     const double inv_cell = 1.0 / g.cell, inv_box = 1.0 / g.box;
     // a coordinate relative to the centre of the group's cell (index h along its axis), in cells
     auto rel = [&](double x, int h) { return (float)(wrap_near(x - h * g.cell, g.box, inv_box) * inv_cell - 0.5); };
     // a particle of a coarser level that the group's own cells do not hold
-    auto outside = [&](int j) {
-        const uint32_t cj = g.wide->key[j] >> si;
+    auto outside = [&](uint32_t key) {
+        const uint32_t cj = key >> si;
         return !(periodic_adjacent((int)compact10(cj >> 2), hx, nci) && periodic_adjacent((int)compact10(cj >> 1), hy, nci) &&
                  periodic_adjacent((int)compact10(cj), hz, nci));
     };
@@ -961,26 +1011,43 @@ __global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr
         const float mx = -wave_minf(on ? -ux : 1e30f), my = -wave_minf(on ? -uy : 1e30f), mz = -wave_minf(on ? -uz : 1e30f);
         const float hleaf = -wave_minf(on ? -uh : 0.0f);
         // a candidate that no row can reach (conservative: the slack covers the rounding)
-        auto culled = [&](float fx, float fy, float fz, float fh) {
-            const float ex = fmaxf(fmaxf(lx - fx, fx - mx), 0.0f), ey = fmaxf(fmaxf(ly - fy, fy - my), 0.0f),
-                        ez = fmaxf(fmaxf(lz - fz, fz - mz), 0.0f), hm = fmaxf(fh, hleaf);
+        auto culled = [&](float fx, float fy, float fz, float fh, float sl) {
+            const float ex = fmaxf(fmaxf(lx - fx, fx - mx) - sl, 0.0f), ey = fmaxf(fmaxf(ly - fy, fy - my) - sl, 0.0f),
+                        ez = fmaxf(fmaxf(lz - fz, fz - mz) - sl, 0.0f), hm = fmaxf(fh, hleaf);
             return small && ex * ex + ey * ey + ez * ez > hm * hm + kSymSlack * (fx * fx + fy * fy + fz * fz + hm * hm + 12.0f);
         };
         int ncoarse = 0;  // part B's particles (above kMaxCoarse: not collected)
         if (wide) {
             const WideGrid &W = *g.wide;
+            // the group's centre and the slack for positions rounded to 32 bits, in cells
+            const float bx = (float)g.box, inv_b = 1.0f / bx, ic = (float)inv_cell, sl = 4e-7f * (float)nci;
+            const float gx = (float)((hx + 0.5) * g.cell), gy = (float)((hy + 0.5) * g.cell), gz = (float)((hz + 0.5) * g.cell);
+            auto near = [&](float d) { return __builtin_fmaf(-__builtin_rintf(d * inv_b), bx, d) * ic; };
             for (int L = 0; L < g.level && ncoarse <= kMaxCoarse; L++) {
                 if (t == 0) runs[L] = ncoarse;
                 if (W.lofs[L + 1] == W.lofs[L]) continue;  // no particle of this level
                 __syncthreads();  // every lane is done with rs before it is built again
                 row_stencil_wide<true>(g, W, L, (uint32_t)c >> (3 * (g.level - L)), 0.0, 0.0, 0.0, -1.0, rs);
                 const int total = rs.pref[rs.nst];
+                int pn = 0;
+                float4 fn = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                auto load_next = [&](int v) {  // the next candidates, while the last are tested
+                    if (v < total) {
+                        pn = total <= kMarked ? row_candidate_marked(rs, v) : row_candidate(rs, v);
+                        fn = W.lpos[pn];
+                    }
+                };
+                load_next(t);
                 for (int v0 = 0; v0 < total; v0 += 64) {
-                    bool keep = false;
+                    const int p = pn;
+                    const float4 f = fn;
+                    load_next(v0 + 64 + t);
+                    bool keep = v0 + t < total && !culled(near(f.x - gx), near(f.y - gy), near(f.z - gz), f.w * ic, sl);
+                    if (!wave_any(keep)) continue;
                     int j = 0;
-                    if (v0 + t < total) {
-                        j = W.lidx[row_candidate(rs, v0 + t)];
-                        keep = outside(j) && !culled(rel(X[j], hx), rel(Y[j], hy), rel(Z[j], hz), (float)(H[j] * inv_cell));
+                    if (keep) {
+                        j = W.lidx[p];
+                        keep = outside(W.lkey[p]);
                     }
                     int nt;
                     const int pos = ncoarse + kept_rank(keep, nt);
@@ -1019,35 +1086,32 @@ __global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr
                 if (sorted[mid] < e.x) before = mid + 1;
                 else above = mid;
             }
-            const int prev = __shfl_up(before, 1, 64), bcount = before - (t ? prev : 0), len = e.y - e.x;
-            const int mine = t <= nst ? bcount + len : 0;
-            int sum = mine;
-            for (int o = 1; o < 32; o <<= 1) {
-                const int up = __shfl_up(sum, o, 64);
-                if (t >= o) sum += up;
-            }
-            if (t <= nst) {
-                cells.start[2 * t] = before - bcount - kCoarseRange;
-                cells.pref[2 * t] = sum - mine;
-                if (t < nst) {
-                    cells.start[2 * t + 1] = e.x;
-                    cells.pref[2 * t + 1] = sum - mine + bcount;
-                }
-            }
-            if (t == nst) {
-                cells.n = 2 * nst + 1;
-                cells.total = sum;
-            }
-            __syncthreads();
+            const int prev = __shfl_up(before, 1, 64), bcount = before - (t ? prev : 0);
+            cells.lay(before - bcount - kCoarseRange, t <= nst ? bcount : 0, e.x, t < nst ? e.y - e.x : 0);
         }
         const int rows = min(a1 - base, 64);
         int n = 0, fill = 0, v0 = 0, pos = 0, j = 0;
         bool more = cells.total > 0, left = false, keep = false;
-        const bool long_walk = wide && small && cells.total > kLongWalk;
+        const bool long_walk = wide && cells.total > kLongWalk;
+        const float ncf = (float)nci, inv_ncf = 1.0f / ncf;
         const float side = (float)g.cell;
         const BlockReach reach{(float)(hx * g.cell) + (0.5f * (lx + mx) + 0.5f) * side, (float)(hy * g.cell) + (0.5f * (ly + my) + 0.5f) * side,
                                (float)(hz * g.cell) + (0.5f * (lz + mz) + 0.5f) * side, 0.5f * (mx - lx) * side, 0.5f * (my - ly) * side,
                                0.5f * (mz - lz) * side, hleaf * side, (float)g.box};
+        // a block within reach of the rows' box and, for few rows, of one of them: a coarse cell's few
+        // rows span a box that holds whole clumps which none of them reaches
+        const float xf = (float)xi, yf = (float)yi, zf = (float)zi, hf = (float)hi;
+        auto hit = [&](const float4 &lo, const float4 &hi) {
+            bool any = reach.hits<true>(lo, hi);
+            if (rows <= 16 && wave_any(any)) {
+                bool one = false;
+                for (int a = 0; a < rows; a++)
+                    one |= BlockReach{lane_value(xf, a), lane_value(yf, a), lane_value(zf, a), 0.0f, 0.0f, 0.0f, lane_value(hf, a),
+                                      reach.box}.hits<true>(lo, hi);
+                any = any && one;
+            }
+            return any;
+        };
         unsigned long long live = ~0ull;
         int run = 0;
         float fx = 0, fy = 0, fz = 0, fh = 0;
@@ -1063,7 +1127,7 @@ __global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr
             while (more && fill < 64) {
                 if (long_walk) {
                     if ((run & 63) == 0)
-                        live = live_runs<true, 64>(reach, g.wide->boxes, v0, cells.total, [&](int v) { return cells.at(v); });
+                        live = live_runs<64>(g.wide->boxes, v0, cells.total, [&](int v) { return cells.at(v); }, hit);
                     const bool skip = !((live >> (run++ & 63)) & 1ull);
                     if (skip) {
                         v0 += 64;
@@ -1072,10 +1136,10 @@ __global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr
                     }
                 }
                 if (v0 + t < cells.total) {
-                    j = cells.at(v0 + t);
+                    j = cells.at_lanes(v0 + t);
                     if (j < 0) j = sorted[j + kCoarseRange];
                     fx = rel(X[j], hx); fy = rel(Y[j], hy); fz = rel(Z[j], hz); fh = (float)(H[j] * inv_cell);
-                    keep = !culled(fx, fy, fz, fh);
+                    keep = !culled(fx, fy, fz, fh, 0.0f);
                 }
                 int nt;
                 pos = fill + kept_rank(keep, nt);
@@ -1097,21 +1161,28 @@ __global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr
             const int cj = mine ? sj[t] : -1;
             const float w = u.x * u.x + u.y * u.y + u.z * u.z;
             const float slack = kSymSlack * (w + u.w + 13.0f);  // (a row's radius is at most the cell side)
+            const unsigned long long tile = nt == 64 ? ~0ull : (1ull << nt) - 1ull;
             for (int a = 0; a < rows; a++) {
-                const float d = __builtin_fmaf(lane_value(qx, a), u.x, __builtin_fmaf(lane_value(qy, a), u.y, __builtin_fmaf(lane_value(qz, a), u.z, w))) +
-                                lane_value(qn, a) - fmaxf(u.w, lane_value(qh, a));
-                const bool other = mine && cj != lane_value(i, a);
-                bool acc = other && d < -slack;
-                const bool close = other && (!small || fabsf(d) <= slack);
-                if (wave_any(close)) {
-                    if (close)
-                        acc = accept_pair<true>(lane_value(xi, a), lane_value(yi, a), lane_value(zi, a), X[cj], Y[cj], Z[cj], lane_value(hi, a), H[cj],
-                                                g.box, g.half);
+                const float r2 = small ? __builtin_fmaf(lane_value(qx, a), u.x, __builtin_fmaf(lane_value(qy, a), u.y, __builtin_fmaf(lane_value(qz, a), u.z, w))) + lane_value(qn, a)
+                                       : wrapped_r2(lane_value(ux, a), lane_value(uy, a), lane_value(uz, a), u, ncf, inv_ncf);
+                // (squares: the larger is the larger as an integer)
+                const float d = r2 - __int_as_float(max(__float_as_int(u.w), lane_value(__float_as_int(qh), a)));
+                const unsigned long long others = tile & ~__builtin_amdgcn_ballot_w64(cj == lane_value(i, a));
+                const unsigned long long within = __builtin_amdgcn_ballot_w64(d < -slack);
+                const unsigned long long close = others & (within ^ __builtin_amdgcn_ballot_w64(d <= slack));
+                unsigned long long acc = others & within;
+                if (close) {
+                    bool in = false;
+                    if ((close >> t) & 1ull)
+                        in = accept_pair<true>(lane_value(xi, a), lane_value(yi, a), lane_value(zi, a), X[cj], Y[cj], Z[cj], lane_value(hi, a), H[cj],
+                                               g.box, g.half);
+                    acc |= __builtin_amdgcn_ballot_w64(in);
                 }
-                int na;
-                const int place = lane_value(n, a) + kept_rank(acc, na);
-                if (acc && place < cap) ell[ell_at(ld, lane_value(r, a), place)] = cj;
-                if (t == a) n += na;
+                if (!acc) continue;
+                const int held = lane_value(n, a);
+                const int place = __builtin_amdgcn_mbcnt_hi((unsigned)(acc >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)acc, held));
+                if (((acc >> t) & 1ull) && place < cap) ell[ell_at(ld, lane_value(r, a), place)] = cj;
+                if (t == a) n += __popcll(acc);
             }
         }
         if (ncoarse > kMaxCoarse) {
@@ -1127,9 +1198,9 @@ __global__ void __launch_bounds__(64) k_build_sym_groups(GridView g, CellRows cr
                     double xj = 0, yj = 0, zj = 0, hj = 0;
                     if (v0 + t < total) {
                         j = W.lidx[row_candidate(rs, v0 + t)];
-                        if (outside(j)) {
+                        if (outside(W.key[j])) {
                             xj = X[j]; yj = Y[j]; zj = Z[j]; hj = H[j];
-                            keep = !culled(rel(xj, hx), rel(yj, hy), rel(zj, hz), (float)(hj * inv_cell));
+                            keep = !culled(rel(xj, hx), rel(yj, hy), rel(zj, hz), (float)(hj * inv_cell), 0.0f);
                         }
                     }
                     for (unsigned long long m = __ballot(keep); m; m &= m - 1) {

@@ -31,8 +31,10 @@ BOXES = {
 }
 
 
-def run(ic, few_rows, precision, active, fd):
+def run(ic, few_rows, precision, active, fd, wide=False):
     g = Hydro(dict(ic["params"]), len(ic["mass"]), precision)
+    if wide:
+        g.set_option("wide_search", 1)
     g.set_option("few_rows", few_rows)
     if fd:
         g.set_option("fd_correction", 1)
@@ -56,6 +58,21 @@ def test_many_rows_equal_row_kernels(name, active, fd, precision):
     print(f"shapes: {name} n={len(ic['mass'])} active={active} fd={fd} precision={precision}", flush=True)
     a = run(ic, 0, precision, active, fd)
     b = run(ic, 10 ** 9, precision, active, fd)
+    for k in FIELDS:
+        same = a[k].view(np.int64 if a[k].dtype == np.float64 else a[k].dtype) == b[k].view(np.int64 if b[k].dtype == np.float64 else b[k].dtype)
+        assert np.isfinite(a[k]).all() and same.all(), (k, int((~same).sum()), same.size)
+
+
+@pytest.mark.parametrize("precision", [GZ_FP64, GZ_FP32_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("name,active", [("two_cells", 1.0), ("four_cells", 0.3), ("eight_cells", 1.0), ("clustered", 1.0), ("clustered", 0.4),
+                                         ("blast", 1.0)])
+def test_groups_of_many_levels_equal_row_kernels(name, active, precision):
+    """The symmetric list of the search over many levels, by groups of rows and row by row: coarse
+    levels (2 and 4 cells a side, where differences wrap), long walks, particles of coarser levels."""
+    ic = BOXES[name]()
+    print(f"levels: {name} n={len(ic['mass'])} active={active} precision={precision}", flush=True)
+    a = run(ic, 0, precision, active, False, wide=True)
+    b = run(ic, 10 ** 9, precision, active, False, wide=True)
     for k in FIELDS:
         same = a[k].view(np.int64 if a[k].dtype == np.float64 else a[k].dtype) == b[k].view(np.int64 if b[k].dtype == np.float64 else b[k].dtype)
         assert np.isfinite(a[k]).all() and same.all(), (k, int((~same).sum()), same.size)
