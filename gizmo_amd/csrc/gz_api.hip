@@ -173,7 +173,7 @@ struct gz_context {
 
     // density iteration state (per slot)
     double *it_h = nullptr, *it_hb = nullptr, *it_l = nullptr, *it_r = nullptr, *it_cn = nullptr;
-    int *it_ci = nullptr, *it_it = nullptr, *todo = nullptr, *todo2 = nullptr;
+    int *it_ci = nullptr, *it_it = nullptr;
     int *counters = nullptr;   // device: [0] next count, [1] rebuild flag, [2] error, [3] overflow,
                                // [4] wake-up flagged, [5] woken count, [6] timestep stop code,
                                // [8..9] wake-up bin limits, [10] active count
@@ -385,8 +385,9 @@ int alloc_state(gz_context *ctx, long cap)
     CHK(dalloc(ctx, &ctx->stage, 9 * n));
     CHK(dalloc(ctx, &ctx->it_h, n)); CHK(dalloc(ctx, &ctx->it_hb, n)); CHK(dalloc(ctx, &ctx->it_l, n));
     CHK(dalloc(ctx, &ctx->it_r, n)); CHK(dalloc(ctx, &ctx->it_cn, n)); CHK(dalloc(ctx, &ctx->it_ci, n));
-    CHK(dalloc(ctx, &ctx->it_it, n)); CHK(dalloc(ctx, &ctx->todo, n)); CHK(dalloc(ctx, &ctx->todo2, n));
-    CHK(dalloc(ctx, &ctx->cnt_d, n)); CHK(dalloc(ctx, &ctx->cnt_s, n));
+    CHK(dalloc(ctx, &ctx->it_it, n));
+    if (!ctx->pool) CHK(dalloc(ctx, &ctx->cnt_d, n));  // (pair counts of timed density rounds)
+    CHK(dalloc(ctx, &ctx->cnt_s, n));
     CHK(dalloc(ctx, &ctx->cells, n)); CHK(dalloc(ctx, &ctx->cflag, n + 1)); CHK(dalloc(ctx, &ctx->cscan, n + 1));
     CHK(dalloc(ctx, &ctx->need, n));
     CHK(dalloc(ctx, &ctx->dacc, kDensSumsFD * n));
@@ -444,7 +445,7 @@ void free_state(gz_context *c)
         v.clear();
     }
     dfree(c->it_h); dfree(c->it_hb); dfree(c->it_l); dfree(c->it_r); dfree(c->it_cn); dfree(c->it_ci); dfree(c->it_it);
-    dfree(c->todo); dfree(c->todo2); dfree(c->cnt_d); dfree(c->cnt_s); dfree(c->ell_d); dfree(c->ell_s);
+    dfree(c->cnt_d); dfree(c->cnt_s); dfree(c->ell_d); dfree(c->ell_s);
     c->counters = nullptr;  // inside u64c
     dfree(c->cstart); dfree(c->cend); dfree(c->nsten); dfree(c->sten); dfree(c->chmax);
     dfree(c->ca0); dfree(c->ca1); dfree(c->cmark); dfree(c->dcells); dfree(c->cells); dfree(c->cflag); dfree(c->cscan); dfree(c->need);

@@ -38,12 +38,11 @@ struct DevParams {
 };
 
 // Neighbour lists (ELL): entry q of row r lives in chunks of kEllChunk consecutive entries of one
-// row; chunk k of every row (ld rows apart), then chunk k+1.  kEllChunk = 1 is column-major: the
-// lanes of a wave, one row each, read entry q from whole lines shared by 16 rows.  Chunks of 16
-// (one line per row chunk) write each line once as a row appends, but lane-per-row readers then
-// touch 64 lines per load and fetch them again as the gathered records evict them (measured on
-// the 2M all-active pass: list writes 3.8 -> 1.1 GB, gradient and force fetches up to 10x, the
-// pass 0.7 ms slower; the list build was no faster).
+// row; chunk k of every row (ld rows apart), then chunk k+1.  4 entries (16 bytes): a wavefront's rows
+// still read entry q from whole lines, shared by 8 rows, and a row's writes go to a quarter of
+// the lines and pages.  Measured against 1 (column-major): the list of 4M lognormal rows 7.05 -> 6.49 ms, their
+// force pass 15.5 -> 14.7, the gradients of 2M rows 1.96 -> 1.86; against 16 (a line per row chunk):
+// those gradients 2.38, the list of 4M rows 6.33.
 constexpr int kEllChunk = 4;
 __host__ __device__ __forceinline__ size_t ell_at(long ld, long r, int q)
 {
