@@ -1139,28 +1139,36 @@ int gradients_stage(gz_context *ctx)
     GradRec<R> *rec = (GradRec<R> *)ctx->rec_grad;
     // few rows among many particles: the row kernel makes the records it reads (no packing launch)
     const bool make = ctx->nact <= ctx->few_rows && ctx->pack_list;
+    const bool few = ctx->nact <= ctx->few_rows;
+    // many rows: their records in the room of the force records, which are packed after this pass
+    auto *lane_rec = (GradLaneRec<R> *)ctx->rec_force;
+    auto pack = [&](auto *to) {
+        using Rec = std::remove_pointer_t<decltype(to)>;
+        if (ctx->pack_list)
+            k_pack_grad_list<R, Rec><<<xcd_grid(ctx->nact), 64, 0, ctx->stream>>>(ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->H,
+                                                                                  ctx->M, ctx->RHO, ctx->PR, ctx->VX, ctx->VY, ctx->VZ, to,
+                                                                                  ctx->X, ctx->Y, ctx->Z, ctx->par.box_size, BoxTable{});
+        else
+            k_pack_grad<R, Rec><<<nblk(ctx->n), kBlock, 0, ctx->stream>>>(ctx->n, ctx->H, ctx->M, ctx->RHO, ctx->PR, ctx->VX, ctx->VY, ctx->VZ,
+                                                                          to, ctx->X, ctx->Y, ctx->Z, ctx->par.box_size, BoxTable{});
+    };
     if (!make) {
         Timed t(ctx, "pack_grad");
-        if (ctx->pack_list)
-            k_pack_grad_list<R><<<xcd_grid(ctx->nact), 64, 0, ctx->stream>>>(ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->H,
-                                                                             ctx->M, ctx->RHO, ctx->PR, ctx->VX, ctx->VY, ctx->VZ, rec,
-                                                                             ctx->X, ctx->Y, ctx->Z, ctx->par.box_size, BoxTable{});
-        else
-            k_pack_grad<R><<<nblk(ctx->n), kBlock, 0, ctx->stream>>>(ctx->n, ctx->H, ctx->M, ctx->RHO, ctx->PR, ctx->VX, ctx->VY, ctx->VZ,
-                                                                     rec, ctx->X, ctx->Y, ctx->Z, ctx->par.box_size, BoxTable{});
+        if (few) pack(rec);
+        else pack(lane_rec);
     }
     Timed t(ctx, "gradients");
     // with its records made in the row kernels too, the force pass's flags are cleared here
     ctx->force_flags_clear = make;
-    if (ctx->nact <= ctx->few_rows)
+    if (few)
         k_gradients_rows<KERN, R><<<xcd_grid(ctx->nact), kListThreads, 0, ctx->stream>>>(
             ctx->dp, ctx->nact, ctx->act, ctx->X, ctx->Y, ctx->Z, ctx->H, rec,
             make ? GradSrc{ctx->H, ctx->M, ctx->RHO, ctx->PR, ctx->VX, ctx->VY, ctx->VZ, ctx->par.box_size} : GradSrc{}, ctx->T, ctx->CN,
             ctx->n, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->GR, ctx->GP, ctx->GV, BoxTable{}, make ? ctx->counters + 2 : nullptr);
     else
-        k_gradients<KERN, R, false><<<xcd_grid(nblk(ctx->nact)), kBlock, 0, ctx->stream>>>(ctx->dp, ctx->nact, ctx->act, ctx->X, ctx->Y, ctx->Z, ctx->H,
-                                                                                    rec, ctx->T, ctx->CN, ctx->n, ctx->ell_s, ctx->ld_s,
-                                                                                    ctx->cnt_s, ctx->GR, ctx->GP, ctx->GV, BoxTable{});
+        k_gradients<KERN, R, false><<<xcd_grid(nblk(ctx->nact)), kBlock, 0, ctx->stream>>>(ctx->dp, ctx->nact, ctx->act, ctx->H, lane_rec, ctx->T,
+                                                                                    ctx->CN, ctx->n, ctx->ell_s, ctx->ld_s, ctx->cnt_s,
+                                                                                    ctx->GR, ctx->GP, ctx->GV, BoxTable{});
     HIPCHK(hipGetLastError());
     ctx->gradients_done = true;
     return 0;

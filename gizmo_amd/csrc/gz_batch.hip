@@ -604,15 +604,22 @@ int gradients_force(gz_batch *b)
     // record once per list entry that names it: cheaper while the lists hold fewer entries than
     // there are particles)
     const bool list = (long)na * 64 < b->cap;
-    if (list)
-        k_pack_grad_list<R><<<xcd_grid(na), 64, 0, b->stream>>>(na, b->act, b->ell, ld, b->cnt, b->H, b->M, b->RHO, b->PR, b->VX, b->VY,
-                                                                b->VZ, rg, b->X, b->Y, b->Z, 1.0, bt);
-    else
-        k_pack_grad<R><<<nb(b->cap), kB, 0, b->stream>>>(b->cap, b->H, b->M, b->RHO, b->PR, b->VX, b->VY, b->VZ, rg, b->X, b->Y, b->Z, 1.0,
-                                                          bt);
     const bool lanes = na > b->few_rows;  // many rows: one lane per row
+    // (their records in the room of the force records, which are packed after the gradients)
+    auto *lane_rec = (GradLaneRec<R> *)b->rec_force;
+    auto pack = [&](auto *to) {
+        using Rec = std::remove_pointer_t<decltype(to)>;
+        if (list)
+            k_pack_grad_list<R, Rec><<<xcd_grid(na), 64, 0, b->stream>>>(na, b->act, b->ell, ld, b->cnt, b->H, b->M, b->RHO, b->PR, b->VX, b->VY,
+                                                                         b->VZ, to, b->X, b->Y, b->Z, 1.0, bt);
+        else
+            k_pack_grad<R, Rec><<<nb(b->cap), kB, 0, b->stream>>>(b->cap, b->H, b->M, b->RHO, b->PR, b->VX, b->VY, b->VZ, to, b->X, b->Y, b->Z,
+                                                                  1.0, bt);
+    };
+    if (lanes) pack(lane_rec);
+    else pack(rg);
     if (lanes)
-        k_gradients<KERN, R, true><<<xcd_grid(nb(na)), kB, 0, b->stream>>>(b->dp, na, b->act, b->X, b->Y, b->Z, b->H, rg, b->T, b->CN, b->cap, b->ell, ld,
+        k_gradients<KERN, R, true><<<xcd_grid(nb(na)), kB, 0, b->stream>>>(b->dp, na, b->act, b->H, lane_rec, b->T, b->CN, b->cap, b->ell, ld,
                                                                       b->cnt, b->GR, b->GP, b->GV, bt);
     else
         k_gradients_rows<KERN, R><<<xcd_grid(na), kListThreads, 0, b->stream>>>(b->dp, na, b->act, b->X, b->Y, b->Z, b->H, rg, GradSrc{}, b->T, b->CN, b->cap,

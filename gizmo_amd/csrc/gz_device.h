@@ -1085,5 +1085,13 @@ template <typename R> struct alignas(16) GradRec : PosRec<R> {
     R h, m;
     double rho, p, v0, v1, v2;
 };
+// the record of the pass over many rows: with the position in the FP64 form too (FP32 form: the
+// fine position is there already), in whole pieces of 16 bytes
+struct alignas(16) GradPosRec {
+    double h, m, rho, p, v0, v1, v2, x, y, z;
+};
+template <typename R> struct GradLaneRecOf { using type = GradPosRec; };
+template <> struct GradLaneRecOf<float> { using type = GradRec<float>; };
+template <typename R> using GradLaneRec = typename GradLaneRecOf<R>::type;
 
 }  // namespace gz

@@ -333,24 +333,24 @@ __global__ void k_density_after(DevParams P, int nrows, const int *act, uint8_t 
                                 unsigned long long *hfinal, BoxTable bt, double hlim = 0, int *gate = nullptr,
                                 unsigned int *done = nullptr, const int *rows = nullptr, int nlist = 0, int *next_rows = nullptr);
 
-template <typename R>
+// Rec: GradRec<R> (row kernels) or GradLaneRec<R> (k_gradients)
+template <typename R, typename Rec>
 __global__ void k_pack_grad(long n, const double *H, const double *M, const double *RHO, const double *PR, const double *VX,
-                            const double *VY, const double *VZ, GradRec<R> *rec, const double *X, const double *Y, const double *Z,
+                            const double *VY, const double *VZ, Rec *rec, const double *X, const double *Y, const double *Z,
                             double box, BoxTable bt);
 template <typename R>
 __global__ void k_pack_force(double gamma, ForceView F, Cell<R> *rec, int *zero2, double box, BoxTable bt);
-template <typename R>
+template <typename R, typename Rec>
 __global__ void k_pack_grad_list(int nrows, const int *act, const int *ell, long ld, const int *cnt, const double *H, const double *M,
                                  const double *RHO, const double *PR, const double *VX, const double *VY, const double *VZ,
-                                 GradRec<R> *rec, const double *X, const double *Y, const double *Z, double box, BoxTable bt);
+                                 Rec *rec, const double *X, const double *Y, const double *Z, double box, BoxTable bt);
 template <typename R>
 __global__ void k_pack_force_list(int nrows, const int *act, const int *ell, long ld, const int *cnt, double gamma, ForceView F,
                                   Cell<R> *rec, int *zero2, double box, BoxTable bt);
 
 // BOXES: each row's box geometry from bt (batches); else the single box of the arguments
 template <int KERN, typename R, bool BOXES>
-__global__ void k_gradients(DevParams P, int nrows, const int *act, const double *X, const double *Y, const double *Z,
-                            const double *H, const GradRec<R> *rec, const double *T, const double *CN, long n, const int *ell, long ld,
+__global__ void k_gradients(DevParams P, int nrows, const int *act, const double *H, const GradLaneRec<R> *rec, const double *T, const double *CN, long n, const int *ell, long ld,
                             const int *cnt, double *GR, double *GP, double *GV, BoxTable bt);
 
 // one workgroup per active row, for passes over few rows: kRowThreads lanes (4 wavefronts)

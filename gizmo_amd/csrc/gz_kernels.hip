@@ -17,8 +17,8 @@ template __global__ void k_build_ell<true>(int, const int *, const int *, const 
                                            const double *, const double *, const uint32_t *, GridView, int *, long, int, int *, int *);
 
 #define GZ_INST_LANES(KERN, R, BOXES)                                                                                           \
-    template __global__ void k_gradients<KERN, R, BOXES>(DevParams, int, const int *, const double *, const double *,           \
-                                                         const double *, const double *, const GradRec<R> *, const double *, const double *,    \
+    template __global__ void k_gradients<KERN, R, BOXES>(DevParams, int, const int *, const double *, const GradLaneRec<R> *,   \
+                                                         const double *, const double *,                                         \
                                                          long, const int *, long, const int *, double *, double *, double *,    \
                                                          BoxTable);                                                              \
     template __global__ void k_force<KERN, R, BOXES, false>(DevParams, Gam<R>, ForceView, const Cell<R> *, ForceRows, BoxTable);
@@ -66,13 +66,19 @@ GZ_INST(6, double)
 GZ_INST_STATS(3, double)
 GZ_INST_STATS(6, double)
 template __global__ void k_riemann_probe<double>(int, Gam<double>, long, const double *, double *, unsigned *);
-template __global__ void k_pack_grad<double>(long, const double *, const double *, const double *, const double *, const double *,
+template __global__ void k_pack_grad<double, GradRec<double>>(long, const double *, const double *, const double *, const double *, const double *,
                                              const double *, const double *, GradRec<double> *, const double *, const double *,
                                              const double *, double, BoxTable);
+template __global__ void k_pack_grad<double, GradPosRec>(long, const double *, const double *, const double *, const double *, const double *,
+                                             const double *, const double *, GradPosRec *, const double *, const double *,
+                                             const double *, double, BoxTable);
 template __global__ void k_pack_force<double>(double, ForceView, Cell<double> *, int *, double, BoxTable);
-template __global__ void k_pack_grad_list<double>(int, const int *, const int *, long, const int *, const double *, const double *,
+template __global__ void k_pack_grad_list<double, GradRec<double>>(int, const int *, const int *, long, const int *, const double *, const double *,
                                                const double *, const double *, const double *, const double *, const double *,
                                                GradRec<double> *, const double *, const double *, const double *, double, BoxTable);
+template __global__ void k_pack_grad_list<double, GradPosRec>(int, const int *, const int *, long, const int *, const double *, const double *,
+                                               const double *, const double *, const double *, const double *, const double *,
+                                               GradPosRec *, const double *, const double *, const double *, double, BoxTable);
 template __global__ void k_pack_force_list<double>(int, const int *, const int *, long, const int *, double, ForceView, Cell<double> *,
                                                 int *, double, BoxTable);
 #undef GZ_INST

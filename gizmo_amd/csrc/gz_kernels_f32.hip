@@ -12,8 +12,8 @@ namespace gz {
 // ---------------------------------------------------------------------------------------
 
 #define GZ_INST_LANES(KERN, R, BOXES)                                                                                           \
-    template __global__ void k_gradients<KERN, R, BOXES>(DevParams, int, const int *, const double *, const double *,           \
-                                                         const double *, const double *, const GradRec<R> *, const double *, const double *,    \
+    template __global__ void k_gradients<KERN, R, BOXES>(DevParams, int, const int *, const double *, const GradLaneRec<R> *,   \
+                                                         const double *, const double *,                                         \
                                                          long, const int *, long, const int *, double *, double *, double *,    \
                                                          BoxTable);                                                              \
     template __global__ void k_force<KERN, R, BOXES, false>(DevParams, Gam<R>, ForceView, const Cell<R> *, ForceRows, BoxTable);
@@ -61,11 +61,11 @@ GZ_INST(6, float)
 GZ_INST_STATS(3, float)
 GZ_INST_STATS(6, float)
 template __global__ void k_riemann_probe<float>(int, Gam<float>, long, const double *, double *, unsigned *);
-template __global__ void k_pack_grad<float>(long, const double *, const double *, const double *, const double *, const double *,
+template __global__ void k_pack_grad<float, GradRec<float>>(long, const double *, const double *, const double *, const double *, const double *,
                                              const double *, const double *, GradRec<float> *, const double *, const double *,
                                              const double *, double, BoxTable);
 template __global__ void k_pack_force<float>(double, ForceView, Cell<float> *, int *, double, BoxTable);
-template __global__ void k_pack_grad_list<float>(int, const int *, const int *, long, const int *, const double *, const double *,
+template __global__ void k_pack_grad_list<float, GradRec<float>>(int, const int *, const int *, long, const int *, const double *, const double *,
                                                const double *, const double *, const double *, const double *, const double *,
                                                GradRec<float> *, const double *, const double *, const double *, double, BoxTable);
 template __global__ void k_pack_force_list<float>(int, const int *, const int *, long, const int *, double, ForceView, Cell<float> *,

@@ -1009,28 +1009,25 @@ __device__ __forceinline__ GradRec<R> make_grad_rec(long j, const GradSrc &s, co
 }
 
 // the gradient record of particle j
-template <typename R>
-__device__ __forceinline__ void pack_grad_one(long j, const double *__restrict__ H, const double *__restrict__ M,
-                                              const double *__restrict__ RHO, const double *__restrict__ PR,
-                                              const double *__restrict__ VX, const double *__restrict__ VY,
-                                              const double *__restrict__ VZ, GradRec<R> *__restrict__ rec,
-                                              const double *__restrict__ X, const double *__restrict__ Y,
-                                              const double *__restrict__ Z, double box, const BoxTable &bt)
+template <typename R, typename Rec>
+__device__ __forceinline__ void pack_grad_one(long j, const GradSrc &s, Rec *__restrict__ rec, const double *__restrict__ X,
+                                              const double *__restrict__ Y, const double *__restrict__ Z, const BoxTable &bt)
 {
-    rec[j] = make_grad_rec<R>(j, GradSrc{H, M, RHO, PR, VX, VY, VZ, box}, X, Y, Z, bt);
+    if constexpr (std::is_same<Rec, GradRec<R>>::value) rec[j] = make_grad_rec<R>(j, s, X, Y, Z, bt);
+    else rec[j] = GradPosRec{s.H[j], s.M[j], s.RHO[j], s.PR[j], s.VX[j], s.VY[j], s.VZ[j], X[j], Y[j], Z[j]};
 }
 
 // every record (passes over many rows)
-template <typename R>
+template <typename R, typename Rec>
 __global__ void k_pack_grad(long n, const double *__restrict__ H, const double *__restrict__ M,
                             const double *__restrict__ RHO, const double *__restrict__ PR, const double *__restrict__ VX,
-                            const double *__restrict__ VY, const double *__restrict__ VZ, GradRec<R> *__restrict__ rec,
+                            const double *__restrict__ VY, const double *__restrict__ VZ, Rec *__restrict__ rec,
                             const double *__restrict__ X, const double *__restrict__ Y, const double *__restrict__ Z, double box,
                             BoxTable bt)
 {
     const long j = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (j >= n) return;
-    pack_grad_one<R>(j, H, M, RHO, PR, VX, VY, VZ, rec, X, Y, Z, box, bt);
+    pack_grad_one<R>(j, GradSrc{H, M, RHO, PR, VX, VY, VZ, box}, rec, X, Y, Z, bt);
 }
 
 // the force record of particle j (effective_soundspeed, src/declarations/cell_data.h:703-712)
@@ -1077,13 +1074,13 @@ __global__ void k_pack_force(double gamma, ForceView F, Cell<R> *__restrict__ re
 
 // Few rows: the records of the rows and of their list entries only, one wavefront per row
 // (a record shared by several rows is written several times with the same bytes)
-template <typename R>
+template <typename R, typename Rec>
 __global__ void __launch_bounds__(64) k_pack_grad_list(int nrows, const int *__restrict__ act, const int *__restrict__ ell, long ld,
                                                        const int *__restrict__ cnt, const double *__restrict__ H,
                                                        const double *__restrict__ M, const double *__restrict__ RHO,
                                                        const double *__restrict__ PR, const double *__restrict__ VX,
                                                        const double *__restrict__ VY, const double *__restrict__ VZ,
-                                                       GradRec<R> *__restrict__ rec, const double *__restrict__ X,
+                                                       Rec *__restrict__ rec, const double *__restrict__ X,
                                                        const double *__restrict__ Y, const double *__restrict__ Z, double box,
                                                        BoxTable bt)
 {
@@ -1092,7 +1089,7 @@ __global__ void __launch_bounds__(64) k_pack_grad_list(int nrows, const int *__r
     const int c = cnt[r];
     for (int q = threadIdx.x; q <= c; q += 64) {
         const int j = q == 0 ? act[r] : ell[ell_at(ld, r, q - 1)];
-        pack_grad_one<R>(j, H, M, RHO, PR, VX, VY, VZ, rec, X, Y, Z, box, bt);
+        pack_grad_one<R>(j, GradSrc{H, M, RHO, PR, VX, VY, VZ, box}, rec, X, Y, Z, bt);
     }
 }
 
@@ -1117,8 +1114,8 @@ __global__ void __launch_bounds__(64) k_pack_force_list(int nrows, const int *__
 // (:1077-1130), fused per active particle
 // ---------------------------------------------------------------------------------------
 // construct_gradient (NV_T^-1 times the sums) and the limiter block of one particle
-template <typename R>
-__device__ inline void gradients_tail(const GradRec<R> &I, bool enabled, const R (&G)[3][5], const R (&mx)[5], const R (&mn)[5],
+template <typename R, typename Rec>
+__device__ inline void gradients_tail(const Rec &I, bool enabled, const R (&G)[3][5], const R (&mx)[5], const R (&mn)[5],
                                       R maxd, const double *__restrict__ T, const double *__restrict__ CN, long n, int i,
                                       double *__restrict__ GR, double *__restrict__ GP, double *__restrict__ GV)
 {
@@ -1148,19 +1145,35 @@ __device__ inline void gradients_tail(const GradRec<R> &I, bool enabled, const R
     }
 }
 
-// four waves per SIMD (the FP64 form then fits 128 registers: 2.18 -> 1.99 ms on a 2M-row pass)
+// 16 bytes from src to LDS at lds + 16 x lane; complete after wait_staged
+__device__ __forceinline__ void lds_load16(const char *src, unsigned char *lds)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
+}
+__device__ __forceinline__ void wait_staged() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// One lane per row, an entry of each row's list at a time.  A lane that reads its own partner's record
+// touches a cache line per lane with each of its seven loads; instead the wavefront loads the 64
+// records piece by piece (16 bytes a lane, so a record is one line for its four or five
+// lanes) straight into LDS, those of the next entry while this one is added.  2M rows FP64 1.86 -> 1.13 ms, FP32 1.68
+// -> 1.07.  Rows sorted by list length, over 2048 rows as the force pass has them or over the workgroup's
+// 256: 1.74 and 1.13 ms, 4M lognormal rows 4.48 and 3.65 against 3.85, so they stay in order.
 template <int KERN, typename R, bool BOXES>
-__global__ void __launch_bounds__(256, 4) k_gradients(DevParams P, int nrows, const int *__restrict__ act, const double *__restrict__ X,
-                                                   const double *__restrict__ Y, const double *__restrict__ Z,
-                                                   const double *__restrict__ H, const GradRec<R> *__restrict__ rec, const double *__restrict__ T,
+__global__ void __launch_bounds__(256, 4) k_gradients(DevParams P, int nrows, const int *__restrict__ act, const double *__restrict__ H,
+                                                   const GradLaneRec<R> *__restrict__ rec, const double *__restrict__ T,
                                                    const double *__restrict__ CN, long n, const int *__restrict__ ell, long ld,
                                                    const int *__restrict__ cnt, double *__restrict__ GR, double *__restrict__ GP,
                                                    double *__restrict__ GV, BoxTable bt)
 {
+    using Rec = GradLaneRec<R>;
+    constexpr int kPieces = (int)sizeof(Rec) / 16;
+    static_assert(sizeof(Rec) % 16 == 0, "whole pieces");
+    __shared__ __align__(16) unsigned char staged[4][2][64 * sizeof(Rec)];
+    const int lane = threadIdx.x & 63;
     const int r = (int)(xcd_block() * blockDim.x + threadIdx.x);
-    if (r >= nrows) return;
-    const int i = act[r];
-    if (BOXES) {
+    const bool row = r < nrows;
+    const int i = row ? act[r] : 0;
+    if (BOXES && row) {
         GridView g{};
         resolve_box(bt, i, P, g);
     }
@@ -1169,50 +1182,78 @@ __global__ void __launch_bounds__(256, 4) k_gradients(DevParams P, int nrows, co
     R mx[5], mn[5];
     for (int b = 0; b < 5; b++) { mx[b] = 0; mn[b] = 0; }
     R maxd = 0;
-    const GradRec<R> I = rec[i];
-    const bool enabled = (I.m > 0 && I.rho > 0);
+    const Rec I = rec[i];
+    const bool enabled = row && I.m > 0 && I.rho > 0;
     const R hi = I.h;
-    if (enabled) {
-        const double xi = X[i], yi = Y[i], zi = Z[i];
-        // the row's radius in FP64 (the kernel's edge factor, pair_kernel)
-        const double hid = std::is_same<R, double>::value ? (double)hi : H[i];
-        const double h2i = hid * hid;
-        const int c = cnt[r];
-        for (int q = 0; q < c; q++) {
-            const int j = ell[ell_at(ld, r, q)];
-            const GradRec<R> J = rec[j];
-            if (!(J.m > 0) || !(J.rho > 0) || !(J.h > 0)) continue;
-            R dp[3];
-            record_dp<R>(P, I, J, xi, yi, zi, X, Y, Z, j, dp[0], dp[1], dp[2]);
-            const R r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
-            if (r2 <= 0) continue;
-            const double r2d = pair_r2d<R>(dp[0], dp[1], dp[2], r2);
-            if ((r2d >= h2i) && (r2d >= (double)J.h * (double)J.h)) continue;
-            const R rr = sqrt(r2);
-            const double rd = std::is_same<R, double>::value ? 0.0 : sqrt(r2d);
-            const bool inside = std::is_same<R, double>::value ? (rr < hi) : (rd < hid);
-            R wk = 0, dwk = 0;
-            pair_kernel<KERN, -1, R>(rr, rd, hid, wk, dwk);
-            if (rr > maxd) maxd = rr;
-            R d[5];
-            d[0] = (R)(J.rho - I.rho);
-            d[1] = (R)(J.p - I.p);
-            d[2] = (R)(J.v0 - I.v0);
-            d[3] = (R)(J.v1 - I.v1);
-            d[4] = (R)(J.v2 - I.v2);
-            for (int b = 0; b < 5; b++) {
-                if (d[b] < mn[b]) mn[b] = d[b];
-                else if (d[b] > mx[b]) mx[b] = d[b];
-            }
-            if (inside) {
-                for (int kk = 0; kk < 3; kk++) {
-                    const R w = -wk * dp[kk];
-                    for (int b = 0; b < 5; b++) G[kk][b] += rounded(w * d[b]);
-                }
+    // the row's radius in FP64 (the kernel's edge factor, pair_kernel)
+    const double hid = std::is_same<R, double>::value ? (double)hi : H[i];
+    const double h2i = hid * hid;
+    const double inv_box = 1.0 / P.box;
+    const int c = enabled ? cnt[r] : 0;
+    int cmax = c;
+    for (int o = 32; o > 0; o >>= 1) cmax = max(cmax, __shfl_xor(cmax, o, 64));
+    unsigned char *const area = staged[threadIdx.x >> 6][0];
+    // the records of the lanes' j (a lane without an entry: any record) into area + at
+    auto stage = [&](int j, int at) {
+        // the reads of the area's last contents are done
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int k = 0; k < kPieces; k++) {
+            const int piece = k * 64 + lane, owner = piece / kPieces;
+            const int jo = __shfl(j, owner, 64);
+            lds_load16((const char *)rec + (size_t)(unsigned)jo * sizeof(Rec) + (piece - owner * kPieces) * 16, area + at + k * 1024);
+        }
+    };
+    int jn = 0;
+    if (cmax > 0) {
+        stage(c > 0 ? ell[ell_at(ld, r, 0)] : i, 0);
+        jn = c > 1 ? ell[ell_at(ld, r, 1)] : i;
+    }
+    for (int q = 0; q < cmax; q++) {
+        const int at = (q & 1) * 64 * (int)sizeof(Rec);
+        wait_staged();
+        if (q + 1 < cmax) {
+            stage(jn, 64 * (int)sizeof(Rec) - at);
+            jn = q + 2 < c ? ell[ell_at(ld, r, q + 2)] : i;
+        }
+        const Rec &J = *(const Rec *)(area + at + lane * (int)sizeof(Rec));
+        if (q >= c || !(J.m > 0) || !(J.rho > 0) || !(J.h > 0)) continue;
+        R dp[3];
+        if constexpr (std::is_same<R, float>::value) {
+            fine_dp(I.fp, J.fp, (float)(P.box * (1.0 / 1024.0)), dp[0], dp[1], dp[2]);
+        } else {
+            dp[0] = wrap_near(I.x - J.x, P.box, inv_box);
+            dp[1] = wrap_near(I.y - J.y, P.box, inv_box);
+            dp[2] = wrap_near(I.z - J.z, P.box, inv_box);
+        }
+        const R r2 = dp[0] * dp[0] + dp[1] * dp[1] + dp[2] * dp[2];
+        if (r2 <= 0) continue;
+        const double r2d = pair_r2d<R>(dp[0], dp[1], dp[2], r2);
+        if ((r2d >= h2i) && (r2d >= (double)J.h * (double)J.h)) continue;
+        const R rr = sqrt(r2);
+        const double rd = std::is_same<R, double>::value ? 0.0 : sqrt(r2d);
+        const bool inside = std::is_same<R, double>::value ? (rr < hi) : (rd < hid);
+        R wk = 0, dwk = 0;
+        pair_kernel<KERN, -1, R>(rr, rd, hid, wk, dwk);
+        if (rr > maxd) maxd = rr;
+        R d[5];
+        d[0] = (R)(J.rho - I.rho);
+        d[1] = (R)(J.p - I.p);
+        d[2] = (R)(J.v0 - I.v0);
+        d[3] = (R)(J.v1 - I.v1);
+        d[4] = (R)(J.v2 - I.v2);
+        for (int b = 0; b < 5; b++) {
+            if (d[b] < mn[b]) mn[b] = d[b];
+            else if (d[b] > mx[b]) mx[b] = d[b];
+        }
+        if (inside) {
+            for (int kk = 0; kk < 3; kk++) {
+                const R w = -wk * dp[kk];
+                for (int b = 0; b < 5; b++) G[kk][b] += rounded(w * d[b]);
             }
         }
     }
-    gradients_tail<R>(I, enabled, G, mx, mn, maxd, T, CN, n, i, GR, GP, GV);
+    if (row) gradients_tail<R>(I, enabled, G, mx, mn, maxd, T, CN, n, i, GR, GP, GV);
 }
 
 // Running sum of a conserved flux total.  FP32: Neumaier-compensated (the lost low bits of each
@@ -1291,10 +1332,6 @@ __device__ inline void force_tail(const DevParams &P, const ForceView &F, int i,
 // would touch one cache line per lane and instruction).  Every lane of the wavefront calls it;
 // want: the lane's j is to be loaded.  The caller waits for the loads (wait_staged) before it
 // reads them, and has read what it needs of the area's last contents.
-__device__ __forceinline__ void lds_load16(const char *src, unsigned char *lds)
-{
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
-}
 template <typename R, int K>
 __device__ __forceinline__ void stage_quad_row(const Cell<R> *__restrict__ rec, int j, int want, unsigned char *wave_lds)
 {
@@ -1331,7 +1368,6 @@ __device__ __forceinline__ void stage_records(const Cell<R> *__restrict__ rec, i
         stage_quad_half<R, 1>(rec, j, want, wave_lds);
     }
 }
-__device__ __forceinline__ void wait_staged() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // the difference of a pair's positions from the staged record of j (FP32 form) or the position
 // arrays (FP64 form)
