@@ -79,6 +79,7 @@ struct gz_batch {
     double *it_h = nullptr, *it_hb = nullptr, *it_l = nullptr, *it_r = nullptr, *it_cn = nullptr;
     int *it_ci = nullptr, *it_it = nullptr;
     void *rec_grad = nullptr, *rec_force = nullptr;
+    int *rl_a = nullptr, *rl_b = nullptr;  // rows still iterating in density rounds: the coming round's, the next one's
     void *flux = nullptr;  // the force pass's stored fluxes
     size_t flux_bytes = 0;
     int *ell = nullptr, *cnt = nullptr;
@@ -233,6 +234,7 @@ int alloc_all(gz_batch *b)
     BCHK(balloc(b, &b->key, n)); BCHK(balloc(b, &b->key64, n)); BCHK(balloc(b, &b->key64b, n));
     BCHK(balloc(b, (char **)&b->rec_grad, n * sizeof(GradRec<double>)));
     BCHK(balloc(b, (char **)&b->rec_force, n * sizeof(Cell<double>)));
+    BCHK(balloc(b, &b->rl_a, n)); BCHK(balloc(b, &b->rl_b, n));
     // room for the force pass's stored fluxes of every row of the batch
     b->flux_bytes = b->par.precision == GZ_FP64 ? force_plan<double>(b->cap, ~(size_t)0).bytes : force_plan<float>(b->cap, ~(size_t)0).bytes;
     BCHK(balloc(b, (char **)&b->flux, b->flux_bytes));
@@ -260,7 +262,7 @@ void free_all(gz_batch *c)
                   &c->iscan, &c->rank, &c->lim, &c->counters, &c->ell, &c->cstart, &c->cend};
     for (auto p : i1) bfree(*p);
     bfree(c->TIB); bfree(c->DTS); bfree(c->ACT); bfree(c->need); bfree(c->sel); bfree(c->due);
-    bfree(c->key); bfree(c->key64); bfree(c->key64b); bfree(c->rec_grad); bfree(c->rec_force); bfree(c->flux); bfree(c->tab);
+    bfree(c->key); bfree(c->key64); bfree(c->key64b); bfree(c->rl_a); bfree(c->rl_b); bfree(c->rec_grad); bfree(c->rec_force); bfree(c->flux); bfree(c->tab);
     bfree(c->hist); bfree(c->slot); bfree(c->u64);
     bfree(c->tmp);
     {
@@ -520,9 +522,22 @@ int density(gz_batch *b)
     DensityIter it{b->it_h, b->it_hb, b->it_l, b->it_r, b->it_cn, b->it_ci, b->it_it};
     DensityOut out{b->cap, b->H, b->NN, b->DRK, b->DIVV, b->RHO, b->PR, b->T, b->FW, b->CN, b->FCE};
     int iters = 0;
+    const bool many = na > b->few_rows;
+    int remaining = na;
     while (true) {
         BHIP(hipMemsetAsync(b->counters, 0, 3 * sizeof(int), b->stream));
-        if (na > b->few_rows) {
+        // the later rounds' few rows: one workgroup each from the list of rows still iterating
+        const int *rows = many && iters > 0 && density_by_row(remaining, na) ? b->rl_a : nullptr;
+        const int nround = rows ? remaining : na;
+        if (rows) {
+            if (remaining <= b->few_rows)
+                k_density_rows<KERN, R, kRowThreads><<<xcd_grid(nround), kRowThreads, 0, b->stream>>>(b->dp, gview(b), na, b->act, b->need, b->key, b->X, b->Y,
+                                                                             b->Z, b->VX, b->VY, b->VZ, b->M, b->it_h, b->dacc, bt, nullptr,
+                                                                             rows, nround);
+            else
+                k_density_rows<KERN, R, 64><<<xcd_grid(nround), 64, 0, b->stream>>>(b->dp, gview(b), na, b->act, b->need, b->key, b->X, b->Y, b->Z, b->VX,
+                                                                           b->VY, b->VZ, b->M, b->it_h, b->dacc, bt, nullptr, rows, nround);
+        } else if (many) {
             BCHK(build_groups(b));
             auto cells_kernel = b->dp.fd4alpha > 0 ? k_density_cells<KERN, R, true> : k_density_cells<KERN, R, false>;
             cells_kernel<<<dim3(xcd_grid(b->grp.ngroups), walk_parts(na, b->grp.ngroups)), 64, 0, b->stream>>>(b->dp, gview(b), b->grp.view(bt), b->act, b->need, b->X, b->Y,
@@ -531,12 +546,15 @@ int density(gz_batch *b)
             k_density_rows<KERN, R, kRowThreads><<<xcd_grid(na), kRowThreads, 0, b->stream>>>(b->dp, gview(b), na, b->act, b->need, b->key, b->X, b->Y, b->Z,
                                                                          b->VX, b->VY, b->VZ, b->M, b->it_h, b->dacc, bt);
         }
-        k_density_after<<<nb(na), kB, 0, b->stream>>>(b->dp, na, b->act, b->need, b->dacc, b->M, b->U, 0, it, out, b->counters + 0,
-                                                      b->counters + 1, b->counters + 2, b->u64 + 1, bt);
+        k_density_after<<<nb(nround), kB, 0, b->stream>>>(b->dp, na, b->act, b->need, b->dacc, b->M, b->U, 0, it, out, b->counters + 0,
+                                                          b->counters + 1, b->counters + 2, b->u64 + 1, bt, 0, nullptr, nullptr, rows, nround,
+                                                          many ? b->rl_b : nullptr);
         BHIP(hipGetLastError());
         BCHK(read_back(b, false));
         iters++;
-        const int remaining = b->hcounters[0], rebuild = b->hcounters[1], e = b->hcounters[2];
+        std::swap(b->rl_a, b->rl_b);
+        remaining = b->hcounters[0];
+        const int rebuild = b->hcounters[1], e = b->hcounters[2];
         if (e == GZ_STOP_MAXITER) return fail(b, e, "density(): kernel radius iteration did not converge in %d rounds", kMaxIter);
         if (e == GZ_STOP_BRACKET) return fail(b, e, "density(): empty radius bracket (Right==0 && Left==0)");
         if (e) return fail(b, e, "density(): device stop code %d", e);

@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from gizmo_amd import ics
+from gizmo_amd.batch import Batch
 from gizmo_amd.hydro import GZ_FP32_MIXED, GZ_FP64, Hydro
 
 pytestmark = pytest.mark.gpu
@@ -76,3 +77,33 @@ def test_groups_of_many_levels_equal_row_kernels(name, active, precision):
     for k in FIELDS:
         same = a[k].view(np.int64 if a[k].dtype == np.float64 else a[k].dtype) == b[k].view(np.int64 if b[k].dtype == np.float64 else b[k].dtype)
         assert np.isfinite(a[k]).all() and same.all(), (k, int((~same).sum()), same.size)
+
+
+INTEG = dict(courant_fac=0.2, err_tol_int_accuracy=0.02, max_size_timestep=0.01, min_size_timestep=0.0, time_begin=0.0, time_max=1.0,
+             min_egy_spec=0.0)
+
+
+@pytest.mark.parametrize("precision", [GZ_FP64, GZ_FP32_MIXED], ids=["fp64", "mixed"])
+def test_batch_rounds_by_row_equal_cell_walks(precision):
+    """A batch whose rows need different numbers of density rounds: the later rounds' few rows by row
+    (one wavefront, four wavefronts each) against the pass that takes every round by row."""
+    rng = np.random.Generator(np.random.Philox(11))
+    boxes = [ics.lattice_box(s, 30 + s, kernel=6, des_num_ngb=64.0, mach_sigma=0.5) for s in (12, 17)]
+    for ic in boxes:
+        far = rng.random(len(ic["h"])) < 0.3  # radii that the rounds have to bring back
+        ic["h"] = np.where(far, ic["h"] * rng.uniform(0.7, 1.3, len(ic["h"])), ic["h"])
+    out = {}
+    for few_rows in (10 ** 9, 0, 1500):
+        b = Batch(dict(boxes[0]["params"]), sum(len(ic["mass"]) for ic in boxes), 2, precision)
+        b.set_option("few_rows", few_rows)
+        ids = [b.add({k: ic[k] for k in ("pos", "vel", "mass", "u", "h")}, ic["params"], INTEG) for ic in boxes]
+        print(f"batch rounds: few_rows={few_rows} precision={precision}", flush=True)
+        b.begin()
+        for _ in range(3):
+            b.step()
+        out[few_rows] = [b.store(i, ("h", "rho", "numngb", "accel", "dtu")) for i in ids]
+        b.close()
+    for few_rows in (0, 1500):
+        for x, y in zip(out[few_rows], out[10 ** 9]):
+            for k in x:
+                assert np.isfinite(x[k]).all() and np.array_equal(x[k], y[k]), (few_rows, k)
