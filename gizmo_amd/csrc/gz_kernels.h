@@ -261,7 +261,6 @@ __global__ void k_scatter_ll(long n, const int *perm, const long long *in, long 
 
 __global__ void k_morton(long n, const double *pos, double box, uint32_t *key, int *val);
 __global__ void k_morton_soa(long n, const double *X, const double *Y, const double *Z, double box, uint32_t *key, int *val);
-__global__ void k_permute_cols(long n, int width, const int *order, const unsigned long long *in, unsigned long long *out);
 __global__ void k_permute_int(long n, const int *order, const int *in, int *out);
 __global__ void k_permute_u8(long n, const int *order, const uint8_t *in, uint8_t *out);
 constexpr int kPermCols = 16;
@@ -271,6 +270,7 @@ struct PermCols {
     int ncol;
 };
 __global__ void k_permute_many(long n, const int *order, PermCols P);
+__global__ void k_copy_many(long n, PermCols P);
 __global__ void k_gather(long n, int width, const int *perm, const double *in, double *out, int soa);
 __global__ void k_gather_int(long n, const int *perm, const int *in, int *out);
 __global__ void k_gather_u8(long n, const int *perm, const uint8_t *in, uint8_t *out);
@@ -401,7 +401,7 @@ __global__ void k_force_rows(DevParams P, Gam<R> G, int nrows, const int *act, F
 struct ForceRows {
     int nrows;
     const int *act;              // the rows' particles
-    const int *ell;              // symmetric list, column-major with leading dimension ld
+    const int *ell;              // symmetric list (ell_at) with leading dimension ld
     long ld;
     const int *cnt;              // list lengths
     const uint8_t *active;       // active flags (nullptr: every particle active)

@@ -7,9 +7,8 @@
 // the 27 neighbour-cell ranges of a cell, sorted by start, visit candidates in ascending
 // device index: the canonical summation order, shared with the CPU oracle.
 //
-// Neighbour lists are ELLPACK: entry q of row r sits at ell[ell_at(ld, r, q)], column-major
-// (the 64 rows of a wave read entry q from four 64-byte lines).  One lane per active particle;
-// wave64.
+// Neighbour lists are ELLPACK: entry q of row r sits at ell[ell_at(ld, r, q)], four entries of a
+// row side by side.  Wave64.
 #pragma once
 #include <type_traits>
 #include "gz_kernels.h"
@@ -69,16 +68,6 @@ __global__ void k_morton_soa(long n, const double *__restrict__ X, const double 
     val[i] = (int)i;
 }
 
-// reorder width columns of 8-byte values (SoA, column stride n): out[c*n + s] = in[c*n + order[s]]
-__global__ void k_permute_cols(long n, int width, const int *__restrict__ order, const unsigned long long *__restrict__ in,
-                               unsigned long long *__restrict__ out)
-{
-    long s = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const long u = order[s];
-    for (int c = 0; c < width; c++) out[(size_t)c * n + s] = in[(size_t)c * n + u];
-}
-
 __global__ void k_permute_int(long n, const int *__restrict__ order, const int *__restrict__ in, int *__restrict__ out)
 {
     long s = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -104,6 +93,20 @@ __global__ void __launch_bounds__(256) k_permute_many(long n, const int *__restr
 #pragma unroll
     for (int c = 0; c < kPermCols; c++)
         if (c < P.ncol) v[c] = P.in[c][u];
+#pragma unroll
+    for (int c = 0; c < kPermCols; c++)
+        if (c < P.ncol) P.out[c][s] = v[c];
+}
+
+// the columns copied, in order (what k_permute_many left in a scratch area, back to its place)
+__global__ void __launch_bounds__(256) k_copy_many(long n, PermCols P)
+{
+    const long s = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (s >= n) return;
+    unsigned long long v[kPermCols];
+#pragma unroll
+    for (int c = 0; c < kPermCols; c++)
+        if (c < P.ncol) v[c] = P.in[c][s];
 #pragma unroll
     for (int c = 0; c < kPermCols; c++)
         if (c < P.ncol) P.out[c][s] = v[c];
