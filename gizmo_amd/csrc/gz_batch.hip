@@ -79,7 +79,7 @@ struct gz_batch {
     double *it_h = nullptr, *it_hb = nullptr, *it_l = nullptr, *it_r = nullptr, *it_cn = nullptr;
     int *it_ci = nullptr, *it_it = nullptr;
     void *rec_grad = nullptr, *rec_force = nullptr;
-    int *rl_a = nullptr, *rl_b = nullptr;  // rows still iterating in density rounds: the coming round's, the next one's
+    int *rl_a = nullptr, *rl_b = nullptr;  // rows still iterating in density rounds (in key64, key64b): the coming round's, the next one's
     void *flux = nullptr;  // the force pass's stored fluxes
     size_t flux_bytes = 0;
     int *ell = nullptr, *cnt = nullptr;
@@ -234,7 +234,8 @@ int alloc_all(gz_batch *b)
     BCHK(balloc(b, &b->key, n)); BCHK(balloc(b, &b->key64, n)); BCHK(balloc(b, &b->key64b, n));
     BCHK(balloc(b, (char **)&b->rec_grad, n * sizeof(GradRec<double>)));
     BCHK(balloc(b, (char **)&b->rec_force, n * sizeof(Cell<double>)));
-    BCHK(balloc(b, &b->rl_a, n)); BCHK(balloc(b, &b->rl_b, n));
+    // (the sort keys of an order are free during a pass)
+    b->rl_a = (int *)b->key64; b->rl_b = (int *)b->key64b;
     // room for the force pass's stored fluxes of every row of the batch
     b->flux_bytes = b->par.precision == GZ_FP64 ? force_plan<double>(b->cap, ~(size_t)0).bytes : force_plan<float>(b->cap, ~(size_t)0).bytes;
     BCHK(balloc(b, (char **)&b->flux, b->flux_bytes));
@@ -262,7 +263,7 @@ void free_all(gz_batch *c)
                   &c->iscan, &c->rank, &c->lim, &c->counters, &c->ell, &c->cstart, &c->cend};
     for (auto p : i1) bfree(*p);
     bfree(c->TIB); bfree(c->DTS); bfree(c->ACT); bfree(c->need); bfree(c->sel); bfree(c->due);
-    bfree(c->key); bfree(c->key64); bfree(c->key64b); bfree(c->rl_a); bfree(c->rl_b); bfree(c->rec_grad); bfree(c->rec_force); bfree(c->flux); bfree(c->tab);
+    bfree(c->key); bfree(c->key64); bfree(c->key64b); bfree(c->rec_grad); bfree(c->rec_force); bfree(c->flux); bfree(c->tab);
     bfree(c->hist); bfree(c->slot); bfree(c->u64);
     bfree(c->tmp);
     {
