@@ -297,7 +297,7 @@ __global__ void k_block_boxes(int n, const double *X, const double *Y, const dou
 __global__ void k_build_sym_groups(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
                                    const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
 // cells of at most this many rows on average: one candidate per lane (k_build_sym_groups), whose
-// time grows with the rows of a cell (4 of 31: 218 us against 524 with a row per lane) where the
+// time grows with the rows of a cell (4 of 31: 183 us against 524 with a row per lane) where the
 // other's does not
 constexpr int kSymFewRows = 16;
 // workgroups along y of the cell walks: enough for the rows of a cell, 64 each, when the cells hold
@@ -417,7 +417,7 @@ struct ForceRows {
     int count_rare;              // count the rows with a face past the Riemann ladder's common case into err[12]
 };
 
-// Four lanes per row, kForceRowsPerBlock rows per workgroup at a time, on force_blocks() workgroups.
+// Four lanes per row, kForceRowsPerBlock rows per workgroup at a time, on kForceBlocks workgroups at most.
 // STATS: count the faces' RiemannRung bits into F.rungs.
 template <int KERN, typename R, bool BOXES, bool STATS = false>
 __global__ void k_force(DevParams P, Gam<R> G, ForceView F, const Cell<R> *rec, ForceRows a, BoxTable bt);
@@ -426,7 +426,7 @@ constexpr int kForceRowsPerBlock = 64;
 // neighbours (at most ~90 entries) in one segment, and a queue that leaves room for the LDS of
 // two workgroups on a CU
 constexpr int kForceSegment = 96;
-// workgroups of the fixed grid: two (FP64) or three (FP32) per CU of 256, by their LDS and registers
+// workgroups of the fixed grid: two per CU of 256, by their registers (and, FP64, their LDS)
 template <typename R> constexpr int kForceBlocks = 2 * 256;
 // The launch of a pass over nrows rows with at most `room` bytes for the stored fluxes (a segment's
 // entries x rows x 4 per workgroup; the whole grid with whole segments takes up to 100 MB).  Less

@@ -228,8 +228,8 @@ __device__ __forceinline__ void row_stencil_wide(const GridView &g, const WideGr
 // Long walks over many levels.  The cells of a coarse level next to a clump hold up to a tenth of all
 // particles (1M lognormal particles: 100K candidates for the rows of one cell), and one
 // wavefront walks them.  The bounding box and the largest radius of every 64 consecutive particles
-// let a lane drop 64 candidates at once.  Density rounds of 1M lognormal rows FP64 2.5 -> 1.9 ms,
-// of 4M rows FP32 5.7 -> 4.3 ms.
+// let a lane drop 64 candidates at once.  Mean density round of 1M lognormal rows FP64 2.5 -> 1.9 ms, of
+// 4M rows FP32 5.7 -> 4.3 ms (before the rounds collected their partners first, below).
 // ---------------------------------------------------------------------------------------
 #ifdef GZ_DEFINE_COMMON_KERNELS
 __global__ void __launch_bounds__(256) k_block_boxes(int n, const double *__restrict__ X, const double *__restrict__ Y,
@@ -945,6 +945,13 @@ __device__ __forceinline__ void stencil_ranges(CellRanges &cr, const int4 *__res
 // k_build_sym_wide).  They are collected first, sorted, and laid between the group's own ranges,
 // so that the walk meets every candidate in ascending order; more than kMaxCoarse of them are
 // inserted into the finished rows one by one.
+//
+// Bound by its VALU instructions (4M lognormal rows: 63% of the issue rate) and the latency of part B's
+// stencils (3 to 6 levels of dependent table reads).  1M lognormal rows 5.0 -> 1.53 ms, 4M 9.1 -> 6.1: at 8
+// cells a side every pair took the exact test and no block was skipped (217 groups of 37,000
+// candidates took 3 to 6 ms each; 1.93 ms without them), part B's candidates came by four gathers and a
+// key each, not by one packed record loaded a step ahead (1.53 and 6.1, with the row loop's
+// masks in scalar registers 1.86 -> 1.68 of that).
 constexpr int kMaxCoarse = 768;
 // bound on the FP32 test's rounding error, per unit of |x_j|^2 + h_j^2 + 13 (|x_i|^2 <= 12 in cells):
 // a dozen roundings of 2^-24 each of at most twice that
