@@ -299,9 +299,10 @@ __device__ __forceinline__ unsigned long long live_runs(const float4 *__restrict
 constexpr int kLongWalk = 1024;  // candidates from which a walk asks for its live runs first
 
 // The place of this thread's entry among the flagged entries of its workgroup, in thread order
-// (total: the flagged entries of the workgroup).  One barrier for several wavefronts, none for one:
-// smask[TPB / 64] must not be read by another round of the caller before the caller's next
-// barrier (two buffers in turn will do).
+// (total: the flagged entries of the workgroup).  One barrier for several wavefronts, none for one.
+// The masks are read behind it, so a call that takes the same smask[TPB / 64] must lie behind another
+// barrier: one of the caller's own, or that of a call in between which took another buffer (two
+// buffers that turn at every call and at nothing else).
 template <int TPB>
 __device__ __forceinline__ int flagged_rank(bool flag, unsigned long long *smask, int &total)
 {
@@ -476,6 +477,7 @@ __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, i
     const BlockReach reach{(float)xi, (float)yi, (float)zi, 0.0f, 0.0f, 0.0f, (float)h, (float)g.box};
     unsigned long long live = ~0ull;
     int head = 0, fill = 0;  // the partners found and not yet added: list places head .. head + fill - 1
+    int turn = 0;  // the rank buffer of the next walked run (a skipped run has no barrier: it must not turn)
     for (int base = 0, run = 0; base < total || fill > 0; base += TPB, run++) {
         bool walk = base < total;
         if (walk && long_walk) {
@@ -496,7 +498,8 @@ __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, i
                 ok = dp0 * dp0 + dp1 * dp1 + dp2 * dp2 < h2;
             }
             int nok;
-            const int pos = flagged_rank<TPB>(ok, smask[run & 1], nok);
+            const int pos = flagged_rank<TPB>(ok, smask[turn], nok);
+            turn ^= 1;
             if (ok) list[(head + fill + pos) & (2 * TPB - 1)] = j;
             fill += nok;
         }
