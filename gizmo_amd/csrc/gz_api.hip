@@ -549,7 +549,7 @@ int build_grid(gz_context *ctx, double rmax, bool cell_walk, bool need_chmax = f
         ctx->sten_valid = false;
     }
     if (cell_walk && !ctx->sten_valid) {
-        k_cell_stencil<<<nblk(32 * ncell), kBlock, 0, ctx->stream>>>(L, ctx->cstart, ctx->cend, ctx->sten, ctx->nsten);
+        k_cell_stencil<<<stencil_grid(ncell), kBlock, 0, ctx->stream>>>(L, ctx->cstart, ctx->cend, ctx->sten, ctx->nsten);
         HIPCHK(hipGetLastError());
         ctx->sten_valid = true;
     }

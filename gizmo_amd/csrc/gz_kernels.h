@@ -1,12 +1,12 @@
 // gz_kernels.h -- kernel declarations and the small views the kernels take by value.
 #pragma once
 #include "gz_device.h"
+#include "gz_plan.h"
 
 namespace gz {
 
 constexpr int kFineLevel = 10;                 // 1024^3 Morton grid
 constexpr int kFine = 1 << kFineLevel;
-constexpr int kXcds = 8;                       // MI355X: 8 XCDs, each with its own L2
 
 // Workgroups are handed to the XCDs round-robin (workgroup b runs on XCD b % 8).  A grid of
 // 8*q workgroups is remapped so that XCD x processes the contiguous logical range
@@ -24,7 +24,6 @@ __device__ __forceinline__ long xcd_block_dealt()
     const long b = blockIdx.x, l = b / kXcds, q = gridDim.x / kXcds, whole = q / 64 * 64;
     return l < whole ? (l / 64 * kXcds + b % kXcds) * 64 + l % 64 : whole * kXcds + (b % kXcds) * (q - whole) + (l - whole);
 }
-inline unsigned xcd_grid(long nblocks) { return (unsigned)(((nblocks + kXcds - 1) / kXcds) * kXcds); }
 
 // Search over kernel radii that span many grid levels.  Every cell of every level 0..lmax is a
 // contiguous range of the Morton order; `start`/`end` hold each cell's range (level L from

@@ -265,36 +265,37 @@ __global__ void __launch_bounds__(256) k_cell_stencil(int level, const int *__re
                                                       int4 *__restrict__ sten, int *__restrict__ nsten)
 {
     const long ncell = 1L << (3 * level);
-    const long c = (blockIdx.x * (long)blockDim.x + threadIdx.x) >> 5;
-    if (c >= ncell) return;  // whole halves of a wavefront leave: the shuffles stay within one half
     const int lane = threadIdx.x & 31;
     const int nc = 1 << level;
-    const int cx = compact10((uint32_t)c >> 2), cy = compact10((uint32_t)c >> 1), cz = compact10((uint32_t)c);
     const int none = 0x7fffffff;
-    int st = none, en = 0;
-    uint32_t code = 0;
-    if (lane < 27) {
-        const int dx = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
-        const int a = (cx + dx + nc) % nc, b = (cy + dy + nc) % nc, d = (cz + dz + nc) % nc;
-        code = (spread10(a) << 2) | (spread10(b) << 1) | spread10(d);
-        st = cstart[code];
-        en = cend[code];
-        if (en <= st) st = none;
+    // (whole halves of a wavefront run and leave together: the shuffles stay within one half)
+    for (long c = (blockIdx.x * (long)blockDim.x + threadIdx.x) >> 5; c < ncell; c += (gridDim.x * (long)blockDim.x) >> 5) {
+        const int cx = compact10((uint32_t)c >> 2), cy = compact10((uint32_t)c >> 1), cz = compact10((uint32_t)c);
+        int st = none, en = 0;
+        uint32_t code = 0;
+        if (lane < 27) {
+            const int dx = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
+            const int a = (cx + dx + nc) % nc, b = (cy + dy + nc) % nc, d = (cz + dz + nc) % nc;
+            code = (spread10(a) << 2) | (spread10(b) << 1) | spread10(d);
+            st = cstart[code];
+            en = cend[code];
+            if (en <= st) st = none;
+        }
+        if (nc < 3) {
+            // neighbours coincide on such grids: the first lane of each start stays
+            bool dup = false;
+            for (int q = 0; q < 27; q++) dup |= __shfl(st, q, 32) == st && q < lane;
+            if (dup) st = none;
+        }
+        int rank = 0, m = 0;
+        for (int q = 0; q < 27; q++) {
+            const int s = __shfl(st, q, 32);
+            rank += s < st;
+            m += s != none;
+        }
+        if (st != none) sten[c * 27 + rank] = make_int4(st, en, lane, (int)code);
+        if (lane == 0) nsten[c] = m;
     }
-    if (nc < 3) {
-        // neighbours coincide on such grids: the first lane of each start stays
-        bool dup = false;
-        for (int q = 0; q < 27; q++) dup |= __shfl(st, q, 32) == st && q < lane;
-        if (dup) st = none;
-    }
-    int rank = 0, m = 0;
-    for (int q = 0; q < 27; q++) {
-        const int s = __shfl(st, q, 32);
-        rank += s < st;
-        m += s != none;
-    }
-    if (st != none) sten[c * 27 + rank] = make_int4(st, en, lane, (int)code);
-    if (lane == 0) nsten[c] = m;
 }
 #endif
 

@@ -56,3 +56,25 @@ def test_long_walk_with_skipped_runs(precision):
         out[few_rows] = g.store(DENSITY_OUT)
         g.close()
     same_bits(out[0], out[10 ** 9], rows)
+
+
+@BOTH
+def test_grid_of_512_cells_a_side(precision):
+    """Many rows on the second finest grid (radii below box / 512; 134 million cells, whose stencils
+    take as many threads as a launch cannot hold), against the row kernels, which find their cells
+    themselves."""
+    rng = np.random.Generator(np.random.Philox(42))
+    side = 14
+    pos = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3) * 7e-4
+    pos = 0.5 + pos + rng.uniform(-1e-4, 1e-4, pos.shape)
+    n = len(pos)
+    out = {}
+    for few_rows in (0, 10 ** 9):
+        print(f"512 cells a side: n={n} few_rows={few_rows} precision={precision}", flush=True)
+        g = Hydro(params(), n, precision)
+        g.set_option("few_rows", few_rows)
+        g.load(dict(pos=pos, vel=np.sin(900.0 * pos), mass=np.full(n, 1.0 / n), u=np.ones(n), h=np.full(n, 0.0015)))
+        g.density()
+        out[few_rows] = g.store(DENSITY_OUT)
+        g.close()
+    same_bits(out[0], out[10 ** 9])
