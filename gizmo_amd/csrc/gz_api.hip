@@ -1232,6 +1232,7 @@ int force_stage(gz_context *ctx)
                     plan = force_plan<R>(ctx->nact, sums);
                 }
             }
+            if (plan.segment < 1) return fail(ctx, GZ_E_MEMORY, "hydro_force(): no room for the stored fluxes (%ld particles)", ctx->cap);
             const ForceRows a{ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->all_active ? nullptr : ctx->ACT, ctx->TB,
                               ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2, ctx->counters + 4,
                               ctx->sched_valid ? ctx->sched : nullptr, flux, plan.segment, ctx->force_split != 0 && !ctx->rung_stats};

@@ -674,6 +674,7 @@ int gradients_force(gz_batch *b)
         k_pack_force<R><<<nb(b->cap), kB, 0, b->stream>>>(b->par.gamma, F, rf, b->counters + 2, 1.0, bt);
     if (lanes) {
         const ForcePlan plan = force_plan<R>(na, b->flux_bytes);
+        if (plan.segment < 1) return fail(b, GZ_E_MEMORY, "hydro_force(): no room for the stored fluxes (%ld particles)", b->cap);
         const ForceRows a{na, b->act, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV, b->WAKE, b->ACC, b->DTU, b->MSV, b->counters + 2,
                           b->counters + 4, nullptr, b->flux, plan.segment, 0};
         k_force<KERN, R, true><<<plan.blocks, kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);

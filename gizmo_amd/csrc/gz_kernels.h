@@ -420,37 +420,6 @@ struct ForceRows {
 // STATS: count the faces' RiemannRung bits into F.rungs.
 template <int KERN, typename R, bool BOXES, bool STATS = false>
 __global__ void k_force(DevParams P, Gam<R> G, ForceView F, const Cell<R> *rec, ForceRows a, BoxTable bt);
-constexpr int kForceRowsPerBlock = 64;
-// at most this many list entries of a row between two rounds of queued faces: the lists of 64
-// neighbours (at most ~90 entries) in one segment, and a queue that leaves room for the LDS of
-// two workgroups on a CU
-constexpr int kForceSegment = 96;
-// workgroups of the fixed grid: two per CU of 256, by their registers (and, FP64, their LDS)
-template <typename R> constexpr int kForceBlocks = 2 * 256;
-// The launch of a pass over nrows rows with at most `room` bytes for the stored fluxes (a segment's
-// entries x rows x 4 per workgroup; the whole grid with whole segments takes up to 100 MB).  Less
-// room: shorter segments, at least eight entries, and then fewer workgroups.
-struct ForcePlan {
-    int blocks, segment;
-    size_t bytes;
-};
-template <typename R> inline ForcePlan force_plan(long nrows, size_t room)
-{
-    const long nrb = (nrows + kForceRowsPerBlock - 1) / kForceRowsPerBlock;
-    const size_t entry = (size_t)kForceRowsPerBlock * 4 * sizeof(R);
-    long blocks = (long)xcd_grid(nrb < kForceBlocks<R> ? nrb : kForceBlocks<R>);
-    long seg = (long)(room / ((size_t)blocks * entry));
-    if (seg > kForceSegment) seg = kForceSegment;
-    if (seg < 8) {
-        seg = 8;
-        blocks = (long)(room / (seg * entry)) / kXcds * kXcds;
-        if (blocks < kXcds) {
-            blocks = kXcds;
-            seg = (long)(room / (blocks * entry));
-        }
-    }
-    return ForcePlan{(int)blocks, (int)seg, (size_t)blocks * seg * entry};
-}
 // few-row force passes over at most this many rows make their records in the row kernel (its
 // MAKE form holds one wave per SIMD: this many rows of two wavefronts fill the chip once)
 constexpr int kMakeForceRows = 512;

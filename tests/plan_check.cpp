@@ -13,6 +13,12 @@ int main()
             long ncell;
             if (std::scanf("%ld", &ncell) != 1) return 1;
             std::printf("%u\n", gz::stencil_grid(ncell));
+        } else if (!std::strcmp(what, "force32") || !std::strcmp(what, "force64")) {
+            long nrows;
+            size_t room;
+            if (std::scanf("%ld %zu", &nrows, &room) != 2) return 1;
+            const gz::ForcePlan p = what[5] == '3' ? gz::force_plan<float>(nrows, room) : gz::force_plan<double>(nrows, room);
+            std::printf("%d %d %zu\n", p.blocks, p.segment, p.bytes);
         } else {
             return 1;
         }

@@ -31,3 +31,19 @@ def test_stencil_launch_fits_at_every_level(ask):
         assert 1 <= blocks and blocks * 256 < 2 ** 32
         if level <= 8:
             assert blocks == max(1, 8 ** level * 32 // 256)
+
+
+@pytest.mark.parametrize("form,width", [("force32", 4), ("force64", 8)])
+def test_force_plan_of_any_room(ask, form, width):
+    """The stored fluxes' launch keeps within its room, takes whole eights of workgroups, and says
+    segment 0 (with which the kernel would not end: the callers refuse it) exactly where the room
+    does not hold an entry of 64 rows x 4 values for each of eight workgroups."""
+    entry = 64 * 4 * width
+    rooms = [0, 1, entry, 8 * entry - 1, 8 * entry, 8 * entry + 1, 63 * entry, 64 * entry, 100 * entry, 512 * 8 * entry - 1,
+             512 * 8 * entry, 512 * 96 * entry, 2 ** 63]
+    for nrows in (1, 64, 65, 121, 8193, 32768, 10 ** 9):
+        whole = min(-(-nrows // 64), 512)
+        for room, (blocks, segment, size) in zip(rooms, ask([(form, nrows, room) for room in rooms])):
+            assert size <= room and size == blocks * segment * entry
+            assert blocks % 8 == 0 and 8 <= blocks <= -(-whole // 8) * 8 and segment <= 96
+            assert (segment == 0) == (room < 8 * entry), (nrows, room)
