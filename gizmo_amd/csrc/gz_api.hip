@@ -116,6 +116,8 @@ struct gz_context {
     unsigned long long *sched_part = nullptr;
     void *flux = nullptr;     // the force pass's stored fluxes
     size_t flux_bytes = 0;
+    double force_room = -1;     // option "force_room": bytes of that buffer (-1: by the capacity)
+    bool flux_refused = false;  // the device refused it since the last load
     int sched_span = 2048;  // rows per sorted block (0: plain order)
     bool sched_valid = false;
 
@@ -258,7 +260,12 @@ int dalloc(gz_context *ctx, T **p, size_t count)
     if (ctx->pool) return pool_take(ctx, (void **)p, count * sizeof(T));
     if (*p) { hipFree(*p); *p = nullptr; }
     hipError_t e = hipMalloc((void **)p, count * sizeof(T));
-    if (e != hipSuccess) { *p = nullptr; return fail(ctx, GZ_E_MEMORY, "hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e)); }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        // reported here: a later launch check must not find it (the runtime keeps it until it is read)
+        (void)hipGetLastError();
+        return fail(ctx, GZ_E_MEMORY, "hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
+    }
     return 0;
 }
 
@@ -1174,6 +1181,36 @@ int gradients_stage(gz_context *ctx)
     return 0;
 }
 
+// Where the force pass over many rows stores fluxes, and the launch that this room allows: a buffer of
+// the context's own, allocated once for any number of its rows (at most 100 MB, or the bytes of the
+// option "force_room"); what is left of a pool; or the density sums, which are free now.  A buffer that
+// the device refuses is not asked for again until the next load: the density sums serve, with
+// shorter segments (the same sums, bit for bit).
+template <typename R>
+ForcePlan flux_room(gz_context *ctx, void *&flux)
+{
+    size_t room = 0;
+    if (ctx->pool) {
+        const size_t at = (ctx->pool_used + 255) & ~(size_t)255;
+        flux = ctx->pool + at;
+        room = at < ctx->pool_size ? ctx->pool_size - at : 0;
+    } else {
+        const size_t want = ctx->force_room < 0 ? force_plan<R>(ctx->cap, ~(size_t)0).bytes : (size_t)ctx->force_room;
+        if (want > ctx->flux_bytes && !ctx->flux_refused) {
+            ctx->flux_refused = dalloc(ctx, (char **)&ctx->flux, want) != 0;
+            ctx->flux_bytes = ctx->flux_refused ? 0 : want;
+            if (ctx->flux_refused) ctx->err[0] = 0;  // the pass goes on without it
+        }
+        flux = ctx->flux;
+        room = ctx->flux_bytes;
+    }
+    const ForcePlan plan = force_plan<R>(ctx->nact, room);
+    const size_t sums = (size_t)kDensSumsFD * ctx->cap * sizeof(double);
+    if (sums <= room || plan.segment == kForceSegment) return plan;
+    flux = ctx->dacc;
+    return force_plan<R>(ctx->nact, sums);
+}
+
 template <int KERN, typename R>
 int force_stage(gz_context *ctx)
 {
@@ -1212,26 +1249,8 @@ int force_stage(gz_context *ctx)
                 ctx->all_active ? nullptr : ctx->ACT, ctx->TB, ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2,
                 ctx->counters + 4, ctx->nact <= kRowPairAtomics ? ctx->u64c + 65 : nullptr, BoxTable{}, gate);
         } else {
-            // the stored fluxes: a buffer of their own, or (in a pool, or without memory for it) what
-            // is left of the pool or the density sums, which are free now
-            void *flux = ctx->flux;
-            ForcePlan plan = force_plan<R>(ctx->nact, ~(size_t)0);
-            if (ctx->flux_bytes < plan.bytes) {
-                const size_t sums = (size_t)kDensSumsFD * ctx->cap * sizeof(double);
-                if (ctx->pool) {
-                    const size_t at = (ctx->pool_used + 255) & ~(size_t)255;
-                    const size_t left = at < ctx->pool_size ? ctx->pool_size - at : 0;
-                    flux = left > sums ? (void *)(ctx->pool + at) : (void *)ctx->dacc;
-                    plan = force_plan<R>(ctx->nact, std::max(left, sums));
-                } else if (dalloc(ctx, (char **)&ctx->flux, plan.bytes) == 0) {
-                    flux = ctx->flux;
-                    ctx->flux_bytes = plan.bytes;
-                } else {
-                    ctx->flux_bytes = 0;
-                    flux = ctx->dacc;
-                    plan = force_plan<R>(ctx->nact, sums);
-                }
-            }
+            void *flux = nullptr;
+            const ForcePlan plan = flux_room<R>(ctx, flux);
             if (plan.segment < 1) return fail(ctx, GZ_E_MEMORY, "hydro_force(): no room for the stored fluxes (%ld particles)", ctx->cap);
             const ForceRows a{ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->all_active ? nullptr : ctx->ACT, ctx->TB,
                               ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2, ctx->counters + 4,
@@ -1725,6 +1744,7 @@ int gz_load(gz_context *ctx, long n, const gz_fields *f)
     CHK(set_device(ctx));
     ctx->n = n;
     ctx->density_ready = false;
+    ctx->flux_refused = false;
     // order along the Morton curve: keys from the caller's positions, stable radix sort
     HIPCHK(hipMemcpyAsync(ctx->stage, f->pos, (size_t)n * 3 * sizeof(double), hipMemcpyDefault, ctx->stream));
     {
@@ -2131,6 +2151,17 @@ int gz_set_option(gz_context *ctx, const char *name, double value)
     if (k == "force_split") {
         if (value != -1 && value != 0 && value != 1) return fail(ctx, GZ_E_ARG, "force_split must be -1, 0 or 1");
         ctx->force_split = (int)value;
+        return 0;
+    }
+    if (k == "force_room") {
+        if (value != -1 && !(value >= 0 && value <= 1e18)) return fail(ctx, GZ_E_ARG, "force_room must be -1 or in [0, 1e18] bytes");
+        if (value != ctx->force_room) {
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+            dfree(ctx->flux);
+            ctx->flux_bytes = 0;
+            ctx->flux_refused = false;
+        }
+        ctx->force_room = value;
         return 0;
     }
     if (k == "fd_correction") {

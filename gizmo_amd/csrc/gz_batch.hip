@@ -152,6 +152,8 @@ int balloc(gz_batch *b, T **p, size_t count)
     if (count == 0) count = 1;
     if (hipMalloc((void **)p, count * sizeof(T)) != hipSuccess) {
         *p = nullptr;
+        // reported here: a later launch check must not find it (the runtime keeps it until it is read)
+        (void)hipGetLastError();
         return fail(b, GZ_E_MEMORY, "hipMalloc of %zu bytes failed", count * sizeof(T));
     }
     b->alloc_bytes[(void *)*p] = count * sizeof(T);
@@ -217,6 +219,20 @@ double bits_to_double(unsigned long long u)
     return d;
 }
 
+// Room for the force pass's stored fluxes: of any number of the batch's rows (at most 100 MB; room -1),
+// or the bytes of the option "force_room".  Without it (refused by the device, or too small) the
+// density sums, which are free during that pass, serve with shorter segments.
+void alloc_flux(gz_batch *b, double room)
+{
+    const size_t whole = b->par.precision == GZ_FP64 ? force_plan<double>(b->cap, ~(size_t)0).bytes
+                                                     : force_plan<float>(b->cap, ~(size_t)0).bytes;
+    b->flux_bytes = room < 0 ? whole : (size_t)room;
+    if (balloc(b, (char **)&b->flux, b->flux_bytes)) {
+        b->flux_bytes = 0;
+        b->err.clear();  // the batch goes on without it
+    }
+}
+
 int alloc_all(gz_batch *b)
 {
     const size_t n = (size_t)b->cap;
@@ -236,9 +252,7 @@ int alloc_all(gz_batch *b)
     BCHK(balloc(b, (char **)&b->rec_force, n * sizeof(Cell<double>)));
     // (the sort keys of an order are free during a pass)
     b->rl_a = (int *)b->key64; b->rl_b = (int *)b->key64b;
-    // room for the force pass's stored fluxes of every row of the batch
-    b->flux_bytes = b->par.precision == GZ_FP64 ? force_plan<double>(b->cap, ~(size_t)0).bytes : force_plan<float>(b->cap, ~(size_t)0).bytes;
-    BCHK(balloc(b, (char **)&b->flux, b->flux_bytes));
+    alloc_flux(b, -1);
     const size_t nbx = nbox_all(b);
     BCHK(balloc(b, &b->tab, nbx)); BCHK(balloc(b, &b->hist, 64 * nbx)); BCHK(balloc(b, &b->slot, kBoxSlots * nbx));
     BCHK(balloc(b, &b->sel, nbx)); BCHK(balloc(b, &b->due, nbx)); BCHK(balloc(b, &b->rank, nbx)); BCHK(balloc(b, &b->lim, 2 * nbx));
@@ -673,10 +687,16 @@ int gradients_force(gz_batch *b)
     else
         k_pack_force<R><<<nb(b->cap), kB, 0, b->stream>>>(b->par.gamma, F, rf, b->counters + 2, 1.0, bt);
     if (lanes) {
-        const ForcePlan plan = force_plan<R>(na, b->flux_bytes);
+        void *flux = b->flux;
+        ForcePlan plan = force_plan<R>(na, b->flux_bytes);
+        const size_t sums = (size_t)kDensSumsFD * b->cap * sizeof(double);
+        if (sums > b->flux_bytes && plan.segment < kForceSegment) {
+            flux = b->dacc;
+            plan = force_plan<R>(na, sums);
+        }
         if (plan.segment < 1) return fail(b, GZ_E_MEMORY, "hydro_force(): no room for the stored fluxes (%ld particles)", b->cap);
         const ForceRows a{na, b->act, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV, b->WAKE, b->ACC, b->DTU, b->MSV, b->counters + 2,
-                          b->counters + 4, nullptr, b->flux, plan.segment, 0};
+                          b->counters + 4, nullptr, flux, plan.segment, 0};
         k_force<KERN, R, true><<<plan.blocks, kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);
     } else {
         k_force_rows<KERN, R><<<xcd_grid(na), kListThreads, 0, b->stream>>>(b->dp, G, na, b->act, F, rf, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV,
@@ -1197,6 +1217,13 @@ int gz_batch_set_option(gz_batch *b, const char *name, double value)
     if (!strcmp(name, "few_rows")) {
         if (!(value >= 0) || value > 2e9) return fail(b, GZ_E_ARG, "few_rows must be in [0, 2e9]");
         b->few_rows = (int)value;
+        return 0;
+    }
+    if (!strcmp(name, "force_room")) {
+        if (value != -1 && !(value >= 0 && value <= 1e18)) return fail(b, GZ_E_ARG, "force_room must be -1 or in [0, 1e18] bytes");
+        BCHK(set_device(b));
+        BCHK(sync(b));
+        alloc_flux(b, value);
         return 0;
     }
     if (!strcmp(name, "fd_correction")) {

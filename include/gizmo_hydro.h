@@ -232,7 +232,11 @@ int gz_drift_all(gz_context *ctx);
    read of the counters after the force pass then settles the step, and when the flag says no,
    the rounds go on and the three passes run again; "force_split" (default -1; 0 or 1) --
    0: the force pass does not count the rows of "force_rare_rows" (the pass itself is the same);
-   "force_waves" (default 0; 2 or 3) -- accepted for callers of earlier versions, without effect.
+   "force_waves" (default 0; 2 or 3) -- accepted for callers of earlier versions, without effect;
+   "force_room" (default -1; bytes) -- device memory that force passes over many rows may take
+   for the fluxes they store (-1: what any number of the context's rows needs, at most 100 MB);
+   with less, or when the device refuses it, the room of the density sums serves and the lists
+   are taken in shorter segments.
    None of these changes a neighbour set or a
    sum, and none has a counterpart in the reference (tuning knobs of this library).
    One option selects physics, the reference's compile-time HYDRO_PARTITION_UNITY_IMPROVE_FD

@@ -5,7 +5,9 @@ that just reach vacuum.  Each is compared with the general path bit for bit, or 
 import numpy as np
 import pytest
 
-from gizmo_amd.hydro import GZ_FP32_MIXED, GZ_FP64, Hydro
+from gizmo_amd import ics
+from gizmo_amd.batch import Batch
+from gizmo_amd.hydro import GZ_FP32_MIXED, GZ_FP64, GizmoHipError, Hydro
 
 pytestmark = pytest.mark.gpu
 
@@ -18,6 +20,28 @@ def params(**kw):
              max_kernel_radius=0.25, time=0.0, time_begin=0.0)
     p.update(kw)
     return p
+
+
+INTEG = dict(courant_fac=0.2, err_tol_int_accuracy=0.02, max_size_timestep=0.01, min_size_timestep=0.0, time_begin=0.0, time_max=1.0,
+             min_egy_spec=0.0)
+FORCE_OUT = ("accel", "dtu", "maxsig", "wakeup")
+
+
+def streams(side, mach, seed):
+    """Gas streams that collide at x = 1/2 and part at x = 0: many faces past the Riemann ladder's
+    common case."""
+    ic = ics.lattice_box(side, seed, kernel=6, des_num_ngb=64.0, mach_sigma=0.3)
+    cs = np.sqrt(ic["params"]["gamma"])
+    ic["vel"][:, 0] += np.where(ic["pos"][:, 0] < 0.5, mach, -mach) * cs
+    return ic
+
+
+def loaded(ic, precision, capacity=None, **options):
+    g = Hydro(dict(ic["params"]), capacity or len(ic["mass"]), precision)
+    for k, v in options.items():
+        g.set_option(k, v)
+    g.load({k: ic[k] for k in ("pos", "vel", "mass", "u", "h")})
+    return g
 
 
 def same_bits(a, b, rows=slice(None)):
@@ -78,3 +102,67 @@ def test_grid_of_512_cells_a_side(precision):
         out[few_rows] = g.store(DENSITY_OUT)
         g.close()
     same_bits(out[0], out[10 ** 9])
+
+
+@BOTH
+@pytest.mark.parametrize("room,spare", [(1e18, 1), (0, 1), (0, 8), (100000, 1), (2e6, 1)])
+def test_force_pass_with_less_room(room, spare, precision):
+    """The force pass over many rows without its scratch (the device refuses 10^18 bytes; none allowed)
+    or with less of it: the density sums' room and short segments.  Against whole segments, twice
+    (the refusal must not reach a later launch check), and against the row kernels."""
+    ic = streams(15, 5.0, 43)
+    n = len(ic["mass"])
+    out = {}
+    for name, options in (("whole", dict(few_rows=0)), ("less", dict(few_rows=0, force_room=room)), ("rows", dict(few_rows=10 ** 9))):
+        print(f"force room: {name} room={room} spare={spare} n={n} precision={precision}", flush=True)
+        g = loaded(ic, precision, spare * n, **options)
+        g.hydro_pass()
+        g.hydro_pass()
+        assert name == "rows" or g.stat("force_rare_rows") > 0
+        out[name] = g.store(FORCE_OUT)
+        g.close()
+    same_bits(out["less"], out["whole"])
+    same_bits(out["rows"], out["whole"])
+
+
+def test_force_pass_without_any_room_is_refused():
+    """So few particles that even the density sums hold less than an entry for each workgroup."""
+    rng = np.random.Generator(np.random.Philox(44))
+    n = 100
+    ic = dict(pos=rng.random((n, 3)), vel=rng.normal(size=(n, 3)), mass=np.full(n, 1.0 / n), u=np.ones(n), h=np.full(n, 0.2))
+    f = dict(ic, rho=np.ones(n), press=np.full(n, 2.0 / 3.0), numngb=np.full(n, 4.0), drkern=np.ones(n), divvel=np.zeros(n), cn=np.ones(n),
+             fce=np.zeros(n), nvt=np.tile([100.0, 100.0, 100.0, 0.0, 0.0, 0.0], (n, 1)), grad_rho=np.zeros((n, 3)), grad_p=np.zeros((n, 3)),
+             grad_v=np.zeros((n, 9)))
+    for room in (0, -1):
+        print(f"no room: n={n} force_room={room}", flush=True)
+        g = Hydro(params(), n, GZ_FP64)
+        g.set_option("few_rows", 0)
+        g.set_option("force_room", room)
+        g.load(f)
+        if room == 0:
+            with pytest.raises(GizmoHipError, match="no room"):
+                g.hydro_force()
+        else:
+            g.hydro_force()
+            assert np.isfinite(g.store(["accel"])["accel"]).all()
+        g.close()
+
+
+@BOTH
+def test_batch_with_less_room(precision):
+    boxes = [streams(s, 3.0, 45 + s) for s in (11, 14)]
+    out = {}
+    for room in (-1, 1e18, 0):
+        b = Batch(dict(boxes[0]["params"]), sum(len(ic["mass"]) for ic in boxes), 2, precision)
+        b.set_option("few_rows", 0)
+        b.set_option("force_room", room)
+        ids = [b.add({k: ic[k] for k in ("pos", "vel", "mass", "u", "h")}, ic["params"], INTEG) for ic in boxes]
+        print(f"batch room: {room} precision={precision}", flush=True)
+        b.begin()
+        for _ in range(2):
+            b.step()
+        out[room] = [b.store(i, ("h", "rho", "accel", "dtu")) for i in ids]
+        b.close()
+    for room in (1e18, 0):
+        for x, y in zip(out[room], out[-1]):
+            same_bits(x, y)
