@@ -533,6 +533,14 @@ int build_groups(gz_batch *b)
     return 0;
 }
 
+// particles per cell where the live boxes' grids hold most (the cost of a walk of their groups)
+double per_cell(const gz_batch *b)
+{
+    std::vector<BoxCells> boxes;
+    for (int id : b->order) boxes.push_back({(long)b->boxes[id].n, 1L << (3 * b->boxes[id].level)});
+    return fullest_cells(boxes);
+}
+
 // ---------------------------------------------------------------------------------------
 // the hot path over the active rows of every box in the pass
 // ---------------------------------------------------------------------------------------
@@ -559,7 +567,7 @@ int density(gz_batch *b)
     while (true) {
         BHIP(hipMemsetAsync(b->counters, 0, 3 * sizeof(int), b->stream));
         // the later rounds' few rows: one workgroup each from the list of rows still iterating
-        const int *rows = many && iters > 0 && density_by_row(remaining, na) ? b->rl_a : nullptr;
+        const int *rows = many && iters > 0 && density_by_row(remaining, b->grp.ngroups, per_cell(b)) ? b->rl_a : nullptr;
         const int nround = rows ? remaining : na;
         if (rows) {
             if (remaining <= b->few_rows)

@@ -356,13 +356,6 @@ __global__ void k_gradients(DevParams P, int nrows, const int *act, const double
 // evaluate that many candidates or list entries at once, then lanes of the first wavefront add
 // the accepted terms in order
 constexpr int kRowThreads = 256;
-// Density rounds after the first of a batch's pass over many rows: up to half of the rows, still
-// iterating, are taken one workgroup each from the list that the closing kernel wrote.  A cell walk costs
-// nearly as much for one row of a cell as for all; on the coarse grids of small boxes it takes 2.1 ns per
-// row of the pass, the row kernel 3.5 ns (twelve boxes of 16^3 to 64^3, a third to two thirds of the rows
-// iterating again: 30.9 -> 26.2 ms of density rounds in 20 steps).  On one large grid the walk takes 0.5
-// to 0.7 ns, and its later rounds keep nearly all rows or none: no list there.
-inline bool density_by_row(long remaining, long na) { return 2 * remaining <= na; }
 // TPB threads per row: kRowThreads when few rows run (each row's rounds are latency-bound),
 // 64 when many do (lanes past a row's last candidate would idle)
 template <int KERN, typename R, int TPB>

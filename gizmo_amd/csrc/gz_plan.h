@@ -1,7 +1,9 @@
 // gz_plan.h -- launch arithmetic of the host: grid sizes and the rules that choose between kernels
 // by sizes.  Plain C++ (no HIP), so that the CPU tests compile it as it is.
 #pragma once
+#include <algorithm>
 #include <cstddef>
+#include <vector>
 
 namespace gz {
 
@@ -16,6 +18,42 @@ inline unsigned stencil_grid(long ncell)
 {
     const long most = 1L << 22, blocks = (kStencilThreads * ncell + 255) / 256;
     return (unsigned)(blocks < most ? blocks : most);
+}
+
+// Density rounds after the first of a batch's pass over many rows: whether the rows still iterating are
+// taken one workgroup each, from the list that the closing kernel wrote, or by a walk of every group
+// (the rows of one cell) again.  By row a row takes 2 to 4 ns (FP64 3 to 6).  A walk takes nearly as long for
+// one row of a group as for all, and longer the more particles the cells hold: 28 to 35 ns a group
+// at 16 to 64 particles per cell, 80 to 100 at 125, 200 at 244; each XCD walks a contiguous eighth
+// of the groups, so the boxes of the fullest cells set the time; and below some 3000 groups it takes as long
+// as one wavefront, 120 to 300 us.  The line: 5 rows per group and a sixth of the particles per cell in the
+// fullest eighth of the cells, of at least 3072 groups.  24 batches (equal boxes of 20^3 to 128^3,
+// mixtures of 12^3 to 110^3, both forms), their later rounds of 10 to 12 steps together: always the walk
+// 428 ms, always by row up to half of the rows 375, this line 338, the faster way of each round 336; up to
+// half of the rows, two boxes of 128^3 took 29.2 ms where the walk takes 19.8.  One box on one
+// grid keeps nearly all rows or none after its first round: no list there.
+constexpr long kFewGroups = 3072;
+struct BoxCells { long particles, cells; };
+// the mean number of particles per cell in the fullest eighth of the boxes' cells
+inline double fullest_cells(std::vector<BoxCells> boxes)
+{
+    std::sort(boxes.begin(), boxes.end(), [](const BoxCells &a, const BoxCells &b) {
+        return (double)a.particles * (double)b.cells > (double)b.particles * (double)a.cells;
+    });
+    double cells = 0;
+    for (const BoxCells &b : boxes) cells += (double)b.cells;
+    const double eighth = cells > 8 ? cells / 8 : 1;
+    double left = eighth, held = 0;
+    for (const BoxCells &b : boxes) {
+        const double part = (double)b.cells < left ? (double)b.cells : left;
+        held += part * (double)b.particles / (double)b.cells;
+        left -= part;
+    }
+    return held / eighth;
+}
+inline bool density_by_row(long remaining, long ngroups, double per_cell)
+{
+    return (double)remaining <= (double)(ngroups > kFewGroups ? ngroups : kFewGroups) * (5.0 + per_cell / 6.0);
 }
 
 // The force pass over many rows (k_force): 64 rows of four lanes each per workgroup at a time.

@@ -19,6 +19,19 @@ int main()
             if (std::scanf("%ld %zu", &nrows, &room) != 2) return 1;
             const gz::ForcePlan p = what[5] == '3' ? gz::force_plan<float>(nrows, room) : gz::force_plan<double>(nrows, room);
             std::printf("%d %d %zu\n", p.blocks, p.segment, p.bytes);
+        } else if (!std::strcmp(what, "by_row")) {
+            // the groups, the rows still iterating, then the kinds of boxes: how many, particles and cells of one
+            long ngroups, remaining, kinds;
+            if (std::scanf("%ld %ld %ld", &ngroups, &remaining, &kinds) != 3) return 1;
+            std::vector<gz::BoxCells> boxes;
+            while (kinds-- > 0) {
+                long count;
+                gz::BoxCells one;
+                if (std::scanf("%ld %ld %ld", &count, &one.particles, &one.cells) != 3) return 1;
+                boxes.insert(boxes.end(), (size_t)count, one);
+            }
+            const double per_cell = gz::fullest_cells(boxes);
+            std::printf("%d %.17g\n", gz::density_by_row(remaining, ngroups, per_cell), per_cell);
         } else {
             return 1;
         }

@@ -166,3 +166,26 @@ def test_batch_with_less_room(precision):
     for room in (1e18, 0):
         for x, y in zip(out[room], out[-1]):
             same_bits(x, y)
+
+
+@BOTH
+def test_batch_later_rounds_walk_and_by_row(precision):
+    """A batch whose second density round keeps so many rows that its groups are walked again, and whose
+    later rounds then take the rest by row, against the pass that takes every round by row."""
+    rng = np.random.Generator(np.random.Philox(47))
+    boxes = [ics.lattice_box(s, 50 + s, kernel=6, des_num_ngb=64.0, mach_sigma=0.5) for s in (31, 47)]
+    for ic in boxes:  # nearly every radius needs a second round, some need more
+        ic["h"] = ic["h"] * rng.uniform(0.85, 1.15, len(ic["h"]))
+    out = {}
+    for few_rows in (0, 10 ** 9):
+        b = Batch(dict(boxes[0]["params"]), sum(len(ic["mass"]) for ic in boxes), 2, precision)
+        b.set_option("few_rows", few_rows)
+        ids = [b.add({k: ic[k] for k in ("pos", "vel", "mass", "u", "h")}, ic["params"], INTEG) for ic in boxes]
+        print(f"batch later rounds: few_rows={few_rows} precision={precision}", flush=True)
+        b.begin()
+        b.step()
+        out[few_rows] = [b.store(i, ("h", "rho", "numngb", "accel", "dtu")) for i in ids]
+        print(f"rounds: {b.stat('density_iterations'):.0f}", flush=True)
+        b.close()
+    for x, y in zip(out[0], out[10 ** 9]):
+        same_bits(x, y)

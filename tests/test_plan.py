@@ -47,3 +47,72 @@ def test_force_plan_of_any_room(ask, form, width):
             assert size <= room and size == blocks * segment * entry
             assert blocks % 8 == 0 and 8 <= blocks <= -(-whole // 8) * 8 and segment <= 96
             assert (segment == 0) == (room < 8 * entry), (nrows, room)
+
+
+# Later density rounds of batches as measured on the MI355X (FP32 form, then FP64, then mixtures of
+# boxes): the boxes (count x particles / cells), the groups, the rows still iterating, microseconds of
+# the walk and by row
+ROUNDS = [
+    ("24x8000/64", 1142, 34573, 150, 116),
+    ("24x8000/64", 1336, 90389, 217, 260),
+    ("3x10648/512 21x10648/64", 1669, 33965, 411, 126),
+    ("7x10648/512 17x10648/64", 4016, 120472, 493, 387),
+    ("5x13824/512 15x13824/64", 1650, 15555, 459, 81),
+    ("12x13824/512 8x13824/64", 6656, 171327, 743, 530),
+    ("12x21952/512", 4863, 34589, 184, 85),
+    ("12x21952/512", 6144, 164142, 225, 330),
+    ("10x32768/512", 3629, 74692, 167, 168),
+    ("10x32768/512", 3595, 135111, 202, 295),
+    ("8x46656/512", 2436, 46512, 280, 136),
+    ("8x46656/512", 3629, 183604, 326, 465),
+    ("6x59319/512", 1841, 22617, 173, 76),
+    ("6x59319/512", 3072, 192438, 298, 537),
+    ("2x91125/4096 4x91125/512", 6309, 72441, 761, 268),
+    ("3x91125/512 3x91125/4096", 13354, 249613, 1390, 798),
+    ("6x140608/4096", 20006, 105506, 591, 226),
+    ("5x140608/4096 1x140608/512", 20992, 475775, 1927, 1782),
+    ("8x262144/4096", 24950, 404623, 822, 942),
+    ("8x262144/4096", 16490, 539596, 755, 1267),
+    ("4x512000/4096", 10022, 89923, 787, 315),
+    ("4x512000/4096", 16384, 1014366, 1386, 2936),
+    ("4x1000000/32768", 111269, 556076, 3153, 1248),
+    ("3x1000000/32768 1x1000000/4096", 102400, 2037913, 9305, 8544),
+    ("2x2097152/32768", 35048, 496640, 1134, 1200),
+    ("2x2097152/32768", 65536, 1685263, 2202, 4093),
+    ("5x13824/512 15x13824/64", 1650, 15554, 446, 107),
+    ("12x13824/512 8x13824/64", 6656, 171327, 776, 757),
+    ("8x46656/512", 2436, 46507, 322, 191),
+    ("8x46656/512", 3629, 183606, 412, 684),
+    ("8x262144/4096", 24950, 404623, 1097, 1380),
+    ("8x262144/4096", 16490, 539582, 989, 1784),
+    ("4x1000000/32768", 111269, 556046, 4336, 1875),
+    ("3x1000000/32768 1x1000000/4096", 102400, 2037926, 12072, 12461),
+    ("1x32768/512 1x42875/512 1x54872/512 2x636056/4096 1x300763/4096", 9752, 666810, 1466, 2202),
+    ("1x32768/512 1x42875/512 1x54872/512 2x636056/4096 1x300763/4096", 7973, 230986, 641, 523),
+    ("1x456533/4096 1x804357/4096 1x1157625/32768 1x493039/4096", 45056, 1892330, 4857, 7279),
+    ("1x456533/4096 1x804357/32768 1x1157625/4096 1x493039/4096", 13106, 81387, 1007, 389),
+    ("1x166375/4096 1x205379/4096 1x262144/4096 1x148877/4096 1x636056/4096 1x681472/4096", 24576, 1320940, 4695, 5818),
+    ("1x166375/4096 1x205379/4096 1x262144/4096 1x148877/4096 1x636056/4096 1x681472/4096", 18956, 129162, 800, 630),
+]
+
+
+def test_later_density_rounds_take_no_slower_way(ask):
+    """The way that the rule takes costs at most a tenth more than the walk of any measured round, and
+    all of them together at most a twentieth more than the faster ways."""
+    questions = []
+    for boxes, groups, remaining, _, _ in ROUNDS:
+        kinds = [k.replace("/", "x").split("x") for k in boxes.split()]
+        questions.append(["by_row", groups, remaining, len(kinds)] + [x for k in kinds for x in k])
+    taken = [row if by_row else walk for (_, _, _, walk, row), (by_row, _) in zip(ROUNDS, ask(questions))]
+    for r, t in zip(ROUNDS, taken):
+        assert t <= 1.1 * r[3], r
+    assert sum(taken) <= 1.05 * sum(min(r[3:]) for r in ROUNDS)
+
+
+def test_particles_per_cell_of_the_fullest_eighth(ask):
+    """Weighted by cells: one small box of full cells among large ones does not set it, half of the
+    boxes do; no boxes and boxes of one cell are answered too."""
+    got = [a[1] for a in ask([("by_row", 1, 1, 2, 1, 1728, 8, 1, 16384, 512), ("by_row", 1, 1, 2, 2, 1000000, 32768, 2, 1000000, 4096),
+                              ("by_row", 1, 1, 1, 3, 50, 1), ("by_row", 1, 1, 0), ("by_row", 1, 1, 1, 1, 0, 1)])]
+    want = [(8 * 216 + 57 * 32) / 65, (8192 * 1e6 / 4096 + 1024 * 1e6 / 32768) / 9216, 50, 0, 0]
+    assert got == pytest.approx(want, rel=1e-12)
