@@ -626,12 +626,16 @@ __device__ inline R guess_p(const Gam<R> &G, const RState<R> &L, const RState<R>
 }
 
 // (p / p_k)^((gamma - 1) / (2 gamma)) of a rarefaction, p <= p_k.  The logarithm times the exponent
-// is of order one, so the exponential's result is within an ulp or two of pow()'s, at a third of
-// its instructions; the wave's slope needs the power -(gamma + 1) / (2 gamma), this one over the
-// pressure ratio (the exponents add to -1).  A wavefront's Newton step costs ~350 instructions
-// instead of ~960 as soon as one of its lanes is in a rarefaction.
+// is of order one for ordinary ratios, so the exponential's result is within an ulp or two of
+// pow()'s, at a third of its instructions (near vacuum the product's rounding grows with the logarithm: a dozen
+// ulps at a ratio of 1e-50, where the power no longer matters beside the 1 it is taken from).
+// The wave's slope needs the power -(gamma + 1) / (2 gamma), this one over the pressure ratio (the
+// exponents add to -1; infinite, as pow()'s, at a ratio of 0).  A wavefront's Newton step costs ~350
+// instructions instead of ~960 as soon as one of its lanes is in a rarefaction.
 template <typename R>
 __device__ __forceinline__ R rarefaction_power(const Gam<R> &G, R ratio) { return exp(G.G1 * log(ratio)); }
+template <typename R>
+__device__ __forceinline__ R rarefaction_slope(R power, R ratio) { return ratio == R(0) ? (R)HUGE_VAL : power / ratio; }
 
 template <typename R>
 __device__ inline int iterative_riemann(const Gam<R> &G, const RState<R> &L, const RState<R> &Rs, R vL, R vR, R csL, R csR, ROut<R> &o)
@@ -670,7 +674,7 @@ __device__ inline int iterative_riemann(const Gam<R> &G, const RState<R> &L, con
         } else {
             const R pr = Pg / L.p, w = rarefaction_power(G, pr);
             WL = G.G4 * csL * (w - R(1));
-            ZL = R(1) / (L.rho * csL) * (w / pr);
+            ZL = R(1) / (L.rho * csL) * rarefaction_slope(w, pr);
         }
         if (Pg > Rs.p) {
             R a0 = G.G5 / Rs.rho, a1 = G.G6 * Rs.p, a2 = sqrt(a0 / (Pg + a1));
@@ -679,7 +683,7 @@ __device__ inline int iterative_riemann(const Gam<R> &G, const RState<R> &L, con
         } else {
             const R pr = Pg / Rs.p, w = rarefaction_power(G, pr);
             WR = G.G4 * csR * (w - R(1));
-            ZR = R(1) / (Rs.rho * csR) * (w / pr);
+            ZR = R(1) / (Rs.rho * csR) * rarefaction_slope(w, pr);
         }
         if (it < 1000 / 2) Pg -= (WL + WR + dvel) / (ZL + ZR);
         else Pg -= R(0.5) * (WL + WR + dvel) / (ZL + ZR);

@@ -189,3 +189,25 @@ def test_batch_later_rounds_walk_and_by_row(precision):
         b.close()
     for x, y in zip(out[0], out[10 ** 9]):
         same_bits(x, y)
+
+
+@BOTH
+def test_rarefactions_that_just_reach_vacuum(oracle_lib, precision):
+    """Two streams that part at exactly the speed at which their rarefactions reach vacuum: the exact
+    solver's first pressure is 0, where a rarefaction's slope is infinite and the pressure stays 0
+    (gamma = 3, with which every quantity of the state is exact in both forms)."""
+    c = np.zeros((2, 24))
+    c[:, 0:2] = c[:, 5:7] = [1.0, 3.0]
+    c[:, 2], c[:, 7] = [-3.0, -2.5], [3.0, 3.5]  # sound speed 3 on both sides
+    c[:, 10] = 1.0
+    c[:, 14:16], c[:, 16:18] = 3.0, 1.0
+    c[:, 18], c[:, 21] = c[:, 7], c[:, 2]
+    for mode in (4, 1, 0) if precision == GZ_FP64 else (4,):
+        print(f"vacuum edge: mode={mode} precision={precision}", flush=True)
+        g = Hydro(params(gamma=3.0), 16, precision)
+        dev, rung = g.riemann_probe(mode, c)
+        g.close()
+        ora, want = oracle_lib.riemann_probe(mode, 3.0, c)
+        assert np.array_equal(dev, ora) and np.array_equal(rung, want), (mode, dev, ora)
+        if mode == 4:
+            assert (ora[:, 0] == 0).all() and np.array_equal(ora[:, 1], [0.0, 0.5])
