@@ -211,3 +211,25 @@ def test_rarefactions_that_just_reach_vacuum(oracle_lib, precision):
         assert np.array_equal(dev, ora) and np.array_equal(rung, want), (mode, dev, ora)
         if mode == 4:
             assert (ora[:, 0] == 0).all() and np.array_equal(ora[:, 1], [0.0, 0.5])
+
+
+@BOTH
+@pytest.mark.parametrize("side", [11, 21], ids=["four_cells", "eight_cells"])
+@pytest.mark.parametrize("scale", [1.0, 1e-46], ids=["unit", "below_fp32"])
+def test_retired_and_light_particles_in_the_cell_walk(side, scale, precision):
+    """Partners are the particles of positive mass: retired ones (mass 0, or below) are none, and ones
+    whose mass rounds to 0 in the FP32 form count as neighbours all the same.  The cell walk against
+    the row kernels."""
+    ic = ics.lattice_box(side, 48, kernel=6, des_num_ngb=64.0, mach_sigma=0.3)
+    rng = np.random.Generator(np.random.Philox(49))
+    n = len(ic["mass"])
+    ic["mass"] = np.where(rng.random(n) < 0.1, rng.choice([0.0, -1.0, -1e-300], n), ic["mass"] * scale)
+    out = {}
+    for few_rows in (0, 10 ** 9):
+        print(f"light particles: n={n} scale={scale} few_rows={few_rows} precision={precision}", flush=True)
+        g = loaded(ic, precision, few_rows=few_rows)
+        g.density()
+        out[few_rows] = g.store(DENSITY_OUT)
+        g.close()
+    assert abs(np.median(out[0]["numngb"][ic["mass"] > 0]) ** 3 - 64.0) < 1.0  # (kept as the cube root of the number)
+    same_bits(out[0], out[10 ** 9])
