@@ -630,12 +630,12 @@ __device__ inline R guess_p(const Gam<R> &G, const RState<R> &L, const RState<R>
 // pow()'s, at a third of its instructions (near vacuum the product's rounding grows with the logarithm: a dozen
 // ulps at a ratio of 1e-50, where the power no longer matters beside the 1 it is taken from).
 // The wave's slope needs the power -(gamma + 1) / (2 gamma), this one over the pressure ratio (the
-// exponents add to -1; infinite, as pow()'s, at a ratio of 0).  A wavefront's Newton step costs ~350
+// exponents add to -1; infinite, as pow()'s, at a ratio of 0, where the added 1e-300 counts alone).  A wavefront's Newton step costs ~350
 // instructions instead of ~960 as soon as one of its lanes is in a rarefaction.
 template <typename R>
 __device__ __forceinline__ R rarefaction_power(const Gam<R> &G, R ratio) { return exp(G.G1 * log(ratio)); }
-template <typename R>
-__device__ __forceinline__ R rarefaction_slope(R power, R ratio) { return ratio == R(0) ? (R)HUGE_VAL : power / ratio; }
+template <typename R>  // (FP64: the FP32 form solves in FP64 too)
+__device__ __forceinline__ R rarefaction_slope(R power, R ratio) { return (power + R(1e-300)) / ratio; }
 
 template <typename R>
 __device__ inline int iterative_riemann(const Gam<R> &G, const RState<R> &L, const RState<R> &Rs, R vL, R vR, R csL, R csR, ROut<R> &o)
