@@ -233,3 +233,32 @@ def test_retired_and_light_particles_in_the_cell_walk(side, scale, precision):
         g.close()
     assert abs(np.median(out[0]["numngb"][ic["mass"] > 0]) ** 3 - 64.0) < 1.0  # (kept as the cube root of the number)
     same_bits(out[0], out[10 ** 9])
+
+
+@pytest.mark.parametrize("ncoarse", [700, 767, 768, 769, 1500])
+def test_groups_with_many_coarse_partners(oracle_lib, ncoarse):
+    """The symmetric list of a tight clump inside the radii of ncoarse particles of three coarser
+    levels: collected and merged up to 768 of them, inserted into the finished rows one by one
+    beyond.  Groups of rows against one wavefront per row, and the sets against the oracle's."""
+    rng = np.random.Generator(np.random.Philox(50))
+    clump = 0.4 + rng.uniform(-0.004, 0.004, (150, 3))
+    away = rng.normal(size=(ncoarse, 3))
+    away *= (rng.uniform(0.03, 0.11, ncoarse) / np.linalg.norm(away, axis=1))[:, None]
+    pos = np.concatenate((clump, 0.4 + away))
+    h = np.concatenate((np.full(150, 0.003), rng.choice([0.125, 0.2, 0.24], ncoarse)))
+    n = len(pos)
+    lists = {}
+    for few_rows in (0, 10 ** 9):
+        print(f"coarse partners: n={n} few_rows={few_rows}", flush=True)
+        g = loaded(dict(params=params(), pos=pos, vel=np.zeros((n, 3)), mass=np.ones(n), u=np.ones(n), h=h), GZ_FP64, wide_search=1,
+                   few_rows=few_rows)
+        lists[few_rows] = g.neighbors(1)
+        g.close()
+    for a, b in zip(lists[0], lists[10 ** 9]):
+        assert np.array_equal(a, b)
+    off, nbr = lists[0]
+    assert (np.diff(off)[:150] >= ncoarse).all()
+    ref_off, ref = oracle_lib.neighbors(params(), pos, h, 1)
+    assert np.array_equal(off, ref_off)
+    for i in range(n):
+        assert np.array_equal(np.sort(nbr[off[i]:off[i + 1]]), ref[off[i]:off[i + 1]]), i
