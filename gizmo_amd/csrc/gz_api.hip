@@ -74,7 +74,8 @@ struct gz_context {
     bool speculate = false, spec = false;
     bool spec_enabled = true;  // option "speculate"
     bool fd = false;           // option "fd_correction": the first-derivative volume correction of the density
-    int force_split = -1;      // option "force_split": 0 leaves the rows with rare faces uncounted
+    int force_split = -1;      // option "force_split": the FP32 form's lanes first (1), never (0), by the last pass (-1)
+    double rare_share = 1;     // share of rows with a face past the common case in the last pass that counted them
     bool force_flags_clear = false;  // the last gradient launch cleared the force pass's flags
     bool in_run_steps = false;       // inside gz_run_steps' loop
     bool prepped = false;            // the last step's closing kick cleared this step's counters
@@ -1252,11 +1253,22 @@ int force_stage(gz_context *ctx)
             void *flux = nullptr;
             const ForcePlan plan = flux_room<R>(ctx, flux);
             if (plan.segment < 1) return fail(ctx, GZ_E_MEMORY, "hydro_force(): no room for the stored fluxes (%ld particles)", ctx->cap);
-            const ForceRows a{ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->all_active ? nullptr : ctx->ACT, ctx->TB,
-                              ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2, ctx->counters + 4,
-                              ctx->sched_valid ? ctx->sched : nullptr, flux, plan.segment, ctx->force_split != 0 && !ctx->rung_stats};
-            auto lanes_kernel = ctx->rung_stats ? k_force<KERN, R, false, true> : k_force<KERN, R, false, false>;
-            lanes_kernel<<<plan.blocks, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
+            ForceRows a{ctx->nact, ctx->act, ctx->ell_s, ctx->ld_s, ctx->cnt_s, ctx->all_active ? nullptr : ctx->ACT, ctx->TB,
+                        ctx->MSV, ctx->WAKE, ctx->ACC, ctx->DTU, ctx->MSV, ctx->counters + 2, ctx->counters + 4,
+                        ctx->sched_valid ? ctx->sched : nullptr, flux, plan.segment, ctx->force_split != 0 && !ctx->rung_stats,
+                        ctx->it_it, nullptr};
+            if constexpr (std::is_same<R, float>::value) {
+                if (!ctx->rung_stats && (ctx->force_split == 1 || (ctx->force_split < 0 && force_by_lanes(ctx->nact, ctx->rare_share)))) {
+                    k_force_lanes<KERN, false><<<xcd_grid(nblk(ctx->nact)), kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a,
+                                                                                                     BoxTable{});
+                    // the rows it left (listed in the density iteration's counts, which are free now)
+                    a.sched = a.rare;
+                    a.nrows_dev = a.err + 12;
+                    a.count_rare = 0;
+                }
+            }
+            auto quads_kernel = ctx->rung_stats ? k_force<KERN, R, false, true> : k_force<KERN, R, false, false>;
+            quads_kernel<<<plan.blocks, kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a, BoxTable{});
         }
         // the pairs of the pass: each row's workgroup adds its own while a few hundred rows are
         // active (atomics on one address execute one after another)
@@ -1288,7 +1300,10 @@ int force_stage(gz_context *ctx)
         }
     }
     // rows with a face past the Riemann ladder's common case (counters[14]: zero unless counted)
-    if (ctx->nact > ctx->few_rows && !ctx->rung_stats) ctx->st.force_rare_rows += ctx->hcounters[14];
+    if (ctx->nact > ctx->few_rows && !ctx->rung_stats) {
+        ctx->st.force_rare_rows += ctx->hcounters[14];
+        if (ctx->force_split != 0) ctx->rare_share = (double)ctx->hcounters[14] / (double)ctx->nact;
+    }
     if (ctx->lazy && ctx->hmax_bound > 0) {
         // the radii the passes' lazy drifts produced (u64c[75], read back with the counters)
         double hl;

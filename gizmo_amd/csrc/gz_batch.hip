@@ -82,6 +82,7 @@ struct gz_batch {
     int *rl_a = nullptr, *rl_b = nullptr;  // rows still iterating in density rounds (in key64, key64b): the coming round's, the next one's
     void *flux = nullptr;  // the force pass's stored fluxes
     size_t flux_bytes = 0;
+    double rare_share = 1;  // share of rows with a face past the Riemann ladder's common case in the last pass over many
     int *ell = nullptr, *cnt = nullptr;
     int ell_cap = 0;
     void *tmp = nullptr;
@@ -703,8 +704,17 @@ int gradients_force(gz_batch *b)
             plan = force_plan<R>(na, sums);
         }
         if (plan.segment < 1) return fail(b, GZ_E_MEMORY, "hydro_force(): no room for the stored fluxes (%ld particles)", b->cap);
-        const ForceRows a{na, b->act, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV, b->WAKE, b->ACC, b->DTU, b->MSV, b->counters + 2,
-                          b->counters + 4, nullptr, flux, plan.segment, 0};
+        ForceRows a{na, b->act, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV, b->WAKE, b->ACC, b->DTU, b->MSV, b->counters + 2,
+                    b->counters + 4, nullptr, flux, plan.segment, std::is_same<R, float>::value, b->it_it, nullptr};
+        if constexpr (std::is_same<R, float>::value) {
+            if (force_by_lanes(na, b->rare_share)) {
+                k_force_lanes<KERN, true><<<xcd_grid(nb(na)), kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);
+                // the rows it left (listed in the density iteration's counts, which are free now)
+                a.sched = a.rare;
+                a.nrows_dev = a.err + 12;
+                a.count_rare = 0;
+            }
+        }
         k_force<KERN, R, true><<<plan.blocks, kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);
     } else {
         k_force_rows<KERN, R><<<xcd_grid(na), kListThreads, 0, b->stream>>>(b->dp, G, na, b->act, F, rf, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV,
@@ -714,6 +724,7 @@ int gradients_force(gz_batch *b)
     k_sum_counts<<<std::min(nb(na), 256u), kB, 0, b->stream>>>(na, b->cnt, b->u64);
     BHIP(hipGetLastError());
     BCHK(read_back(b, false));
+    if (lanes && std::is_same<R, float>::value) b->rare_share = (double)b->hcounters[14] / (double)na;
     if (b->hcounters[2]) return fail(b, GZ_STOP_RIEMANN, "hydro_force(): Riemann solver failed to find a positive pressure");
     return 0;
 }

@@ -407,12 +407,18 @@ struct ForceRows {
     void *flux;                  // scratch: a segment's fluxes of each workgroup (ForcePlan)
     int segment;                 // list entries of a row between two rounds of queued faces
     int count_rare;              // count the rows with a face past the Riemann ladder's common case into err[12]
+    int *rare;                   // k_force_lanes: receives the rows it leaves, their number in err[12]
+    const int *nrows_dev;        // FP32 form: the number of rows, on the device (nullptr: nrows)
 };
 
 // Four lanes per row, kForceRowsPerBlock rows per workgroup at a time, on kForceBlocks workgroups at most.
 // STATS: count the faces' RiemannRung bits into F.rungs.
 template <int KERN, typename R, bool BOXES, bool STATS = false>
 __global__ void k_force(DevParams P, Gam<R> G, ForceView F, const Cell<R> *rec, ForceRows a, BoxTable bt);
+// FP32 form, one lane per row: rows whose faces all take the Riemann ladder's common case; the others are
+// listed in a.rare, for k_force (force_by_lanes)
+template <int KERN, bool BOXES>
+__global__ void k_force_lanes(DevParams P, Gam<float> G, ForceView F, const Cell<float> *rec, ForceRows a, BoxTable bt);
 // few-row force passes over at most this many rows make their records in the row kernel (its
 // MAKE form holds one wave per SIMD: this many rows of two wavefronts fill the chip once)
 constexpr int kMakeForceRows = 512;

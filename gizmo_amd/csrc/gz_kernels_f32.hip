@@ -51,6 +51,13 @@ namespace gz {
                                                    int *, unsigned long long *, BoxTable, const int *);
 GZ_INST(3, float)
 GZ_INST(6, float)
+// the force kernel of quiet gas
+#define GZ_INST_QUIET(KERN, BOXES)                                                                                               \
+    template __global__ void k_force_lanes<KERN, BOXES>(DevParams, Gam<float>, ForceView, const Cell<float> *, ForceRows, BoxTable);
+GZ_INST_QUIET(3, false)
+GZ_INST_QUIET(6, false)
+GZ_INST_QUIET(3, true)
+GZ_INST_QUIET(6, true)
 // the force kernels that count the Riemann rungs of their faces (one box)
 #define GZ_INST_STATS(KERN, R)                                                                                                   \
     template __global__ void k_force<KERN, R, false, true>(DevParams, Gam<R>, ForceView, const Cell<R> *, ForceRows, BoxTable);     \

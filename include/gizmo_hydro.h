@@ -231,7 +231,11 @@ int gz_drift_all(gz_context *ctx);
    a device flag: the round converged every row and no radius outgrew the list's grid); one
    read of the counters after the force pass then settles the step, and when the flag says no,
    the rounds go on and the three passes run again; "force_split" (default -1; 0 or 1) --
-   0: the force pass does not count the rows of "force_rare_rows" (the pass itself is the same);
+   the FP32 form's force pass over more than few_rows rows takes the rows whose faces all take the
+   Riemann ladder's common case one lane per row and leaves the others to the general kernel
+   (1), takes all rows through the general kernel (0, which also leaves the rows of
+   "force_rare_rows" uncounted, in either form), or (-1) the former from 196608 rows on while at
+   most a quarter of the rows had a face past the common case in the pass before;
    "force_waves" (default 0; 2 or 3) -- accepted for callers of earlier versions, without effect;
    "force_room" (default -1; bytes) -- device memory that force passes over many rows may take
    for the fluxes they store (-1: what any number of the context's rows needs, at most 100 MB);

@@ -32,6 +32,11 @@ int main()
             }
             const double per_cell = gz::fullest_cells(boxes);
             std::printf("%d %.17g\n", gz::density_by_row(remaining, ngroups, per_cell), per_cell);
+        } else if (!std::strcmp(what, "lanes")) {
+            long nrows;
+            double share;
+            if (std::scanf("%ld %lf", &nrows, &share) != 2) return 1;
+            std::printf("%d\n", gz::force_by_lanes(nrows, share));
         } else {
             return 1;
         }

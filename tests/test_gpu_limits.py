@@ -262,3 +262,57 @@ def test_groups_with_many_coarse_partners(oracle_lib, ncoarse):
     assert np.array_equal(off, ref_off)
     for i in range(n):
         assert np.array_equal(np.sort(nbr[off[i]:off[i + 1]]), ref[off[i]:off[i + 1]]), i
+
+
+def patchy(side, seed, share):
+    """Quiet gas with a slab of violent motion, `share` of the box: the rows with a face past the Riemann
+    ladder's common case."""
+    ic = ics.lattice_box(side, seed, kernel=6, des_num_ngb=64.0, mach_sigma=0.003)
+    rng = np.random.Generator(np.random.Philox(seed))
+    ic["vel"][ic["pos"][:, 0] < share] += rng.normal(size=(int((ic["pos"][:, 0] < share).sum()), 3)) * 0.8
+    return ic
+
+
+@pytest.mark.parametrize("share,active", [(0.0, 1.0), (0.1, 1.0), (0.1, 0.95)])
+def test_quiet_gas_by_lanes(share, active):
+    """The FP32 form's pass over many rows of quiet gas: from the second pass on one lane per row takes the
+    rows of the common case and leaves the others to the general kernel, which takes all of them
+    with the option force_split at 0.  Wake-up flags, too, where some neighbours are inactive."""
+    ic = patchy(59, 51, share)
+    n = len(ic["mass"])
+    rows = np.random.Generator(np.random.Philox(52)).random(n) < active
+    out, rare = {}, {}
+    for split in (0, -1, 1):
+        print(f"quiet gas: n={n} share={share} active={active} force_split={split}", flush=True)
+        g = loaded(ic, GZ_FP32_MIXED, force_split=split)
+        for _ in range(2):
+            g.hydro_pass()
+        if active < 1.0:
+            g.set_active(rows)
+        g.timing_reset()
+        g.hydro_pass()
+        rare[split] = g.stat("force_rare_rows") / rows.sum()
+        out[split] = g.store(FORCE_OUT)
+        g.close()
+    print(f"rows past the common case: {rare[-1]:.3f}", flush=True)
+    # (a row has such a face only with a moving particle within reach: in the slab, or a radius from it)
+    assert rare[0] == 0 and rare[-1] == rare[1] <= 0.25 and share <= rare[1] <= (share + 2 * ic["h"].max() if share else 0)
+    same_bits(out[-1], out[0])
+    same_bits(out[1], out[0])
+
+
+def test_quiet_gas_by_lanes_in_a_batch():
+    boxes = [patchy(s, 53 + s, x) for s, x in ((48, 0.0), (50, 0.1))]
+    out = {}
+    for few_rows in (8192, 10 ** 9):
+        b = Batch(dict(boxes[0]["params"]), sum(len(ic["mass"]) for ic in boxes), 2, GZ_FP32_MIXED)
+        b.set_option("few_rows", few_rows)
+        ids = [b.add({k: ic[k] for k in ("pos", "vel", "mass", "u", "h")}, ic["params"], INTEG) for ic in boxes]
+        print(f"quiet batch: few_rows={few_rows}", flush=True)
+        b.begin()
+        for _ in range(3):
+            b.step()
+        out[few_rows] = [b.store(i, ("h", "rho", "accel", "dtu", "vel")) for i in ids]
+        b.close()
+    for x, y in zip(out[8192], out[10 ** 9]):
+        same_bits(x, y)

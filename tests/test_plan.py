@@ -116,3 +116,17 @@ def test_particles_per_cell_of_the_fullest_eighth(ask):
                               ("by_row", 1, 1, 1, 3, 50, 1), ("by_row", 1, 1, 0), ("by_row", 1, 1, 1, 1, 0, 1)])]
     want = [(8 * 216 + 57 * 32) / 65, (8192 * 1e6 / 4096 + 1024 * 1e6 / 32768) / 9216, 50, 0, 0]
     assert got == pytest.approx(want, rel=1e-12)
+
+
+# The FP32 form's force pass as measured on the MI355X: rows, the share of them with a face past the
+# Riemann ladder's common case, microseconds of the general kernel alone and behind one lane per row
+PASSES = [(140608, 0, 403, 362), (140608, 0.0004, 413, 463), (140608, 0.2374, 509, 607), (262144, 0, 598, 473), (262144, 0, 687, 456),
+          (262144, 0.0187, 805, 564), (262144, 0.2377, 880, 715), (262144, 0.7338, 933, 1177), (512000, 0, 1387, 920),
+          (512000, 0.0983, 1719, 1142), (1030301, 0.2388, 3541, 2689), (1030301, 0.7333, 3732, 4408), (2097152, 0, 4744, 3319),
+          (2097152, 0, 5542, 3407), (2097152, 0.0006, 5591, 3522), (2097152, 0.1631, 6972, 4656), (2097152, 0.7333, 7491, 8775)]
+
+
+def test_quiet_force_passes_go_by_lanes(ask):
+    """At most a tenth and 50 us more than the faster way of every measured pass."""
+    for (rows, share, general, lanes), (by_lanes,) in zip(PASSES, ask([("lanes", p[0], p[1]) for p in PASSES])):
+        assert (lanes if by_lanes else general) <= 1.1 * min(general, lanes) + 50, (rows, share)
