@@ -732,7 +732,7 @@ int build_wide(gz_context *ctx, bool lists)
     W.lpos = ctx->wlpos;
     W.lkey = ctx->wlkey;
     Timed t(ctx, "ngb_build");
-    k_block_boxes<<<nblk(n), kBlock, 0, ctx->stream>>>((int)n, ctx->X, ctx->Y, ctx->Z, ctx->H, ctx->wboxes);
+    k_block_boxes<<<nblk(n), kBlock, 0, ctx->stream>>>((int)n, ctx->X, ctx->Y, ctx->Z, ctx->H, 1.0 / box, ctx->wboxes);
     HIPCHK(hipGetLastError());
     if (ctx->wide_key_version != ctx->key_version || lmax > ctx->wide_lmax) {
         k_wide_bounds<<<nblk(n), kBlock, 0, ctx->stream>>>(W);
@@ -757,7 +757,7 @@ int build_wide(gz_context *ctx, bool lists)
             W.lofs[L] = acc;
             if (L <= kFineLevel) acc += counts[L];
         }
-        k_wide_list_bounds<<<nblk(n), kBlock, 0, ctx->stream>>>(W, ctx->plev, ctx->X, ctx->Y, ctx->Z, ctx->H);
+        k_wide_list_bounds<<<nblk(n), kBlock, 0, ctx->stream>>>(W, ctx->plev, ctx->X, ctx->Y, ctx->Z, ctx->H, 1.0 / box);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipMemcpyAsync(ctx->wide_dev, &W, sizeof W, hipMemcpyHostToDevice, ctx->stream));

@@ -41,8 +41,8 @@ struct WideGrid {
     int *lstart, *lend;
     long long loff[kFineLevel + 1];
     int lofs[kFineLevel + 2];
-    const float4 *boxes;       // per 64 particles of the order: lowest corner and largest radius, highest corner
-    float4 *lpos;              // per entry of lidx: position and radius, rounded (for tests with slack)
+    const float4 *boxes;       // per 64 particles of the order, in units of the box: lowest corner and largest radius, highest corner
+    float4 *lpos;              // per entry of lidx: position and radius in units of the box, rounded (for tests with slack)
     uint32_t *lkey;            // per entry of lidx: its key
 };
 
@@ -240,7 +240,8 @@ __global__ void k_group_stencil(GridView g, int ngroups, const uint32_t *gkey, c
 // search over many grid levels
 __global__ void k_wide_bounds(WideGrid W);
 __global__ void k_particle_level(int n, const double *H, double box, double margin, int lmax, int *plev, int *level_count);
-__global__ void k_wide_list_bounds(WideGrid W, const int *plev, const double *X, const double *Y, const double *Z, const double *H);
+__global__ void k_wide_list_bounds(WideGrid W, const int *plev, const double *X, const double *Y, const double *Z, const double *H,
+                                   double inv_box);
 __global__ void k_build_sym_wide(GridView g, int nrows, const int *act, const double *X, const double *Y, const double *Z,
                                  const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
 
@@ -292,7 +293,7 @@ __global__ void k_cell_rows_list(int nact, const int *act, const uint32_t *key, 
                                  int *cells);
 __global__ void k_build_sym_cells(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
                                   const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
-__global__ void k_block_boxes(int n, const double *X, const double *Y, const double *Z, const double *H, float4 *boxes);
+__global__ void k_block_boxes(int n, const double *X, const double *Y, const double *Z, const double *H, double inv_box, float4 *boxes);
 __global__ void k_build_sym_groups(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
                                    const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
 // cells of at most this many rows on average: one candidate per lane (k_build_sym_groups), whose

@@ -233,12 +233,15 @@ __device__ __forceinline__ void row_stencil_wide(const GridView &g, const WideGr
 // ---------------------------------------------------------------------------------------
 #ifdef GZ_DEFINE_COMMON_KERNELS
 __global__ void __launch_bounds__(256) k_block_boxes(int n, const double *__restrict__ X, const double *__restrict__ Y,
-                                                     const double *__restrict__ Z, const double *__restrict__ H, float4 *__restrict__ boxes)
+                                                     const double *__restrict__ Z, const double *__restrict__ H, double inv_box,
+                                                     float4 *__restrict__ boxes)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     const bool on = j < n;
-    // rounded outwards by the caller's slack (2^-23 of the box)
-    const float x = on ? (float)X[j] : 0.0f, y = on ? (float)Y[j] : 0.0f, z = on ? (float)Z[j] : 0.0f, h = on ? (float)H[j] : 0.0f;
+    // in units of the box, whose squares FP32 holds whatever the caller's units are; rounded outwards by
+    // the caller's slack (2^-23 of the box)
+    const float x = on ? (float)(X[j] * inv_box) : 0.0f, y = on ? (float)(Y[j] * inv_box) : 0.0f, z = on ? (float)(Z[j] * inv_box) : 0.0f,
+                h = on ? (float)(H[j] * inv_box) : 0.0f;
     const float lx = wave_minf(on ? x : 1e30f), ly = wave_minf(on ? y : 1e30f), lz = wave_minf(on ? z : 1e30f);
     const float mx = -wave_minf(on ? -x : 1e30f), my = -wave_minf(on ? -y : 1e30f), mz = -wave_minf(on ? -z : 1e30f), hm = -wave_minf(-h);
     if (on && (j & 63) == 0) {
@@ -248,18 +251,18 @@ __global__ void __launch_bounds__(256) k_block_boxes(int n, const double *__rest
 }
 #endif
 
-// what a block's particles are tested against: the rows' bounding box (centre, half extents) and radius
+// what a block's particles are tested against: the rows' bounding box (centre, half extents) and radius,
+// in units of the box
 struct BlockReach {
-    float cx, cy, cz, ex, ey, ez, h, box;
+    float cx, cy, cz, ex, ey, ez, h;
     // whether a pair of a row and a particle of block b may lie within the larger radius (SYM) or the
     // row's; the slack covers the FP32 rounding of the positions and the boxes
     template <bool SYM> __device__ __forceinline__ bool hits(const float4 &lo, const float4 &hi) const
     {
-        const float half = 0.5f * box;
         auto gap = [&](float c, float e, float l, float m) {
             float d = fabsf(c - 0.5f * (l + m));
-            d = d > half ? box - d : d;
-            return fmaxf(d - e - 0.5f * (m - l) - 2e-6f * box, 0.0f);
+            d = d > 0.5f ? 1.0f - d : d;
+            return fmaxf(d - e - 0.5f * (m - l) - 2e-6f, 0.0f);
         };
         const float gx = gap(cx, ex, lo.x, hi.x), gy = gap(cy, ey, lo.y, hi.y), gz = gap(cz, ez, lo.z, hi.z);
         const float r = (SYM ? fmaxf(h, lo.w) : h) * (1.0f + 1e-5f);
@@ -474,7 +477,7 @@ __global__ void __launch_bounds__(TPB) k_density_rows(DevParams P, GridView g, i
     };
     const bool long_walk = g.wide && total > kLongWalk;
     const bool marked = total <= kMarked;
-    const BlockReach reach{(float)xi, (float)yi, (float)zi, 0.0f, 0.0f, 0.0f, (float)h, (float)g.box};
+    const BlockReach reach{(float)(xi * inv_box), (float)(yi * inv_box), (float)(zi * inv_box), 0.0f, 0.0f, 0.0f, (float)(h * inv_box)};
     unsigned long long live = ~0ull;
     int head = 0, fill = 0;  // the partners found and not yet added: list places head .. head + fill - 1
     int turn = 0;  // the rank buffer of the next walked run (a skipped run has no barrier: it must not turn)
@@ -613,7 +616,7 @@ __global__ void __launch_bounds__(256) k_particle_level(int n, const double *__r
 // the range of every cell of level L among the particles of level L (positions in lidx)
 __global__ void __launch_bounds__(256) k_wide_list_bounds(WideGrid W, const int *__restrict__ plev, const double *__restrict__ X,
                                                           const double *__restrict__ Y, const double *__restrict__ Z,
-                                                          const double *__restrict__ H)
+                                                          const double *__restrict__ H, double inv_box)
 {
     const long p = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (p >= W.n) return;
@@ -625,7 +628,7 @@ __global__ void __launch_bounds__(256) k_wide_list_bounds(WideGrid W, const int 
     if (p == lo || (W.key[W.lidx[p - 1]] >> s) != c) W.lstart[W.loff[L] + c] = (int)p;
     if (p + 1 == hi || (W.key[W.lidx[p + 1]] >> s) != c) W.lend[W.loff[L] + c] = (int)(p + 1);
     W.lkey[p] = W.key[j];
-    W.lpos[p] = make_float4((float)X[j], (float)Y[j], (float)Z[j], (float)H[j]);
+    W.lpos[p] = make_float4((float)(X[j] * inv_box), (float)(Y[j] * inv_box), (float)(Z[j] * inv_box), (float)(H[j] * inv_box));
 }
 
 __device__ __forceinline__ bool periodic_adjacent(int a, int b, int nc)
@@ -1029,10 +1032,10 @@ __global__ void __launch_bounds__(64, 4) k_build_sym_groups(GridView g, CellRows
         int ncoarse = 0;  // part B's particles (above kMaxCoarse: not collected)
         if (wide) {
             const WideGrid &W = *g.wide;
-            // the group's centre and the slack for positions rounded to 32 bits, in cells
-            const float bx = (float)g.box, inv_b = 1.0f / bx, ic = (float)inv_cell, sl = 4e-7f * (float)nci;
-            const float gx = (float)((hx + 0.5) * g.cell), gy = (float)((hy + 0.5) * g.cell), gz = (float)((hz + 0.5) * g.cell);
-            auto near = [&](float d) { return __builtin_fmaf(-__builtin_rintf(d * inv_b), bx, d) * ic; };
+            // the group's centre in units of the box, and the slack for positions rounded to 32 bits, in cells
+            const float ic = (float)nci, inv_c = 1.0f / ic, sl = 4e-7f * ic;
+            const float gx = ((float)hx + 0.5f) * inv_c, gy = ((float)hy + 0.5f) * inv_c, gz = ((float)hz + 0.5f) * inv_c;
+            auto near = [&](float d) { return (d - __builtin_rintf(d)) * ic; };
             for (int L = 0; L < g.level && ncoarse <= kMaxCoarse; L++) {
                 if (t == 0) runs[L] = ncoarse;
                 if (W.lofs[L + 1] == W.lofs[L]) continue;  // no particle of this level
@@ -1104,20 +1107,19 @@ __global__ void __launch_bounds__(64, 4) k_build_sym_groups(GridView g, CellRows
         bool more = cells.total > 0, left = false, keep = false;
         const bool long_walk = wide && cells.total > kLongWalk;
         const float ncf = (float)nci, inv_ncf = 1.0f / ncf;
-        const float side = (float)g.cell;
-        const BlockReach reach{(float)(hx * g.cell) + (0.5f * (lx + mx) + 0.5f) * side, (float)(hy * g.cell) + (0.5f * (ly + my) + 0.5f) * side,
-                               (float)(hz * g.cell) + (0.5f * (lz + mz) + 0.5f) * side, 0.5f * (mx - lx) * side, 0.5f * (my - ly) * side,
-                               0.5f * (mz - lz) * side, hleaf * side, (float)g.box};
+        const float side = inv_ncf;  // the cell's, in units of the box
+        const BlockReach reach{((float)hx + 0.5f * (lx + mx) + 0.5f) * side, ((float)hy + 0.5f * (ly + my) + 0.5f) * side,
+                               ((float)hz + 0.5f * (lz + mz) + 0.5f) * side, 0.5f * (mx - lx) * side, 0.5f * (my - ly) * side,
+                               0.5f * (mz - lz) * side, hleaf * side};
         // a block within reach of the rows' box and, for few rows, of one of them: a coarse cell's few
         // rows span a box that holds whole clumps which none of them reaches
-        const float xf = (float)xi, yf = (float)yi, zf = (float)zi, hf = (float)hi;
+        const float xf = (float)(xi * inv_box), yf = (float)(yi * inv_box), zf = (float)(zi * inv_box), hf = (float)(hi * inv_box);
         auto hit = [&](const float4 &lo, const float4 &hi) {
             bool any = reach.hits<true>(lo, hi);
             if (rows <= 16 && wave_any(any)) {
                 bool one = false;
                 for (int a = 0; a < rows; a++)
-                    one |= BlockReach{lane_value(xf, a), lane_value(yf, a), lane_value(zf, a), 0.0f, 0.0f, 0.0f, lane_value(hf, a),
-                                      reach.box}.hits<true>(lo, hi);
+                    one |= BlockReach{lane_value(xf, a), lane_value(yf, a), lane_value(zf, a), 0.0f, 0.0f, 0.0f, lane_value(hf, a)}.hits<true>(lo, hi);
                 any = any && one;
             }
             return any;

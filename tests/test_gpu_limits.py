@@ -316,3 +316,24 @@ def test_quiet_gas_by_lanes_in_a_batch():
         b.close()
     for x, y in zip(out[8192], out[10 ** 9]):
         same_bits(x, y)
+
+
+@pytest.mark.parametrize("box", [1.0, 1e-21, 3e-22, 3e24])
+def test_wide_search_in_other_units(box):
+    """Long walks of the search over many levels in a box of any size (FP64): the squares of distances
+    lie far below and above what FP32 holds.  Against one grid, bit for bit."""
+    ic = ics.lognormal_box(20000, 57, ng=32)
+    s = box
+    ic["params"] = dict(ic["params"], box=s, max_kernel_radius=0.25 * s)
+    out = {}
+    for wide in (0, 1):
+        print(f"wide units: box={box} wide={wide}", flush=True)
+        g = Hydro(ic["params"], len(ic["mass"]), GZ_FP64)
+        g.set_option("wide_search", wide)
+        g.load(dict(pos=ic["pos"] * s, vel=ic["vel"], mass=ic["mass"], u=ic["u"], h=ic["h"] * s))
+        g.density()
+        out[wide] = (g.store(DENSITY_OUT), g.neighbors(1))
+        g.close()
+    same_bits(out[1][0], out[0][0])
+    for a, b in zip(out[1][1], out[0][1]):
+        assert np.array_equal(a, b)
