@@ -732,8 +732,11 @@ int build_wide(gz_context *ctx, bool lists)
     W.lpos = ctx->wlpos;
     W.lkey = ctx->wlkey;
     Timed t(ctx, "ngb_build");
-    k_block_boxes<<<nblk(n), kBlock, 0, ctx->stream>>>((int)n, ctx->X, ctx->Y, ctx->Z, ctx->H, 1.0 / box, ctx->wboxes);
-    HIPCHK(hipGetLastError());
+    // (the list of few rows walks row by row, without the boxes)
+    if (n > kLongWalk && (!lists || ctx->nact > ctx->few_rows)) {
+        k_block_boxes<<<nblk(n), kBlock, 0, ctx->stream>>>((int)n, ctx->X, ctx->Y, ctx->Z, ctx->H, 1.0 / box, ctx->wboxes);
+        HIPCHK(hipGetLastError());
+    }
     if (ctx->wide_key_version != ctx->key_version || lmax > ctx->wide_lmax) {
         k_wide_bounds<<<nblk(n), kBlock, 0, ctx->stream>>>(W);
         HIPCHK(hipGetLastError());

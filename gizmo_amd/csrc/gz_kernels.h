@@ -293,6 +293,7 @@ __global__ void k_cell_rows_list(int nact, const int *act, const uint32_t *key, 
                                  int *cells);
 __global__ void k_build_sym_cells(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
                                   const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);
+constexpr int kLongWalk = 1024;  // candidates from which a walk asks for its live runs first (the block boxes' only use)
 __global__ void k_block_boxes(int n, const double *X, const double *Y, const double *Z, const double *H, double inv_box, float4 *boxes);
 __global__ void k_build_sym_groups(GridView g, CellRows cr, const int *act, const double *X, const double *Y, const double *Z,
                                    const double *H, int *ell, long ld, int cap, int *cnt, int *overflow);

@@ -299,7 +299,6 @@ __device__ __forceinline__ unsigned long long live_runs(const float4 *__restrict
     }
     return __ballot(live);
 }
-constexpr int kLongWalk = 1024;  // candidates from which a walk asks for its live runs first
 
 // The place of this thread's entry among the flagged entries of its workgroup, in thread order
 // (total: the flagged entries of the workgroup).  One barrier for several wavefronts, none for one.
