@@ -217,7 +217,7 @@ def roofline_full_pass(fp, form):
     bytes_total = fp["n_active"] * (m["S_i"] + m["S_out"]) + fp["pairs"] * (m["S_j"] + 4)
     achieved = bytes_total / (ms / 1e3) / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4), "kernel": f"k_force<6,{'double' if form == 'fp64' else 'float'}>",
+            "frac": round(achieved / HBM_PEAK_GBS, 4), "kernel": "k_force<6,double>" if form == "fp64" else "k_force_lanes<6>, k_force<6,float>",
             "launches": 1, "bytes_per_launch": int(bytes_total), "avg_launch_ms": ms}
 
 

@@ -76,6 +76,7 @@ struct gz_context {
     bool fd = false;           // option "fd_correction": the first-derivative volume correction of the density
     int force_split = -1;      // option "force_split": the FP32 form's lanes first (1), never (0), by the last pass (-1)
     double rare_share = 1;     // share of rows with a face past the common case in the last pass that counted them
+    double list_even = 0;      // list sum over 64 x the sum of the waves' longest lists in the last pass over many rows
     bool force_flags_clear = false;  // the last gradient launch cleared the force pass's flags
     bool in_run_steps = false;       // inside gz_run_steps' loop
     bool prepped = false;            // the last step's closing kick cleared this step's counters
@@ -1029,27 +1030,31 @@ int density_rounds(gz_context *ctx, int iters, bool speculate)
 
 constexpr int kRowPairAtomics = 1024;  // at most this many rows count their pairs with one atomic each
 
-// the order in which the lanes of the force pass take the rows: longest symmetric list first
-// within each block of sched_span rows (the gradient pass, cheaper per pair, keeps the plain
-// order: its scattered writes would cost more than the even waves save)
+// the order in which the force pass takes the rows: longest symmetric list first within each
+// block of sched_span rows (the gradient pass, cheaper per pair, keeps the plain order: its
+// scattered writes would cost more than the even waves save); and how even the plain order is,
+// which the next pass's choice of kernel asks (force_by_lanes)
 int build_sched(gz_context *ctx)
 {
-    const int na = ctx->nact;
+    const int na = ctx->nact, span = ctx->sched_span;
+    const bool fp64 = ctx->par.precision == GZ_FP64;
+    if (span == 0 && (fp64 || na < kLaneRows)) return 0;
     const int nparts = (int)((na + 1023) / 1024);
     if (!ctx->sched) {
         CHK(dalloc(ctx, &ctx->sched, ctx->cap));
         CHK(dalloc(ctx, &ctx->sched_part, 2 * ((ctx->cap + 1023) / 1024) + 2));
     }
-    // FP64 pairs are compute-bound: always sorted; FP32 pairs only when the waves are uneven
-    const double min_even = ctx->par.precision == GZ_FP64 ? 2.0 : 0.75;
     unsigned long long *total = ctx->sched_part + 2 * nparts;
-    const int span = ctx->sched_span;
     Timed t(ctx, "ngb_build");
     k_sched_stats<<<nparts, 1024, 0, ctx->stream>>>(na, ctx->cnt_s, ctx->sched_part);
-    k_sched_total<<<1, 1024, 0, ctx->stream>>>(nparts, ctx->sched_part, total);
-    k_sched_sort<<<(unsigned)((na + span - 1) / span), 1024, 0, ctx->stream>>>(na, span, ctx->cnt_s, total, min_even, ctx->sched);
+    k_sched_total<<<1, 1024, 0, ctx->stream>>>(nparts, ctx->sched_part, total, ctx->counters + 7);
+    if (span > 0) {
+        // FP64 pairs are compute-bound: always sorted; FP32 pairs only when the waves are uneven
+        k_sched_sort<<<(unsigned)((na + span - 1) / span), 1024, 0, ctx->stream>>>(na, span, ctx->cnt_s, total, fp64 ? 2.0 : kPlainEven,
+                                                                                  ctx->sched);
+        ctx->sched_valid = true;
+    }
     HIPCHK(hipGetLastError());
-    ctx->sched_valid = true;
     return 0;
 }
 
@@ -1126,7 +1131,7 @@ int ensure_sym(gz_context *ctx)
             ctx->sym_valid = true;
             ctx->sym_check_pending = ctx->defer_sym_check;
             ctx->sched_valid = false;
-            if (!few && ctx->sched_span > 0) CHK(build_sched(ctx));
+            if (!few) CHK(build_sched(ctx));
             // the records the gradient and force passes read: every record when many rows are
             // active, else only those of the rows and their neighbours, packed from the list (a
             // record once per list entry that names it: cheaper while the lists hold fewer
@@ -1261,7 +1266,7 @@ int force_stage(gz_context *ctx)
                         ctx->sched_valid ? ctx->sched : nullptr, flux, plan.segment, ctx->force_split != 0 && !ctx->rung_stats,
                         ctx->it_it, nullptr};
             if constexpr (std::is_same<R, float>::value) {
-                if (!ctx->rung_stats && (ctx->force_split == 1 || (ctx->force_split < 0 && force_by_lanes(ctx->nact, ctx->rare_share)))) {
+                if (!ctx->rung_stats && (ctx->force_split == 1 || (ctx->force_split < 0 && force_by_lanes(ctx->nact, ctx->rare_share, ctx->list_even)))) {
                     k_force_lanes<KERN, false><<<xcd_grid(nblk(ctx->nact)), kBlock, 0, ctx->stream>>>(ctx->dp, gam<R>(ctx->dp), F, rec, a,
                                                                                                      BoxTable{});
                     // the rows it left (listed in the density iteration's counts, which are free now)
@@ -1306,6 +1311,7 @@ int force_stage(gz_context *ctx)
     if (ctx->nact > ctx->few_rows && !ctx->rung_stats) {
         ctx->st.force_rare_rows += ctx->hcounters[14];
         if (ctx->force_split != 0) ctx->rare_share = (double)ctx->hcounters[14] / (double)ctx->nact;
+        ctx->list_even = 1e-6 * ctx->hcounters[7];
     }
     if (ctx->lazy && ctx->hmax_bound > 0) {
         // the radii the passes' lazy drifts produced (u64c[75], read back with the counters)
@@ -1984,6 +1990,7 @@ int gz_stat(gz_context *ctx, const char *name, double *value)
         *value = (double)v;
         return 0;
     }
+    if (k == "list_even") { *value = ctx->list_even; return 0; }
     if (k == "force_pairs_total") {
         unsigned long long v = 0;
         HIPCHK(hipMemcpy(&v, ctx->u64c + 65, sizeof v, hipMemcpyDeviceToHost));

@@ -82,6 +82,7 @@ struct gz_batch {
     int *rl_a = nullptr, *rl_b = nullptr;  // rows still iterating in density rounds (in key64, key64b): the coming round's, the next one's
     void *flux = nullptr;  // the force pass's stored fluxes
     size_t flux_bytes = 0;
+    double list_even = 0;   // list sum over 64 x the sum of the waves' longest lists in the last pass over as many rows as lanes take
     double rare_share = 1;  // share of rows with a face past the Riemann ladder's common case in the last pass over many
     int *ell = nullptr, *cnt = nullptr;
     int ell_cap = 0;
@@ -707,7 +708,14 @@ int gradients_force(gz_batch *b)
         ForceRows a{na, b->act, b->ell, ld, b->cnt, b->ACT, b->TB, b->MSV, b->WAKE, b->ACC, b->DTU, b->MSV, b->counters + 2,
                     b->counters + 4, nullptr, flux, plan.segment, std::is_same<R, float>::value, b->it_it, nullptr};
         if constexpr (std::is_same<R, float>::value) {
-            if (force_by_lanes(na, b->rare_share)) {
+            if (na >= kLaneRows) {
+                // how even the lists are, for the next pass
+                const int nparts = (na + 1023) / 1024;
+                unsigned long long *part = (unsigned long long *)b->stage;
+                k_sched_stats<<<nparts, 1024, 0, b->stream>>>(na, b->cnt, part);
+                k_sched_total<<<1, 1024, 0, b->stream>>>(nparts, part, part + 2 * nparts, b->counters + 7);
+            }
+            if (force_by_lanes(na, b->rare_share, b->list_even)) {
                 k_force_lanes<KERN, true><<<xcd_grid(nb(na)), kB, 0, b->stream>>>(b->dp, G, F, rf, a, bt);
                 // the rows it left (listed in the density iteration's counts, which are free now)
                 a.sched = a.rare;
@@ -724,7 +732,10 @@ int gradients_force(gz_batch *b)
     k_sum_counts<<<std::min(nb(na), 256u), kB, 0, b->stream>>>(na, b->cnt, b->u64);
     BHIP(hipGetLastError());
     BCHK(read_back(b, false));
-    if (lanes && std::is_same<R, float>::value) b->rare_share = (double)b->hcounters[14] / (double)na;
+    if (lanes && std::is_same<R, float>::value) {
+        b->rare_share = (double)b->hcounters[14] / (double)na;
+        if (na >= kLaneRows) b->list_even = 1e-6 * b->hcounters[7];
+    }
     if (b->hcounters[2]) return fail(b, GZ_STOP_RIEMANN, "hydro_force(): Riemann solver failed to find a positive pressure");
     return 0;
 }

@@ -434,7 +434,7 @@ __global__ void k_riemann_probe(int mode, Gam<R> G, long n, const double *in, do
 // order are uneven enough (list sum over 64 x the sum of the waves' longest lists below
 // min_even; the scattered reads of the sorted order cost more than even waves save otherwise)
 __global__ void k_sched_stats(int nrows, const int *cnt, unsigned long long *partial);
-__global__ void k_sched_total(int nparts, const unsigned long long *partial, unsigned long long *total);
+__global__ void k_sched_total(int nparts, const unsigned long long *partial, unsigned long long *total, int *even);
 constexpr int kSchedMaxSpan = 2048;
 __global__ void k_sched_sort(int nrows, int span, const int *cnt, const unsigned long long *total, double min_even, int *sched);
 

@@ -1754,9 +1754,9 @@ __global__ void __launch_bounds__(1024) k_sched_stats(int nrows, const int *__re
     }
 }
 
-// the totals of the partial sums (one block)
+// the totals of the partial sums, and how even the waves of the plain order are (in millionths; one block)
 __global__ void __launch_bounds__(1024) k_sched_total(int nparts, const unsigned long long *__restrict__ partial,
-                                                      unsigned long long *__restrict__ total)
+                                                      unsigned long long *__restrict__ total, int *__restrict__ even)
 {
     __shared__ unsigned long long ss[16], sm[16];
     unsigned long long a = 0, b = 0;
@@ -1773,6 +1773,7 @@ __global__ void __launch_bounds__(1024) k_sched_total(int nparts, const unsigned
         for (int k = 0; k < (int)(blockDim.x >> 6); k++) { x += ss[k]; y += sm[k]; }
         total[0] = x;
         total[1] = y;
+        *even = (int)(1e6 * (double)x / (64.0 * (double)(y > 0 ? y : 1)));
     }
 }
 

@@ -91,15 +91,23 @@ template <typename R> inline ForcePlan force_plan(long nrows, size_t room)
     return ForcePlan{(int)blocks, (int)seg, (size_t)blocks * seg * entry};
 }
 
+// How even the lists of a pass are in the rows' plain order: their sum over 64 times the sum of the
+// wavefronts' longest.  Below this the FP32 form sorts its rows by list length, block by block.
+constexpr double kPlainEven = 0.75;
 // Whether a pass over many rows of the FP32 form goes through one lane per row first (k_force_lanes), the rows
 // with a face past the Riemann ladder's common case behind it through k_force: by the share of such
-// rows in the pass before (a guess of speed alone: every row's sums are the same; a context's first
-// pass takes k_force).  Lanes first against k_force alone, 2M rows: no such rows 3.3 and 4.7 ms (a blast) or
-// 3.4 and 5.5, 5% 3.9 and 6.6, 24% 5.2 and 7.1, 40% 6.4 and 7.3, 73% 8.8 and 7.5; 262K rows: none 0.46 and
-// 0.69, 24% 0.72 and 0.88, 40% 0.93 and 0.90; 141K rows, two workgroups of lanes per CU: none 0.36 and 0.40, but
-// 0.04% of the rows 0.46 and 0.41 (the few rows' own launch), 24% 0.61 and 0.51.
+// rows and the evenness of the lists in the pass before (a guess of speed alone: every row's sums are
+// the same; a context's first pass takes k_force).  Lanes first against k_force alone, 2M rows: no such
+// rows 3.3 and 4.7 ms (a blast) or 3.4 and 5.5, 5% 3.9 and 6.6, 24% 5.2 and 7.1, 40% 6.4 and 7.3, 73% 8.8 and 7.5; 262K
+// rows: none 0.46 and 0.69, 24% 0.72 and 0.88, 40% 0.93 and 0.90; 141K rows, two workgroups of lanes per CU: none
+// 0.36 and 0.40, but 0.04% of the rows 0.46 and 0.41 (the few rows' own launch), 24% 0.61 and 0.51.  512K rows, no such
+// rows, lists of evenness 0.92 0.92 and 1.39, 0.79 0.94 and 1.43, 0.71 1.37 and 1.20 (a wavefront of lanes lasts as long
+// as its longest list); 1M rows of a lognormal field (0.53) 3.7 and 3.0.
 constexpr long kLaneRows = 196608;
 constexpr double kLaneShare = 0.25;
-inline bool force_by_lanes(long nrows, double rare_share) { return nrows >= kLaneRows && rare_share <= kLaneShare; }
+inline bool force_by_lanes(long nrows, double rare_share, double list_even)
+{
+    return nrows >= kLaneRows && rare_share <= kLaneShare && list_even >= kPlainEven;
+}
 
 }  // namespace gz

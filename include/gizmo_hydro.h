@@ -127,7 +127,9 @@ int gz_synchronize(gz_context *ctx);
    "pairs_symmetric", "ngb_rebuilds", "n_active", "ell_widen"), and totals since the last
    gz_timing_reset ("active_updates": active particles through the hot path, "resorts",
    "force_pairs_total": neighbour pairs of every force launch, "force_rare_rows": rows of
-   force passes over many rows with a face past the Riemann ladder's common case).  With the option
+   force passes over many rows with a face past the Riemann ladder's common case); "list_even":
+   how even the lists of the last pass over many rows were, their sum over 64 times the sum of
+   the longest of each 64 rows.  With the option
    "riemann_stats" set to 1, the force passes of a single box also count, per face, the rungs of
    the Riemann ladder it took (each at most once per face) since the option was last set:
    "riemann_faces" (faces that reached the Riemann solve), "riemann_hllc", "riemann_vacuum",
@@ -235,7 +237,8 @@ int gz_drift_all(gz_context *ctx);
    Riemann ladder's common case one lane per row and leaves the others to the general kernel
    (1), takes all rows through the general kernel (0, which also leaves the rows of
    "force_rare_rows" uncounted, in either form), or (-1) the former from 196608 rows on while at
-   most a quarter of the rows had a face past the common case in the pass before;
+   most a quarter of the rows had a face past the common case in the pass before and its lists
+   were even ("list_even" of gz_stat at least 0.75);
    "force_waves" (default 0; 2 or 3) -- accepted for callers of earlier versions, without effect;
    "force_room" (default -1; bytes) -- device memory that force passes over many rows may take
    for the fluxes they store (-1: what any number of the context's rows needs, at most 100 MB);

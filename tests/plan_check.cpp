@@ -34,9 +34,9 @@ int main()
             std::printf("%d %.17g\n", gz::density_by_row(remaining, ngroups, per_cell), per_cell);
         } else if (!std::strcmp(what, "lanes")) {
             long nrows;
-            double share;
-            if (std::scanf("%ld %lf", &nrows, &share) != 2) return 1;
-            std::printf("%d\n", gz::force_by_lanes(nrows, share));
+            double share, even;
+            if (std::scanf("%ld %lf %lf", &nrows, &share, &even) != 3) return 1;
+            std::printf("%d\n", gz::force_by_lanes(nrows, share, even));
         } else {
             return 1;
         }
