@@ -1627,7 +1627,8 @@ __global__ void __launch_bounds__(256, 2)
 // wavefronts per SIMD hide the loads of the records where k_force's two wait for them).  A row with a face
 // past that case is listed for k_force, and nothing of it is written but its neighbours' wake-up
 // flags, which k_force sets again to the same values.  Each row's sums are k_force's, bit for bit.
-// 2M rows at rest or nearly so 5.5 -> 3.4 ms.  Bound by the gathers of the records (a lane reads its own).
+// 2M rows at rest or nearly so 5.5 -> 3.4 ms.  Bound by its VALU instructions (0.19 of an issue rate of 0.25;
+// the quads' 0.16), with 8.3 GB from beyond the L2 (a lane reads its own partner's record, 16K rows in flight on an XCD).
 template <int KERN, bool BOXES>
 __global__ void __launch_bounds__(256) k_force_lanes(DevParams P0, Gam<float> G, ForceView F, const Cell<float> *__restrict__ rec,
                                                      ForceRows a, BoxTable bt)
