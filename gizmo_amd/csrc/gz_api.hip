@@ -1105,7 +1105,7 @@ int ensure_sym(gz_context *ctx)
         {
             Timed t(ctx, "ngb_build");
             if (wide && !few)
-                k_build_sym_groups<<<xcd_grid(ctx->grp.ngroups), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
+                k_build_sym_groups<<<dim3(xcd_grid(ctx->grp.ngroups), group_parts(ctx->grp.ngroups)), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
                                                                                        ctx->X, ctx->Y, ctx->Z, ctx->H, ctx->ell_s, ctx->ld_s,
                                                                                        ctx->cap_s, ctx->cnt_s, ctx->counters + 3);
             else if (wide)
@@ -2282,7 +2282,7 @@ long gz_neighbors(gz_context *ctx, int symmetric, long *offsets, int *nbr, long 
             ctx->overflow_clear = false;
             if (hipMemsetAsync(ctx->counters + 3, 0, sizeof(int), ctx->stream) != hipSuccess) { rc = GZ_E_HIP; break; }
             if (ctx->nact > ctx->few_rows)
-                k_build_sym_groups<<<xcd_grid(ctx->grp.ngroups), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
+                k_build_sym_groups<<<dim3(xcd_grid(ctx->grp.ngroups), group_parts(ctx->grp.ngroups)), 64, 0, ctx->stream>>>(grid_view(ctx), ctx->grp.view(BoxTable{}), ctx->act,
                                                                                        ctx->X, ctx->Y, ctx->Z, ctx->H, ell, ld, capl, cnt,
                                                                                        ctx->counters + 3);
             else

@@ -315,7 +315,7 @@ struct SymLaunch {
 };
 inline SymLaunch sym_launch(long nrows, long ncells)
 {
-    if (nrows <= kSymFewRows * ncells) return {k_build_sym_groups, dim3(xcd_grid(ncells))};
+    if (nrows <= kSymFewRows * ncells) return {k_build_sym_groups, dim3(xcd_grid(ncells), group_parts(ncells))};
     return {k_build_sym_cells, dim3(xcd_grid(ncells), walk_parts(nrows, ncells))};
 }
 

@@ -20,6 +20,16 @@ inline unsigned stencil_grid(long ncell)
     return (unsigned)(blocks < most ? blocks : most);
 }
 
+// Workgroups along y of the walk of ngroups row groups (k_build_sym_groups, whose time grows with a group's
+// rows): while the groups do not fill the chip's 4096 places for its wavefronts, several share a group.  The
+// list stage of 19,472 particles of a shock tube searched over many levels 1014 -> 447 us (with a lane per
+// row 483), of a 33^3 lattice 457 -> 295; from 4096 groups on one workgroup each, as before.
+inline unsigned group_parts(long ngroups)
+{
+    const long p = 4096 / (ngroups > 0 ? ngroups : 1);
+    return (unsigned)(p < 1 ? 1 : (p > 8 ? 8 : p));
+}
+
 // Density rounds after the first of a batch's pass over many rows: whether the rows still iterating are
 // taken one workgroup each, from the list that the closing kernel wrote, or by a walk of every group
 // (the rows of one cell) again.  By row a row takes 2 to 4 ns (FP64 3 to 6).  A walk takes nearly as long for

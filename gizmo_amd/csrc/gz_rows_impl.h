@@ -1010,8 +1010,12 @@ __global__ void __launch_bounds__(64, 4) k_build_sym_groups(GridView g, CellRows
                  periodic_adjacent((int)compact10(cj), hz, nci));
     };
     if (!wide) stencil_ranges(cells, sten, nst);
-    for (int base = a0; base < a1; base += 64) {
-        const bool on = base + t < a1;
+    // a group's rows in equal parts of at most 64, dealt to the workgroups along y: where those are several,
+    // parts of 16 rows or more (group_parts)
+    const int parts = max((a1 - a0 + 63) / 64, min((int)gridDim.y, (a1 - a0 + 15) / 16)), part_rows = (a1 - a0 + parts - 1) / parts;
+    for (int part = blockIdx.y; part < parts; part += gridDim.y) {
+        const int base = a0 + part * part_rows;
+        const bool on = t < part_rows && base + t < a1;
         const int r = on ? (cr.grow ? cr.grow[base + t] : base + t) : 0;
         int i = -1;
         double xi = 0, yi = 0, zi = 0, hi = 0;
@@ -1101,7 +1105,7 @@ __global__ void __launch_bounds__(64, 4) k_build_sym_groups(GridView g, CellRows
             const int prev = __shfl_up(before, 1, 64), bcount = before - (t ? prev : 0);
             cells.lay(before - bcount - kCoarseRange, t <= nst ? bcount : 0, e.x, t < nst ? e.y - e.x : 0);
         }
-        const int rows = min(a1 - base, 64);
+        const int rows = min(a1 - base, part_rows);
         int n = 0, fill = 0, v0 = 0, pos = 0, j = 0;
         bool more = cells.total > 0, left = false, keep = false;
         const bool long_walk = wide && cells.total > kLongWalk;

@@ -32,6 +32,10 @@ int main()
             }
             const double per_cell = gz::fullest_cells(boxes);
             std::printf("%d %.17g\n", gz::density_by_row(remaining, ngroups, per_cell), per_cell);
+        } else if (!std::strcmp(what, "parts")) {
+            long ngroups;
+            if (std::scanf("%ld", &ngroups) != 1) return 1;
+            std::printf("%u\n", gz::group_parts(ngroups));
         } else if (!std::strcmp(what, "lanes")) {
             long nrows;
             double share, even;

@@ -49,6 +49,14 @@ def test_force_plan_of_any_room(ask, form, width):
             assert (segment == 0) == (room < 8 * entry), (nrows, room)
 
 
+def test_few_groups_share_their_rows_out(ask):
+    """Groups that leave the chip's places for wavefronts idle are taken by several workgroups each, as
+    many as fit and at most eight; groups that fill them by one."""
+    for ngroups, (parts,) in zip((0, 1, 511, 512, 1500, 4095, 4096, 10 ** 7), ask([("parts", g) for g in (0, 1, 511, 512, 1500, 4095, 4096, 10 ** 7)])):
+        assert 1 <= parts <= 8 and (parts == 1 or parts * ngroups <= 4096)
+        assert parts == 8 or (parts + 1) * ngroups > 4096
+
+
 # Later density rounds of batches as measured on the MI355X (FP32 form, then FP64, then mixtures of
 # boxes): the boxes (count x particles / cells), the groups, the rows still iterating, microseconds of
 # the walk and by row
